@@ -1426,63 +1426,111 @@ __global__ void accept_kernel(const int2 *__restrict__ pairs, const float *__res
     }
 }
 
-// The same FP64 r, RCK_P pairs per wave: the wave walks its pairs' rows
-// RCK_T time points at a time; in load m a lane reads element
-// lane % RCK_T of pair m * (64 / RCK_T) + lane / RCK_T, so every load covers
-// whole RCK_T * 8-byte runs of a few rows (a thread-per-pair loop touches 64
-// rows per load) and a pair's t points take t / RCK_T dependent rounds.  The
-// rounded products go through LDS and lane p < RCK_P adds pair p's in time
-// order: the same products and the same sequential sum as r64_pair.  Row
-// offsets i * t in 32 bits (n * t < 2^32, checked by the caller).  The loop
-// bounds are uniform over the block.
-constexpr int RCK_P = 64, RCK_T = 1024 / RCK_P, RCK_M = 16;
-__global__ __launch_bounds__(256) void recheck_rows(const int2 *__restrict__ pairs,
-                                                    const unsigned long long *__restrict__ cnt, long long cap,
-                                                    const double *__restrict__ z, int t, double *__restrict__ r_out,
-                                                    const float *__restrict__ rfast,
-                                                    unsigned long long *__restrict__ errmax, SelHist sh)
-{
+// FP64 r of P pairs by one wave, exactly as r64_pair forms it (lane p < P holds
+// pair p in e and gets its unclamped sum).  The wave walks the pairs' rows TC
+// time points at a time: TC / 2 lanes read one row's run of TC * 8 bytes, 16
+// bytes each, so a load covers whole runs of a few rows (a thread per pair
+// touches 64 rows per load and is bound by the texture addresser: 64 lines
+// for 512 bytes).  The rounded products go through LDS and lane p adds pair
+// p's in time order; the next run's loads are in flight under the sums.
+// P * TC = 1024 keeps 16 loads of 16 bytes per lane in flight.  P = 64 sums
+// on every lane (bulk); P = 16 takes t / 64 dependent rounds instead of t / 16
+// (lists that do not fill the chip with 64 pairs per wave).
+// Two layouts.  Rows: z[i * t + l], l = 0 .. t - 1; a row starts at a multiple
+// of 8 bytes only (odd t): d2u has that alignment, and a global 16-byte load
+// needs no more than 4; the run past t is read at the row's last two points
+// and masked to zero (a zero product leaves the sum: it starts at +0); n * t <
+// 2^32 and t >= 2, checked by the caller.  CHUNKS (P = 64): zchunk_copy's
+// z[(c * n + i) * 16 + l % 16], zero past t, so every run is one 128-byte line
+// (a row's run straddles two); c counts the chunks from the caller's first.
+// prod: this wave's P * (TC + 2) doubles of LDS; the padding of two keeps the
+// 16-byte row reads off each other's banks.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef double d2a __attribute__((ext_vector_type(2)));
+template <int P, bool CHUNKS = false>
+struct PairSum {
+    static constexpr int TC = 1024 / P, LPR = TC / 2, RPL = 64 / LPR, M = P / RPL, LDP = TC + 2;
+    static constexpr int LDS_DOUBLES = P * LDP;
+    static_assert(!CHUNKS || TC == 16, "a chunk is one run");
+    // rows: t points per row (n unused); chunks: len / 16 chunks of n rows
+    static __device__ __forceinline__ double run(int2 e, const double *__restrict__ z, int n, int len, double sum,
+                                                 int lane, double *__restrict__ prod)
+    {
 #pragma clang fp contract(off)
-    __shared__ double prod[4][RCK_P][RCK_T + 1];
-    constexpr int PPL = 64 / RCK_T;  // pairs per load
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lt = lane % RCK_T, lp = lane / RCK_T;
-    const long long c = (long long)min((unsigned long long)cap, *cnt);
-    double err = 0.0;
-    for (long long b0 = (long long)blockIdx.x * 4 * RCK_P; b0 < c; b0 += (long long)gridDim.x * 4 * RCK_P) {
-        const long long q = b0 + w * RCK_P + lane;
-        const int2 e = lane < RCK_P && q < c ? pairs[q] : make_int2(0, 0);
-        // row offsets of the pairs this lane loads for
-        unsigned oa[RCK_M], ob[RCK_M];
+        const int rl = lane / LPR, cl = 2 * (lane % LPR);
+        const unsigned stride = CHUNKS ? (unsigned)TC : (unsigned)len;
+        unsigned oa[M], ob[M];
 #pragma unroll
-        for (int m = 0; m < RCK_M; m++) {
-            const int src = m * PPL + lp;
-            oa[m] = (unsigned)__shfl(e.x, src) * (unsigned)t;
-            ob[m] = (unsigned)__shfl(e.y, src) * (unsigned)t;
+        for (int m = 0; m < M; m++) {
+            oa[m] = (unsigned)__shfl(e.x, m * RPL + rl) * stride;
+            ob[m] = (unsigned)__shfl(e.y, m * RPL + rl) * stride;
         }
-        double sum = 0.0;
-        for (int l0 = 0; l0 < t; l0 += RCK_T) {
-            const int l = l0 + lt;
-            const bool in = l < t;
-            double x[RCK_M], y[RCK_M];
+        d2a x[M], y[M];
+        auto load = [&](int l0) {
+            if (CHUNKS) {
+                const double *zc = z + (long long)l0 * n + cl;  // chunk l0 / 16
 #pragma unroll
-            for (int m = 0; m < RCK_M; m++) {
-                x[m] = in ? z[oa[m] + (unsigned)l] : 0.0;
-                y[m] = in ? z[ob[m] + (unsigned)l] : 0.0;
-            }
+                for (int m = 0; m < M; m++) {
+                    x[m] = *(const d2a *)(zc + oa[m]);
+                    y[m] = *(const d2a *)(zc + ob[m]);
+                }
+            } else {
+                const unsigned l = (unsigned)min(l0 + cl, len - 2);
 #pragma unroll
-            for (int m = 0; m < RCK_M; m++) prod[w][m * PPL + lp][lt] = x[m] * y[m];
-            __syncthreads();
-            if (lane < RCK_P) {
-                const int kt = min(RCK_T, t - l0);
-                for (int k = 0; k < kt; k++) {
-                    const double pk = prod[w][lane][k];
-                    sum += pk;
+                for (int m = 0; m < M; m++) {
+                    x[m] = *(const d2u *)(z + (oa[m] + l));
+                    y[m] = *(const d2u *)(z + (ob[m] + l));
                 }
             }
-            __syncthreads();
+        };
+        load(0);
+        for (int l0 = 0; l0 < len; l0 += TC) {
+            const int l = l0 + cl;
+            const bool both = CHUNKS || l + 1 < len, last = !CHUNKS && l + 1 == len;  // last: point len - 1, read as .y
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                const double p0 = x[m].x * y[m].x, p1 = x[m].y * y[m].y;
+                d2a w;
+                w.x = both ? p0 : (last ? p1 : 0.0);
+                w.y = both ? p1 : 0.0;
+                *(d2a *)(prod + (m * RPL + rl) * LDP + cl) = w;
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (l0 + TC < len) load(l0 + TC);
+            if (P == 64 || lane < P) {
+#pragma unroll
+                for (int k = 0; k < TC; k += 2) {
+                    const d2a w = *(const d2a *)(prod + lane * LDP + k);
+                    sum += w.x;
+                    sum += w.y;
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
         }
-        if (lane < RCK_P && q < c) {
-            const double r = sum > 1.0 ? 1.0 : (sum < -1.0 ? -1.0 : sum);
+        return sum;
+    }
+};
+constexpr int PAIR_LDS = PairSum<64>::LDS_DOUBLES > PairSum<16>::LDS_DOUBLES ? PairSum<64>::LDS_DOUBLES
+                                                                             : PairSum<16>::LDS_DOUBLES;
+static_assert(PAIR_LDS % 2 == 0, "each wave's products start 16-byte aligned");
+
+__device__ __forceinline__ double clamp_r(double r) { return r > 1.0 ? 1.0 : (r < -1.0 ? -1.0 : r); }
+
+// The same FP64 r of a list of pairs.  A list that gives every wave of the
+// grid 64 pairs takes 64 per wave, a shorter one 16.
+template <int P>
+__device__ __forceinline__ double recheck_list(const int2 *__restrict__ pairs, long long c,
+                                               const double *__restrict__ z, int t, double *__restrict__ r_out,
+                                               const float *__restrict__ rfast, const SelHist &sh, int lane, int w,
+                                               double *prod)
+{
+    double err = 0.0;
+    for (long long b0 = ((long long)blockIdx.x * 4 + w) * P; b0 < c; b0 += (long long)gridDim.x * 4 * P) {
+        const long long q = b0 + lane;
+        const bool own = lane < P && q < c;
+        const int2 e = own ? pairs[q] : make_int2(0, 0);
+        const double r = clamp_r(PairSum<P>::run(e, z, 0, t, 0.0, lane, prod));
+        if (own) {
             r_out[q] = r;
             if (rfast) err = fmax(err, fabs((double)rfast[q] - r));
             if (sh.h) {
@@ -1492,13 +1540,29 @@ __global__ __launch_bounds__(256) void recheck_rows(const int2 *__restrict__ pai
             }
         }
     }
+    return err;
+}
+
+__global__ __launch_bounds__(256) void recheck_rows(const int2 *__restrict__ pairs,
+                                                    const unsigned long long *__restrict__ cnt, long long cap,
+                                                    const double *__restrict__ z, int t, double *__restrict__ r_out,
+                                                    const float *__restrict__ rfast,
+                                                    unsigned long long *__restrict__ errmax, SelHist sh)
+{
+    __shared__ __align__(16) double prod[4][PAIR_LDS];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const long long c = (long long)min((unsigned long long)cap, *cnt);
+    double err = c >= (long long)gridDim.x * 256
+                     ? recheck_list<64>(pairs, c, z, t, r_out, rfast, sh, lane, w, prod[w])
+                     : recheck_list<16>(pairs, c, z, t, r_out, rfast, sh, lane, w, prod[w]);
     if (!rfast) return;
     for (int o = 32; o > 0; o >>= 1) err = fmax(err, __shfl_xor(err, o));
     if (lane == 0 && err > 0.0) atomicMax(errmax, (unsigned long long)__double_as_longlong(err));
 }
 
 // FP64 r of the first min(cap, *cnt) listed pairs (recheck_rows when the row
-// offsets fit 32 bits; grid of at most 8 work-groups per CU, bound by cap).
+// offsets fit 32 bits; grid of at most 4 work-groups per CU, the LDS's limit,
+// bound by cap).
 // sh.h: also the selection histogram of the r (zeroed by the caller).
 inline void launch_recheck(const pg_ctx *ctx, hipStream_t st, const int2 *pairs, const unsigned long long *cnt,
                            long long cap, const double *z, int n, int t, double *r_out, const float *rfast,
@@ -1506,7 +1570,7 @@ inline void launch_recheck(const pg_ctx *ctx, hipStream_t st, const int2 *pairs,
 {
     if (cap <= 0) return;
     if ((unsigned long long)n * (unsigned long long)t < (1ull << 32)) {
-        const long long g = std::min<long long>(pg_cdiv(cap, 4 * RCK_P), 8LL * std::max(ctx->num_cu, 1));
+        const long long g = std::min<long long>(pg_cdiv(cap, 64), 4LL * std::max(ctx->num_cu, 1));
         recheck_rows<<<(unsigned)g, 256, 0, st>>>(pairs, cnt, cap, z, t, r_out, rfast, errmax, sh);
     } else {
         recheck_kernel<<<(unsigned)pg_cdiv(cap, 256), 256, 0, st>>>(pairs, cnt, cap, z, t, r_out, rfast, errmax,
@@ -1543,6 +1607,8 @@ struct EdgeSrc {
     float keep_above;
     const float *keep_above_dev;  // if set, the bound is read from device memory
     long long extra_cap;
+    float *seg_w, *extra_w;       // weighted builds: FP32 of the FP64 r of each kept entry (edge_values)
+    long long w_cap;              // segment stride of seg_w: no segment holds more entries
 };
 
 __device__ __forceinline__ float src_bound(const EdgeSrc &s)
@@ -1583,10 +1649,13 @@ constexpr int SEG_THREADS = 1024;          // one work-group per segment: 16 wav
 constexpr int SEG_UNROLL = PG_SEG_UNROLL;  // segment entries per thread per batch
 
 // One thread's batch of source g: entries k0 + u * SEG_THREADS, their r~ when
-// the source is filtered (else NaN, which every keep test passes).
+// the source is filtered (else NaN, which every keep test passes); W: their
+// weights (undefined for entries the filter drops).
+template <bool W = false>
 struct SegBatch {
     int2 e[SEG_UNROLL];
     float r[SEG_UNROLL];
+    float w[W ? SEG_UNROLL : 1];
     bool in[SEG_UNROLL];
     __device__ __forceinline__ void fetch(const EdgeSrc &s, int g, long long k0, long long c)
     {
@@ -1597,6 +1666,7 @@ struct SegBatch {
             in[u] = k < c;
             e[u] = in[u] ? src_edge(s, g, k) : make_int2(0, 0);
             r[u] = in[u] && filt ? s.seg_r[(long long)g * s.seg_cap + k] : __int_as_float(0x7fc00000);
+            if (W) w[u] = in[u] ? (g < s.nseg ? s.seg_w[(long long)g * s.w_cap + k] : s.extra_w[k]) : 0.0f;
         }
     }
     __device__ __forceinline__ bool keep(int u, float ka) const { return in[u] && !(r[u] <= ka); }
@@ -1604,22 +1674,22 @@ struct SegBatch {
 
 // f(batch) over this thread's batches of source g; pipelined: the next
 // batch's loads are issued before f works on the current one.
-template <class F>
+template <bool W = false, class F>
 __device__ __forceinline__ void seg_batches(const EdgeSrc &s, int g, long long c, F &&f)
 {
     const long long step = (long long)SEG_THREADS * SEG_UNROLL;
 #if PG_SEG_PIPE
-    SegBatch a;
+    SegBatch<W> a;
     a.fetch(s, g, threadIdx.x, c);
     for (long long k0 = threadIdx.x; k0 < c; k0 += step) {
-        SegBatch b;
+        SegBatch<W> b;
         b.fetch(s, g, k0 + step, c);
         f(a);
         a = b;
     }
 #else
     for (long long k0 = threadIdx.x; k0 < c; k0 += step) {
-        SegBatch a;
+        SegBatch<W> a;
         a.fetch(s, g, k0, c);
         f(a);
     }
@@ -1637,7 +1707,7 @@ __global__ __launch_bounds__(SEG_THREADS) void bucket_count(EdgeSrc s, int nbk, 
     const int g = g0 + blockIdx.x;
     const long long c = src_count(s, g);
     const float ka = src_bound(s);
-    seg_batches(s, g, c, [&](const SegBatch &a) {
+    seg_batches(s, g, c, [&](const SegBatch<> &a) {
 #pragma unroll
         for (int u = 0; u < SEG_UNROLL; u++)
             if (a.keep(u, ka)) {
@@ -1683,7 +1753,7 @@ __global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(8))
     const long long c = ctl->ok ? src_count(s, g) : 0;
     const float lo = ctl->L2, hi = ctl->U2;
     unsigned nd = 0;
-    seg_batches(s, g, c, [&](const SegBatch &a) {
+    seg_batches(s, g, c, [&](const SegBatch<> &a) {
 #pragma unroll
         for (int u = 0; u < SEG_UNROLL; u++) {
             if (!a.in[u]) continue;
@@ -1810,14 +1880,114 @@ __global__ __launch_bounds__(1024) void bucket_scan_global(const long long *__re
     if (tid == 1023) bstart[nbk] = run;
 }
 
+// z64 (rows of t) as 16-point chunks of 128-byte lines, [tc][n][16], zero past
+// t.  One thread per two points of the output.
+__global__ __launch_bounds__(256) void zchunk_copy(const double *__restrict__ z, int n, int t, double *__restrict__ zc)
+{
+    const long long k = (long long)blockIdx.x * 256 + threadIdx.x;  // (row, pair of the chunk)
+    const int c = blockIdx.y, i = (int)(k >> 3), l = c * 16 + 2 * (int)(k & 7);
+    if (i >= n) return;
+    const double *a = z + (long long)i * t;
+    d2a v;
+    v.x = l < t ? a[l] : 0.0;
+    v.y = l + 1 < t ? a[l + 1] : 0.0;
+    *(d2a *)(zc + ((long long)c * n + i) * 16 + 2 * (k & 7)) = v;
+}
+
+// Weights of a weighted build: the FP32 of the FP64 r of every kept entry,
+// into seg_w / extra_w beside the entry.  Work-groups [0, nseg * nsub) share
+// the segments (blockIdx % nseg; nseg is a multiple of the 8 XCDs, so a
+// segment stays on the XCD whose Gram work-groups filled it and the rows of a
+// supertile meet in that L2), the rest the selected list.  Each wave compacts
+// the kept entries of 64-entry batches into 64-pair groups (a filter keeps as
+// little as a quarter of a segment) and sums them with PairSum.  One launch
+// takes chunks [c0, c1) of the series and keeps the FP64 partial sums beside
+// the entries: the rows that the 64 Gram work-groups of an XCD's supertile
+// touch (about 3,000, 1.5 MB for VAL_SLICE chunks) stay in its 4 MB L2.
+// Bound by the L2's reads.  Measured (n = 120,000, t = 300, 22.6 M pairs /
+// n = 40,009, t = 187, 16 + 8 + 4 M pairs of three sparsities): 6.6 / 4.8 ms
+// with slices of 4 chunks, 7.5 / 4.7 of 6, 6.9 / 6.4 of 2, 9.5 / 5.4 unsliced;
+// on unaligned rows of z64 13.5 / 8.1 unsliced, 9.6 / 8.2 sliced; a thread per
+// pair inside bucket_scatter took 18.9 / 33.3 ms.
+constexpr int VAL_SLICE = 4;
+__global__ __launch_bounds__(256) void edge_values(EdgeSrc s, const double *__restrict__ zc, int n, int tc, int nsub,
+                                                   int c0, int c1, double *__restrict__ part,
+                                                   double *__restrict__ epart)
+{
+    __shared__ __align__(16) double prod[4][PairSum<64>::LDS_DOUBLES];
+    __shared__ int2 le[4][128];
+    __shared__ unsigned lk[4][128];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int nsb = s.nseg * nsub, b = blockIdx.x;
+    const bool in_seg = b < nsb;
+    const int g = in_seg ? b % s.nseg : s.nseg;
+    const long long wid = (long long)(in_seg ? b / s.nseg : b - nsb) * 4 + w;
+    const long long step = 64ll * 4 * (in_seg ? nsub : (int)gridDim.x - nsb);
+    const long long c = src_count(s, g);
+    const float ka = src_bound(s);
+    const bool filt = s.seg_r && in_seg;
+    float *out = in_seg ? s.seg_w + (long long)g * s.w_cap : s.extra_w;
+    double *sums = in_seg ? part + (long long)g * s.w_cap : epart;
+    const bool first = c0 == 0, last = c1 == tc;
+    int have = 0;  // pairs waiting in le / lk; wave-uniform
+    for (long long k0 = wid * 64; k0 < c || have > 0; k0 += step) {
+        if (k0 < c) {
+            const long long k = k0 + lane;
+            bool keep = k < c;
+            const int2 e = keep ? src_edge(s, g, k) : make_int2(0, 0);
+            if (filt && keep) keep = !(s.seg_r[(long long)g * s.seg_cap + k] <= ka);
+            const unsigned long long m = __ballot(keep);
+            if (keep) {
+                const int at = have + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                le[w][at] = e;
+                lk[w][at] = (unsigned)k;
+            }
+            have += __popcll(m);
+            __builtin_amdgcn_wave_barrier();
+            if (have == 0 || (have < 64 && k0 + step < c)) continue;
+        }
+        const int take = min(have, 64);
+        const int2 e = lane < take ? le[w][lane] : make_int2(0, 0);
+        const unsigned k = lk[w][lane];
+        double r = !first && lane < take ? sums[k] : 0.0;
+        r = PairSum<64, true>::run(e, zc + (long long)c0 * n * 16, n, (c1 - c0) * 16, r, lane, prod[w]);
+        if (lane < take) {
+            if (last) out[k] = (float)clamp_r(r);
+            else sums[k] = r;
+        }
+        // the waiting rest moves down
+        const int2 e2 = le[w][64 + lane];
+        const unsigned k2 = lk[w][64 + lane];
+        __builtin_amdgcn_wave_barrier();
+        le[w][lane] = e2;
+        lk[w][lane] = k2;
+        __builtin_amdgcn_wave_barrier();
+        have -= take;
+    }
+}
+
+// The same with a thread per entry, for series beyond PairSum's 32-bit offsets.
+__global__ __launch_bounds__(256) void edge_values_wide(EdgeSrc s, const double *__restrict__ z, int t)
+{
+    const int g = blockIdx.y;
+    const long long c = src_count(s, g);
+    const float ka = src_bound(s);
+    for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < c; k += (long long)gridDim.x * 256) {
+        if (s.seg_r && g < s.nseg && s.seg_r[(long long)g * s.seg_cap + k] <= ka) continue;
+        const int2 e = src_edge(s, g, k);
+        float *out = g < s.nseg ? s.seg_w + (long long)g * s.w_cap : s.extra_w;
+        out[k] = (float)r64_pair(z, t, e.x, e.y);
+    }
+}
+
 // Entries beyond `cap` (a selection that did not hold; the caller checks
 // row[n] and rebuilds) are dropped rather than written.
-// W: the FP64 r of every entry goes along (weighted CSR).
+// W: the weight of every entry goes along (weighted CSR).
 template <bool W>
 __global__ __launch_bounds__(SEG_THREADS) void bucket_scatter(EdgeSrc s, int nbk, const long long *__restrict__ off,
                                                               const long long *__restrict__ bstart,
                                                               unsigned *__restrict__ ent, float *__restrict__ entv,
-                                                              const double *__restrict__ z, int t, long long cap)
+                                                              long long cap)
 {
     // per-bucket: this segment's output base (bstart + off; below cap, which
     // is at most INT32_MAX, whenever anything is written) and a cursor
@@ -1832,7 +2002,7 @@ __global__ __launch_bounds__(SEG_THREADS) void bucket_scatter(EdgeSrc s, int nbk
     const long long c = src_count(s, g);
     const float ka = src_bound(s);
     if (bstart[nbk] > cap) return;
-    seg_batches(s, g, c, [&](const SegBatch &a) {
+    seg_batches<W>(s, g, c, [&](const SegBatch<W> &a) {
 #pragma unroll
         for (int u = 0; u < SEG_UNROLL; u++) {
             if (!a.keep(u, ka)) continue;
@@ -1843,9 +2013,8 @@ __global__ __launch_bounds__(SEG_THREADS) void bucket_scatter(EdgeSrc s, int nbk
             ent[pf] = ((unsigned)(e.x & (BROWS - 1)) << 25) | (unsigned)e.y;
             ent[pr] = ((unsigned)(e.y & (BROWS - 1)) << 25) | (unsigned)e.x;
             if (W) {
-                const float r = (float)r64_pair(z, t, e.x, e.y);
-                entv[pf] = r;
-                entv[pr] = r;
+                entv[pf] = a.w[u];
+                entv[pr] = a.w[u];
             }
         }
     });
@@ -3298,6 +3467,7 @@ struct CorrRun {
     int2 *seg = nullptr, *bandl = nullptr;
     float *seg_r = nullptr, *band_r = nullptr;
     long long seg_cap = 0, band_cap = 0;
+    long long seg_used = 0;  // bound on the segments' counts (the largest, once the host has seen them)
     int *row = nullptr, *col = nullptr;
     float *val = nullptr;
     bool ran_hist = false, ran_emit = false;
@@ -3457,6 +3627,7 @@ struct CorrRun {
     pg_status emit_launch(long long seg_cap0, long long band_cap0, bool store_r, bool clear = true)
     {
         seg_cap = (seg_cap0 + 63) / 64 * 64;  // segments 256-byte aligned (vector loads)
+        seg_used = seg_cap;
         band_cap = band_cap0;
         PG_TRY(pg_bufT(ctx, "corr.seg", (size_t)(nwg * seg_cap), &seg));
         if (store_r) PG_TRY(pg_bufT(ctx, "corr.segr", (size_t)(nwg * seg_cap), &seg_r));
@@ -3489,7 +3660,10 @@ struct CorrRun {
             PG_HIP(ctx, hipMemcpyAsync(hcnt, counters, sizeof hcnt, hipMemcpyDeviceToHost, st));
             PG_HIP(ctx, hipStreamSynchronize(st));
             const long long mx = max_segment();
-            if (mx <= seg_cap && (long long)hcnt[0] <= band_cap) return PG_OK;
+            if (mx <= seg_cap && (long long)hcnt[0] <= band_cap) {
+                seg_used = (mx + 31) / 32 * 32;
+                return PG_OK;
+            }
             if (attempt == 2) break;
             sc = std::max(seg_cap, mx + mx / 8 + 4096);
             bcap = std::max(band_cap, (long long)hcnt[0] + (long long)hcnt[0] / 8 + 4096);
@@ -3529,10 +3703,41 @@ struct CorrRun {
         return PG_OK;
     }
 
+    // The weights of src's kept entries, into buffers beside its lists.
+    pg_status launch_edge_values(EdgeSrc &src)
+    {
+        src.w_cap = seg_used;
+        const size_t nw = (size_t)std::max<long long>(src.nseg * src.w_cap, 1), ne = (size_t)std::max<long long>(src.extra_cap, 1);
+        PG_TRY(pg_bufT(ctx, "corr.segw", nw, &src.seg_w));
+        PG_TRY(pg_bufT(ctx, "corr.extraw", ne, &src.extra_w));
+        // a chunk's row offsets are 32-bit
+        if (n < (1 << 28)) {
+            // three work-groups of 43 KB fit a CU: about that many in all
+            const int nsub = (int)std::max<long long>(1, pg_cdiv(3LL * std::max(ctx->num_cu, 1), std::max(src.nseg, 1)));
+            const long long ex = std::max<long long>(1, std::min<long long>(pg_cdiv(src.extra_cap, 256), 2LL * std::max(ctx->num_cu, 1)));
+            const int slice = VAL_SLICE;
+            const int tc = (int)pg_cdiv(t, 16);
+            double *zc, *part = nullptr, *epart = nullptr;
+            PG_TRY(pg_bufT(ctx, "corr.zc", (size_t)tc * n * 16, &zc));
+            if (tc > slice) {
+                PG_TRY(pg_bufT(ctx, "corr.segp", nw, &part));
+                PG_TRY(pg_bufT(ctx, "corr.extrap", ne, &epart));
+            }
+            zchunk_copy<<<dim3((unsigned)pg_cdiv(n, 32), (unsigned)tc), 256, 0, st>>>(z64, n, t, zc);
+            for (int c0 = 0; c0 < tc; c0 += slice)
+                edge_values<<<(unsigned)(src.nseg * nsub + ex), 256, 0, st>>>(src, zc, n, tc, nsub, c0,
+                                                                              std::min(tc, c0 + slice), part, epart);
+        } else {
+            edge_values_wide<<<dim3(8, (unsigned)src.nseg + 1), 256, 0, st>>>(src, z64, t);
+        }
+        PG_KERNEL_CHECK(ctx);
+        return PG_OK;
+    }
+
     // CSR build (bucketed counting sort), launched without a host check.
     // seg_counted: every source's bucket counts are in place (the segments'
     // from window_count, the selected list's from select_write).
-    pg_status launch_csr(const EdgeSrc &src, long long nnz, bool seg_counted = false)
+    pg_status launch_csr(EdgeSrc src, long long nnz, bool seg_counted = false)
     {
         if (nnz > INT32_MAX) return pg_fail(ctx, PG_ENOTSUP, "nnz %lld exceeds int32 CSR", (long long)nnz);
         const size_t nnzs = (size_t)std::max<long long>(nnz, 1);
@@ -3566,12 +3771,14 @@ struct CorrRun {
             const void *scatter_fn = weighted ? (const void *)bucket_scatter<true> : (const void *)bucket_scatter<false>;
             if (shs > 64 * 1024)
                 PG_HIP(ctx, set_shared_limit(ctx, scatter_fn, shs));
-            if (weighted)
-                bucket_scatter<true><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, entv, z64,
-                                                                               t, (long long)nnzs);
-            else
+            if (weighted) {
+                PG_TRY(launch_edge_values(src));
+                bucket_scatter<true><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, entv,
+                                                                               (long long)nnzs);
+            } else {
                 bucket_scatter<false><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, nullptr,
-                                                                                z64, t, (long long)nnzs);
+                                                                                (long long)nnzs);
+            }
             if (lbits) {
                 PG_HIP(ctx, set_shared_limit(ctx, rows_bits_fn(bp.rank), (int)lbits));
                 launch_rows_bits(ctx, bp, st, bstart, ent, n, nbk, row, col, (long long)nnzs);
@@ -4580,7 +4787,7 @@ pg_status pg_cohort_corr_enqueue(PgCohortCorr *P, int s, const float *dbold, int
                                                                                      P->boff, P->btot);
     bucket_scan_global<<<1, 1024, 0, st>>>(P->btot, S.nbk, P->bstart);
     bucket_scatter<false><<<(unsigned)nsrcb, SEG_THREADS, (size_t)S.nbk * 8, st>>>(es, S.nbk, P->boff, P->bstart,
-                                                                                   P->ent, nullptr, P->z64, S.t, nnz);
+                                                                                   P->ent, nullptr, nnz);
     if (S.bits_lds) {
         BitsPlan bp;
         bp.rank = S.bits_rank;
