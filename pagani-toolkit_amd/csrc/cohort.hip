@@ -95,7 +95,7 @@ extern "C" pg_status pg_cohort_run(pg_ctx *ctx, pg_subject *subj, int32_t nsub, 
     std::vector<int32_t> n((size_t)nsub), t((size_t)nsub);
     std::vector<float> sp((size_t)nsub);
     int max_n = 1;
-    long long max_src = 0;
+    long long max_src = 0, max_nnz = 0;
     for (int s = 0; s < nsub; s++) {
         const pg_subject &S = subj[s];
         if (S.n < 1 || S.t < 2 || !(S.sparsity > 0.0f && S.sparsity <= 100.0f))
@@ -112,6 +112,7 @@ extern "C" pg_status pg_cohort_run(pg_ctx *ctx, pg_subject *subj, int32_t nsub, 
         t[s] = S.t;
         sp[s] = S.sparsity;
         max_n = std::max(max_n, S.n);
+        max_nnz = std::max<long long>(max_nnz, 2 * pg_sparsity_pairs(S.n, S.sparsity));
         if (S.bc) max_src = std::max<long long>(max_src, S.nsrc);
     }
 
@@ -123,7 +124,7 @@ extern "C" pg_status pg_cohort_run(pg_ctx *ctx, pg_subject *subj, int32_t nsub, 
     // PAGANI_COHORT_LEVELS: BFS level launches per batch group in the graph
     int levels = BFS_LEVELS;
     if (const char *e = std::getenv("PAGANI_COHORT_LEVELS")) levels = std::max(1, std::min(1024, std::atoi(e)));
-    PG_TRY(pg_cohort_metrics_plan(ctx, max_n, std::max<long long>(max_src, 1), levels, &pm));
+    PG_TRY(pg_cohort_metrics_plan(ctx, max_n, max_nnz, std::max<long long>(max_src, 1), levels, &pm));
     std::unique_ptr<PgCohortMetrics, void (*)(PgCohortMetrics *)> pm_guard(pm, pg_cohort_metrics_free);
     const int grp = pg_cohort_metrics_group(pm);
     // sources of every subject, padded with -1 to whole groups of batches

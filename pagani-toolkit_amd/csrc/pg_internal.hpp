@@ -176,7 +176,8 @@ bool pg_cohort_corr_in_graph(const PgCohortCorr *P, int s);
 pg_status pg_cohort_corr_enqueue(PgCohortCorr *P, int s, const float *dbold, int32_t *row, int32_t *col,
                                  unsigned *status);
 void pg_cohort_corr_free(PgCohortCorr *P);
-pg_status pg_cohort_metrics_plan(pg_ctx *ctx, int max_n, long long max_nsrc, int levels, PgCohortMetrics **out);
+pg_status pg_cohort_metrics_plan(pg_ctx *ctx, int max_n, long long max_nnz, long long max_nsrc, int levels,
+                                 PgCohortMetrics **out);
 int pg_cohort_metrics_group(const PgCohortMetrics *M);
 pg_status pg_cohort_metrics_enqueue(PgCohortMetrics *M, const int32_t *row, const int32_t *col, int n,
                                     const int32_t *srcs, long long nsrc, int32_t *deg, float *cp, double *bc,

@@ -25,3 +25,65 @@ def test_weighted_values_bitwise(ctx, n, t):
         np.testing.assert_array_equal(row, orow)
         np.testing.assert_array_equal(col, ocol)
         np.testing.assert_array_equal(val.view(np.uint32), oval.view(np.uint32))
+
+
+def _graph(n, m, seed, hub=0):
+    """Random network of about m edges plus a vertex joined to `hub` others
+    that are themselves a ring, as sorted symmetric CSR with weights."""
+    rng = np.random.default_rng(seed)
+    a, b = rng.integers(0, n, m), rng.integers(0, n, m)
+    if hub:
+        h = rng.permutation(n - 1)[:hub] + 1
+        a = np.concatenate([a, np.zeros(hub, np.int64), h])
+        b = np.concatenate([b, h, np.roll(h, 1)])
+    lo, hi = np.minimum(a, b), np.maximum(a, b)
+    key = np.unique(lo[lo != hi] * np.int64(n) + hi[lo != hi])
+    lo, hi = key // n, key % n
+    w = rng.uniform(0.05, 1.0, key.size).astype(np.float32)
+    both = np.concatenate([key, hi * n + lo])
+    order = np.argsort(both)
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(both[order] // n, minlength=n))
+    return row, (both[order] % n).astype(np.int32), np.concatenate([w, w])[order]
+
+
+# 65,534 / 65,535 / 65,536: the last 16-bit lists, the first 32-bit ones
+@pytest.mark.parametrize("n,m,hub", [(2, 3, 0), (3, 9, 0), (63, 700, 0), (64, 1500, 20), (257, 12000, 256),
+                                     (5000, 60000, 1500), (65534, 150000, 1023), (65535, 150000, 1024),
+                                     (65536, 150000, 1025)])
+def test_clustering_lists(ctx, n, m, hub):
+    """Triangles, binary and weighted clustering over the packed upper lists:
+    lists that end inside a group, hubs around the 1,024 factors held in LDS."""
+    row, col, val = _graph(n, m, n + m, hub)
+    say(f"clustering lists n={n} nnz={col.size} hub={hub}")
+    np.testing.assert_array_equal(ctx.triangles(row, col), O.triangles(row, col))
+    cp, mean = ctx.cp_binary(row, col)
+    ocp, omean = O.cp_binary(row, col)
+    np.testing.assert_array_equal(cp.view(np.uint32), ocp.view(np.uint32))
+    assert abs(mean - omean) <= 1e-12 * max(abs(omean), 1e-300)
+    for kind in (1, 2):
+        for mode in (0, 1):
+            say(f"weighted kind={kind} mode={mode}")
+            c, mw = ctx.cp_weighted(row, col, val, kind, mode)
+            oc, omw = O.cp_weighted(row, col, val, kind, mode)
+            np.testing.assert_allclose(c, oc, rtol=1e-12, atol=0)
+            assert abs(mw - omw) <= 1e-12 * max(abs(omw), 1e-300)
+
+
+def test_clustering_zero_and_negative_weights(ctx):
+    """Zero weights close no triangle; a negative product has no real root."""
+    row, col, val = _graph(300, 9000, 5)
+    for kind in (1, 2):
+        v = val.copy()
+        # both directions of an edge keep one weight: drawn by the pair
+        src = np.repeat(np.arange(300), np.diff(row))
+        pick = (np.minimum(src, col) * 300 + np.maximum(src, col)) % 11
+        v[pick == 0] = 0.0
+        if kind == 2:
+            v[pick == 1] *= -1.0
+        say(f"zero and negative weights kind={kind}")
+        c, _ = ctx.cp_weighted(row, col, v, kind, 0)
+        oc, _ = O.cp_weighted(row, col, v, kind, 0)
+        np.testing.assert_array_equal(np.isnan(c), np.isnan(oc))
+        ok = ~np.isnan(oc)
+        np.testing.assert_allclose(c[ok], oc[ok], rtol=1e-12, atol=0)
