@@ -6,13 +6,13 @@
 // The power iteration on B^(g) + beta I is one CSR SpMV (FP32 weights, FP64
 // accumulation) plus the rank-one degree term and the diagonal correction; all
 // norms and dot products are FP64 on the device.  Every round whose members
-// are known (a wave) iterates together: two launches per iteration cover all
+// are known (a wave) iterates together: one launch per iteration covers all
 // of the wave's groups, each group stops on the device at the reference's
 // test, and the host checks the wave once per BATCH iterations.
 //
-// The bisection bookkeeping (group membership, sub-CSR, label order) is host
-// code like the reference's Partition_GPU and runs in the reference's round
-// order, so labels match it.
+// The bisection bookkeeping (group membership, label order) is host code like
+// the reference's Partition_GPU and runs in the reference's round order, so
+// labels match it; the groups' edges are laid out on the device.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,16 +24,22 @@
 #include <vector>
 
 #include "pg_internal.hpp"
+#include "pg_spmv.hpp"
 
 namespace {
 
 constexpr int MAX_ITER = 10000;      // modularity_GPU.cu:25
 constexpr double EPS = 1e-6;         // modularity_GPU.cu:28
 constexpr double RAYLEIGH_TOL = 1e-8;  // default relative tolerance of the quotient stop
-constexpr int TPB = 256;             // threads per block
-constexpr int NPB_MAX = 1024;        // nodes per work block, upper limit
+constexpr int TPB = pgdev::SP_TPB;   // threads per block
+constexpr int NPB_MAX = pgdev::SP_ROWS;  // nodes per work block, upper limit
 constexpr int GSUM_MAX = 512;        // target for block partials per group
 constexpr int BATCH = 64;            // power iterations queued per host check
+
+// A work block's group and the group's ranges, one scalar load.
+struct Block {
+    int g, fb, nb, no, ng, pad[3];
+};
 
 // One wave of independent groups (the rounds created but not yet processed),
 // concatenated: group g owns nodes [no[g], no[g] + ng[g]) of the wave and
@@ -41,13 +47,11 @@ constexpr int BATCH = 64;            // power iterations queued per host check
 // per-group sum is a fixed-order sum of its blocks' partials.
 struct Wave {
     int nnodes, nblk;
-    int npb;               // nodes per work block (64 .. NPB_MAX)
-    const int *bgrp;       // [nblk] group of each block
+    int npb;               // nodes per work block (16 .. NPB_MAX)
+    const Block *blk;      // [nblk]
     const int *no, *ng, *fb, *nb;   // [G]
     const int *gid;        // [nnodes] global id (start vector)
-    const int *srow;       // [nnodes + 1] into scol/sval (wave-global)
-    const int *scol;       // wave-global node index
-    const float *sval;
+    pgdev::SpLayout lay;   // edges inside the groups, columns relative to the group
     const double *k, *sumbg;
     double m2;
     int stopmode;          // pg_mod_stop
@@ -55,194 +59,135 @@ struct Wave {
     int max_iter;          // iterations per pass
     // per group state
     int ngroups;
-    int *stop, *iters, *it0;
+    int *iters;
+    int2 *state;           // [G] stopped, launch index the pass began with
     const int *restart;    // [G] 1: (re)start the group's pass from the start vector
-    double *beta, *vnorm, *lam;
-    // vectors: iteration li of a group reads buf[li & 1] and leaves its
-    // normalised result in buf[(li + 1) & 1]; per-block partials
-    double *buf[2], *vres, *pdot, *pss, *pe1, *pe2;
-    // Rayleigh quotient: per-block partials of x.y and x.x (phase S), and the
-    // quotient of iteration li of group g in rho[2 g + (li & 1)] (phase N)
-    double *pxy, *pxx, *rho;
+    double *beta, *lam;
+    // vectors: y_li, the result of iteration li before normalising (li = 0:
+    // the start vector, not normalised), is in buf[li % 3]; its norm (1 for
+    // li = 0) in vn[3 g + li % 3]
+    double *buf[3], *vn, *vres;
+    // per-block partials of the launch with the iteration's parity
+    double *part[2];
+    double *rho;           // [G][2] Rayleigh quotient of iteration li in rho[2 g + (li & 1)]
 };
 
-__device__ double block_sum(double x, double *red)
-{
-    const int tid = threadIdx.x;
-    red[tid] = x;
-    __syncthreads();
-    for (int o = TPB / 2; o > 0; o >>= 1) {
-        if (tid < o) red[tid] += red[tid + o];
-        __syncthreads();
-    }
-    const double r = red[0];
-    __syncthreads();
-    return r;
-}
+// |y|^2, y . k, and by the stopping rule v . y and v . v, or |v - v_prev|^2
+// and |v + v_prev|^2
+enum { P_YY, P_YK, P_A, P_B, NPART };
 
-// fixed-order sum of the group's block partials (every block gets the same value)
-__device__ double group_sum(const double *part, int f, int m, double *red)
+// Iteration li of a group (li = launches since its pass began) is one launch:
+// from the previous launch's partials come the norm of y_li, v_li . k and the
+// quotient of iteration li - 1 (the Rayleigh stop); then
+//   y_(li+1) = (B^(g) + beta I) v_li,  v_li = y_li / |y_li|,
+// a CSR SpMV of the raw y_li (pg_spmv.hpp; FP32 weights, FP64 sums) scaled once
+// per row, with the partials of |y|^2, y . k, v . y, v . v.  |v_li -+ v_(li-1)|
+// needs |y_li|, so its partials are taken here too and the vector stop looks
+// at them one launch later: the launch that finds it leaves y_li and y_(li-1)
+// in place.  n = 14,011 with 4.9 M weighted entries: 9.9 us an iteration, half of
+// it the launch and the chain of loads up to the first row (55 us as two
+// launches that gathered the vector from L2 with a wave per row, four per
+// CU).  Every skip below is uniform in a block.
+template <bool W>
+__global__ __launch_bounds__(TPB) void mod_iter(Wave w, int it)
 {
-    double s = 0.0;
-    for (int q = threadIdx.x; q < m; q += TPB) s += part[f + q];
-    return block_sum(s, red);
-}
-
-// One power iteration is two launches.  (S) the stop test on the previous
-// iteration's partials, then y = B^(g) x + beta x (CSR SpMV, FP32 weights,
-// FP64 accumulation, one wave per row) into the other buffer, and the partial
-// of |y|^2; x . k comes from the partials of the previous launch.  (N) y /= |y|
-// in place, the partials of |y - x|^2, |y + x|^2 and y . k.  Work blocks b =
-// blockIdx.x, blockIdx.x + gridDim.x, ... cover the wave; every skip below is
-// uniform in a block.
-struct PhaseSmem {
-    double red[TPB];
-    double rowv[NPB_MAX];
-    int skip;
-};
-
-__device__ __forceinline__ void phase_s(const Wave &w, int it, PhaseSmem &sm)
-{
-#pragma clang fp contract(off)
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int b = blockIdx.x; b < w.nblk; b += gridDim.x) {
-        const int g = w.bgrp[b];
-        const int li = it - w.it0[g];  // iterations completed in this pass
-        // stop[g] may be set by this launch's first block of g; every block of
-        // g reaches the same decision below, so either reading skips
-        if (threadIdx.x == 0) sm.skip = w.stop[g] || li < 0;
-        __syncthreads();
-        const int skip = sm.skip;
-        __syncthreads();
-        if (skip) continue;
-        if (li > 0) {
-            bool done;
-            if (w.stopmode == PG_MOD_STOP_VECTOR) {
-                const double e1 = sqrt(group_sum(w.pe1, w.fb[g], w.nb[g], sm.red));
-                const double e2 = sqrt(group_sum(w.pe2, w.fb[g], w.nb[g], sm.red));
+    extern __shared__ double xs[];
+    __shared__ double rowv[NPB_MAX];
+    __shared__ int2 pt[NPB_MAX];
+    __shared__ double red[TPB / 64 * NPART], tot[NPART];
+    __shared__ int skip;
+    const int tid = threadIdx.x, b = blockIdx.x;
+    const Block B = w.blk[b];
+    const int2 state = w.state[B.g];
+    const int li = it - state.y;  // iterations completed in this pass
+    const double *y = w.buf[li % 3], *yp = w.buf[(li + 2) % 3];
+    double *yn = w.buf[(li + 1) % 3];
+    const int i0 = B.no + (b - B.fb) * w.npb, nr = min(B.no + B.ng - i0, w.npb);
+    const bool vec = w.stopmode == PG_MOD_STOP_VECTOR;
+    const int i = i0 + min(tid, max(nr - 1, 0));
+    double yi, ki, si, ypi, beta, vnp, vn, sum[NPART];
+    const bool go = pgdev::sp_rows<W>(w.lay, i0, nr, y + B.no, B.ng, xs, pt, rowv, [&]() {
+        // every load that does not wait for the partials goes out before them
+        yi = y[i];
+        ki = w.k[i];
+        si = w.sumbg[i];
+        ypi = vec ? yp[i] : 0.0;
+        beta = w.beta[B.g];
+        vnp = w.vn[3 * B.g + (li + 2) % 3];
+        // the stop flag may be set by this launch's first block of the group;
+        // every block of it reaches the same decision below, so either
+        // reading skips
+        if (tid == 0) skip = state.x;
+        pgdev::sp_partials<NPART>(w.part[(it + 1) & 1], B.fb, B.nb, sum, tot);  // its barrier publishes skip
+        if (skip) return false;
+        const bool lead = b == B.fb && tid == 0;
+        vn = li > 0 ? sqrt(sum[P_YY]) : 1.0;
+        if (lead) w.vn[3 * B.g + li % 3] = vn;
+        if (li == 0) return true;
+        int done = 0, at = li;
+        if (vec) {
+            if (li > 1) {
+                const double e1 = sqrt(sum[P_A]), e2 = sqrt(sum[P_B]);
                 done = !(e1 > EPS && e2 > EPS);
-            } else {
-                // quotients of the last two completed iterations (written by
-                // earlier launches)
-                done = false;
-                if (li >= 2) {
-                    const double ra = w.rho[2 * g + ((li - 1) & 1)], rb = w.rho[2 * g + ((li - 2) & 1)];
-                    done = fabs(ra - rb) <= w.tol * fabs(ra);
-                }
+                if (done) at = li - 1;
             }
-            if (done || li >= w.max_iter) {
-                if (b == w.fb[g] && threadIdx.x == 0) {
-                    w.iters[g] = li;
-                    w.stop[g] = 1;
-                }
-                continue;
+        } else {
+            // quotients of the last two completed iterations
+            const double ra = sum[P_A] / sum[P_B];
+            if (lead) w.rho[2 * B.g + ((li - 1) & 1)] = ra;
+            if (li >= 2) {
+                const double rb = w.rho[2 * B.g + (li & 1)];
+                done = fabs(ra - rb) <= w.tol * fabs(ra);
             }
         }
-        const double *x = w.buf[li & 1];
-        double *y = w.buf[(li + 1) & 1];
-        const double vk = group_sum(w.pdot, w.fb[g], w.nb[g], sm.red);
-        const double beta = w.beta[g];
-        const int i0 = w.no[g] + (b - w.fb[g]) * w.npb, i1 = min(w.no[g] + w.ng[g], i0 + w.npb);
-        for (int i = i0 + wv; i < i1; i += TPB / 64) {
-            double acc = 0.0;
-            for (int e = w.srow[i] + lane; e < w.srow[i + 1]; e += 64) acc += x[w.scol[e]] * (double)w.sval[e];
-            for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
-            if (lane == 0) sm.rowv[i - i0] = acc;
+        if (!done && li < w.max_iter) return true;
+        if (lead) {
+            w.iters[B.g] = at;
+            w.state[B.g].x = 1;
         }
-        __syncthreads();
-        double s = 0.0, sxy = 0.0, sxx = 0.0;
-        for (int i = i0 + threadIdx.x; i < i1; i += TPB) {
-            double acc = sm.rowv[i - i0];
-            acc -= vk / w.m2 * w.k[i] + (w.sumbg[i] - beta) * x[i];
-            y[i] = acc;
-            s += acc * acc;
-            sxy += x[i] * acc;
-            sxx += x[i] * x[i];
-        }
-        s = block_sum(s, sm.red);
-        if (threadIdx.x == 0) w.pss[b] = s;
-        if (w.stopmode == PG_MOD_STOP_RAYLEIGH) {
-            sxy = block_sum(sxy, sm.red);
-            sxx = block_sum(sxx, sm.red);
-            if (threadIdx.x == 0) {
-                w.pxy[b] = sxy;
-                w.pxx[b] = sxx;
-            }
+        return false;
+    });
+    if (!go) return;
+    const double sc = 1.0 / vn, vk = sum[P_YK] * sc;
+    double p[NPART] = {0.0, 0.0, 0.0, 0.0};
+    if (tid < nr) {
+        const double x = yi * sc;
+        const double acc = rowv[tid] * sc - (vk / w.m2 * ki + (si - beta) * x);
+        yn[i] = acc;
+        p[P_YY] = acc * acc;
+        p[P_YK] = acc * ki;
+        if (!vec) {
+            p[P_A] = x * acc;
+            p[P_B] = x * x;
+        } else if (li > 0) {
+            const double xp = ypi / vnp;
+            p[P_A] = (x - xp) * (x - xp);
+            p[P_B] = (x + xp) * (x + xp);
         }
     }
-}
-
-__device__ __forceinline__ void phase_n(const Wave &w, int it, PhaseSmem &sm)
-{
-#pragma clang fp contract(off)
-    for (int b = blockIdx.x; b < w.nblk; b += gridDim.x) {
-        const int g = w.bgrp[b];
-        const int li = it - w.it0[g];
-        if (w.stop[g] || li < 0) continue;  // stop[] is not written during this launch
-        const double *x = w.buf[li & 1];
-        double *y = w.buf[(li + 1) & 1];
-        const double vn = sqrt(group_sum(w.pss, w.fb[g], w.nb[g], sm.red));
-        const int i0 = w.no[g] + (b - w.fb[g]) * w.npb, i1 = min(w.no[g] + w.ng[g], i0 + w.npb);
-        double p1 = 0.0, p2 = 0.0, pk = 0.0;
-        for (int i = i0 + threadIdx.x; i < i1; i += TPB) {
-            const double v = y[i] / vn;
-            y[i] = v;
-            const double a = v - x[i], c = v + x[i];
-            p1 += a * a;
-            p2 += c * c;
-            pk += v * w.k[i];
-        }
-        p1 = block_sum(p1, sm.red);
-        p2 = block_sum(p2, sm.red);
-        pk = block_sum(pk, sm.red);
-        if (threadIdx.x == 0) {
-            w.pe1[b] = p1;
-            w.pe2[b] = p2;
-            w.pdot[b] = pk;
-            if (b == w.fb[g]) w.vnorm[g] = vn;
-        }
-        if (w.stopmode == PG_MOD_STOP_RAYLEIGH && b == w.fb[g]) {
-            // this iteration's quotient from phase S's partials (fixed order)
-            const double xy = group_sum(w.pxy, w.fb[g], w.nb[g], sm.red);
-            const double xx = group_sum(w.pxx, w.fb[g], w.nb[g], sm.red);
-            if (threadIdx.x == 0) w.rho[2 * g + (li & 1)] = xy / xx;
-        }
-    }
-}
-
-// One phase of one iteration.  (A cooperative single-launch form with grid
-// barriers between the phases measured slower: 80 us against 62 us per
-// iteration of the three-launch form on a 1.1M-edge wave.)
-template <int P>
-__global__ __launch_bounds__(TPB) void mod_phase(Wave w, int it)
-{
-    __shared__ PhaseSmem sm;
-    if (P == 0) phase_s(w, it, sm);
-    else phase_n(w, it, sm);
+    pgdev::sp_block_sums<NPART>(p, nr, red, w.part[it & 1] + (long long)b * NPART);
 }
 
 // Groups flagged in restart[]: buf[0] = global ids (the start vector) and the
-// partials of x . k for the first iteration.
-__global__ __launch_bounds__(TPB) void mod_start(Wave w)
+// partials of x . k, as left by the launch before the pass's first, it.
+__global__ __launch_bounds__(TPB) void mod_start(Wave w, int it)
 {
-#pragma clang fp contract(off)
-    __shared__ double red[TPB];
-    for (int b = blockIdx.x; b < w.nblk; b += gridDim.x) {
-        const int g = w.bgrp[b];
-        if (!w.restart[g]) continue;
-        const int i0 = w.no[g] + (b - w.fb[g]) * w.npb, i1 = min(w.no[g] + w.ng[g], i0 + w.npb);
-        double pk = 0.0;
-        for (int i = i0 + threadIdx.x; i < i1; i += TPB) {
-            const double x = (double)w.gid[i];
-            w.buf[0][i] = x;
-            pk += x * w.k[i];
-        }
-        pk = block_sum(pk, red);
-        if (threadIdx.x == 0) w.pdot[b] = pk;
+    __shared__ double red[TPB / 64 * NPART];
+    const int b = blockIdx.x;
+    const Block B = w.blk[b];
+    if (!w.restart[B.g]) return;
+    const int i0 = B.no + (b - B.fb) * w.npb, nr = min(B.no + B.ng - i0, w.npb);
+    double p[NPART] = {0.0, 0.0, 0.0, 0.0};
+    if ((int)threadIdx.x < nr) {
+        const int i = i0 + threadIdx.x;
+        const double x = (double)w.gid[i];
+        w.buf[0][i] = x;
+        p[P_YK] = x * w.k[i];
     }
+    pgdev::sp_block_sums<NPART>(p, nr, red, w.part[(it + 1) & 1] + (long long)b * NPART);
 }
 
-// For the groups in list[]: lam[g] = +-|v| by the sign of v[mi] v0[mi] at the
+// For the groups in list[]: lam[g] = +-|y| by the sign of v[mi] v0[mi] at the
 // first largest |v[mi]| (the reference's strict '>' scan), v = the final
 // vector, v0 = the one before (Rayleigh stop: the last quotient); vres[] = v.
 __global__ __launch_bounds__(TPB) void mod_lambda(Wave w, const int *list)
@@ -252,12 +197,13 @@ __global__ __launch_bounds__(TPB) void mod_lambda(Wave w, const int *list)
     const int g = list[blockIdx.x], tid = threadIdx.x;
     const int a = w.no[g], z = a + w.ng[g];
     const int li = w.iters[g];
-    const double *v = w.buf[li & 1], *v0 = w.buf[(li + 1) & 1];
+    const double *y = w.buf[li % 3], *y0 = w.buf[(li + 2) % 3];
+    const double vn = w.vn[3 * g + li % 3], vn0 = w.vn[3 * g + (li + 2) % 3];
     double best = -1.0;
     int bi = 0x7fffffff;
     for (int i = a + tid; i < z; i += TPB) {
-        const double x = fabs(v[i]);
-        w.vres[i] = v[i];
+        const double v = y[i] / vn, x = fabs(v);
+        w.vres[i] = v;
         if (x > best) { best = x; bi = i; }
     }
     rv[tid] = best;
@@ -273,10 +219,53 @@ __global__ __launch_bounds__(TPB) void mod_lambda(Wave w, const int *list)
     }
     if (tid == 0) {
         const int mi = ri[0];
-        const double vn = w.vnorm[g];
         if (w.stopmode == PG_MOD_STOP_RAYLEIGH) w.lam[g] = w.rho[2 * g + ((li - 1) & 1)];
-        else w.lam[g] = (mi < z && v[mi] * v0[mi] > 0) ? vn : -vn;
+        else w.lam[g] = (mi < z && (y[mi] / vn) * (y0[mi] / vn0) > 0) ? vn : -vn;
     }
+}
+
+// k of every vertex: degree, or the FP64 sum of its weights (one wave per row).
+__global__ __launch_bounds__(256) void mod_strength(const int *__restrict__ row, const float *__restrict__ val, int n,
+                                                    double *__restrict__ k)
+{
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= n) return;
+    const int a = row[i], b = row[i + 1];
+    double s = 0.0;
+    if (val) {
+        for (int e = a + lane; e < b; e += 64) s += (double)val[e];
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    } else {
+        s = (double)(b - a);
+    }
+    if (lane == 0) k[i] = s;
+}
+
+// sumbg[a] = kin[a] - k_i K_g / 2m, i = gid[a]; kw[a] = k_i.  In place of kin.
+__global__ void mod_correction(const int *__restrict__ gid, const int *__restrict__ res, int r0,
+                               const double *__restrict__ k, const double *__restrict__ Kg, double m2, int nnodes,
+                               double *__restrict__ kw, double *__restrict__ sumbg)
+{
+    const int a = blockIdx.x * blockDim.x + threadIdx.x;
+    if (a >= nnodes) return;
+    const int i = gid[a];
+    kw[a] = k[i];
+    sumbg[a] = sumbg[a] - k[i] * Kg[res[i] - r0] / m2;
+}
+
+// Per row the FP64 weight (count without val) of its entries inside its own module.
+__global__ __launch_bounds__(256) void mod_inside(const int *__restrict__ row, const int *__restrict__ col,
+                                                  const float *__restrict__ val, const int *__restrict__ lab, int n,
+                                                  double *__restrict__ in)
+{
+    const int i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (i >= n) return;
+    const int l = lab[i];
+    double s = 0.0;
+    for (int e = row[i] + lane; e < row[i + 1]; e += 64)
+        if (lab[col[e]] == l) s += val ? (double)val[e] : 1.0;
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0) in[i] = s;
 }
 
 }  // namespace
@@ -309,35 +298,40 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
     PG_TRY(pg_check_csr_args(ctx, row, col, n, nnz));
     PG_HIP(ctx, hipSetDevice(ctx->device));
     hipStream_t st = ctx->stream;
-    // host copies: the bisection driver builds each group's sub-CSR
-    std::vector<int> R((size_t)n + 1), Cc((size_t)nnz);
-    std::vector<float> V(val ? (size_t)nnz : 0);
-    auto fetch = [&](void *dst, const void *src, size_t bytes) -> pg_status {
-        if (bytes == 0) return PG_OK;
-        if (pg_is_device_ptr(src)) PG_HIP(ctx, hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
-        else std::memcpy(dst, src, bytes);
-        return PG_OK;
-    };
-    PG_TRY(fetch(R.data(), row, ((size_t)n + 1) * 4));
-    PG_TRY(fetch(Cc.data(), col, (size_t)nnz * 4));
-    if (val) PG_TRY(fetch(V.data(), val, (size_t)nnz * 4));
-    // the driver indexes host and device arrays with these offsets and columns
-    if (R[0] != 0 || R[n] != nnz) return pg_fail(ctx, PG_EFORMAT, "row[0]=%d row[n]=%d, nnz=%lld", R[0], R[n], (long long)nnz);
-    for (int i = 0; i < n; i++)
-        if (R[i] > R[i + 1]) return pg_fail(ctx, PG_EFORMAT, "row offsets decrease at %d", i);
-    for (int64_t e = 0; e < nnz; e++)
-        if (Cc[(size_t)e] < 0 || Cc[(size_t)e] >= n)
-            return pg_fail(ctx, PG_EFORMAT, "column %d at %lld outside [0, %d)", Cc[(size_t)e], (long long)e, n);
+    const int *drow, *dcol;
+    const float *dval = nullptr;
+    PG_TRY(pg_in(ctx, row, (size_t)n + 1, "in.row", &drow));
+    PG_TRY(pg_in(ctx, col, (size_t)nnz, "in.col", &dcol));
+    if (val) PG_TRY(pg_in(ctx, val, (size_t)nnz, "in.val", &dval));
+    PG_TRY(pg_validate_csr(ctx, drow, dcol, n, nnz, false));
+    const size_t nn = (size_t)n + 1;
+    double *d_kall, *d_in;
+    int *d_res, *d_rloc, *d_part;
+    PG_TRY(pg_bufT(ctx, "mod.kall", nn, &d_kall));
+    PG_TRY(pg_bufT(ctx, "mod.inside", nn, &d_in));
+    PG_TRY(pg_bufT(ctx, "mod.res", nn, &d_res));
+    PG_TRY(pg_bufT(ctx, "mod.rloc", nn, &d_rloc));
+    // edges inside the groups of a wave: sized once for the whole network
+    pgdev::SpLayout lay;
+    {
+        const int nseg = pgdev::sp_nseg(n);
+        const size_t room = pgdev::sp_room(n, nnz, nseg);
+        PG_TRY(pg_bufT(ctx, "mod.idx", room, &lay.idx));
+        lay.val = nullptr;
+        if (dval) PG_TRY(pg_bufT(ctx, "mod.lval", room, &lay.val));
+        PG_TRY(pg_bufT(ctx, "mod.part", 2 * nn * nseg, &d_part));
+        lay.part = (int2 *)d_part;
+    }
 
     std::vector<double> k((size_t)n);
     double m2 = 0.0;
-    for (int i = 0; i < n; i++) {
-        double ki = 0.0;
-        if (kmode == PG_MOD_BINARY_K || !val) ki = (double)(R[i + 1] - R[i]);
-        else for (int e = R[i]; e < R[i + 1]; e++) ki += (double)V[e];
-        k[i] = ki;
-        m2 += ki;
+    if (n > 0) {
+        mod_strength<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, kmode == PG_MOD_BINARY_K ? nullptr : dval, n, d_kall);
+        PG_KERNEL_CHECK(ctx);
+        PG_HIP(ctx, hipMemcpyAsync(k.data(), d_kall, (size_t)n * 8, hipMemcpyDeviceToHost, st));
+        PG_HIP(ctx, hipStreamSynchronize(st));
     }
+    for (int i = 0; i < n; i++) m2 += k[i];
     std::vector<int> res((size_t)n, 0), adj((size_t)2 * n + 2, 0);
     int maxr = 0, index = 1, nrounds = 0;
     if (lambda0) *lambda0 = 0.0;
@@ -353,7 +347,7 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
     // order exactly as the sequential driver (modularity_GPU.cu:405-525).
     int lo = 0, nwave = 0;
     std::vector<int> rloc((size_t)n);
-    // PAGANI_MOD_TRACE=1: one line per wave on stderr (groups, nodes, edges,
+    // PAGANI_MOD_TRACE=1: one line per wave on stderr (groups, nodes,
     // iterations, seconds)
     const char *trace_env = std::getenv("PAGANI_MOD_TRACE");
     const bool trace = opts->progress || (trace_env && trace_env[0] == '1');
@@ -376,12 +370,16 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
             if (res[i] >= lo && res[i] < hi) gcount[res[i] - lo]++;
         std::vector<int> no((size_t)G), ng((size_t)G), fb((size_t)G), nb((size_t)G);
         int nnodes = 0, nblk = 0;
-        // small work blocks for parallelism, large enough that no group has
-        // more than GSUM_MAX block partials to sum
+        // about one work block per CU (its LDS holds a vector segment), none
+        // over two groups, no group with more than GSUM_MAX block partials
         int gmax = 1;
-        for (int g = 0; g < G; g++) gmax = std::max(gmax, gcount[g]);
-        int npb = 64;
-        while (npb < NPB_MAX && pg_cdiv(gmax, npb) > GSUM_MAX) npb *= 2;
+        long long all = 0;
+        for (int g = 0; g < G; g++) {
+            gmax = std::max(gmax, gcount[g]);
+            all += gcount[g];
+        }
+        int npb = (int)std::min<long long>(NPB_MAX, std::max<long long>(16, pg_cdiv(all, std::max(ctx->num_cu, 1))));
+        while (npb < NPB_MAX && pg_cdiv(gmax, npb) > GSUM_MAX) npb = std::min(NPB_MAX, 2 * npb);
         for (int g = 0; g < G; g++) {
             no[g] = nnodes;
             ng[g] = gcount[g];
@@ -390,108 +388,84 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
             nnodes += ng[g];
             nblk += nb[g];
         }
-        std::vector<int> gid((size_t)nnodes), fill(no), bgrp((size_t)nblk);
+        std::vector<int> gid((size_t)nnodes), fill(no);
+        std::vector<Block> blk((size_t)nblk);
         for (int g = 0; g < G; g++)
-            for (int q = 0; q < nb[g]; q++) bgrp[fb[g] + q] = g;
+            for (int q = 0; q < nb[g]; q++) blk[fb[g] + q] = Block{g, fb[g], nb[g], no[g], ng[g], {0, 0, 0}};
         for (int i = 0; i < n; i++)
             if (res[i] >= lo && res[i] < hi) {
                 const int g = res[i] - lo;
                 rloc[i] = fill[g];
                 gid[fill[g]++] = i;
             }
-        // sub-CSRs: edges inside the same round, wave-global node indices
-        std::vector<int> srow((size_t)nnodes + 1, 0), scol;
-        std::vector<float> sval;
-        std::vector<double> kw((size_t)nnodes), sumbg((size_t)nnodes), Kg((size_t)G, 0.0);
+        std::vector<double> Kg((size_t)G, 0.0);
         for (int a = 0; a < nnodes; a++) Kg[res[gid[a]] - lo] += k[gid[a]];
-        scol.reserve((size_t)nnz);
-        sval.reserve((size_t)nnz);
-        for (int a = 0; a < nnodes; a++) {
-            const int i = gid[a], r = res[i];
-            double kin = 0.0;
-            for (int e = R[i]; e < R[i + 1]; e++) {
-                const int j = Cc[e];
-                if (res[j] != r) continue;
-                const float wv = val ? V[e] : 1.0f;
-                scol.push_back(rloc[j]);
-                sval.push_back(wv);
-                kin += (kmode == PG_MOD_BINARY_K && val) ? 1.0 : (double)wv;
-            }
-            srow[a + 1] = (int)scol.size();
-            kw[a] = k[i];
-            sumbg[a] = kin - k[i] * Kg[r - lo] / m2;
-        }
-        const size_t gn = scol.size();
 
         Wave w;
-        int *d_bgrp, *d_no, *d_ng, *d_fb, *d_nb, *d_gid, *d_srow, *d_scol, *d_restart, *d_stop, *d_iters, *d_it0,
-            *d_list;
-        float *d_sval;
-        double *d_k, *d_sumbg, *d_beta, *d_vnorm, *d_lam, *d_b0, *d_b1, *d_vres, *d_pdot, *d_pss, *d_pe1, *d_pe2,
-            *d_pxy, *d_pxx, *d_rho;
-        PG_TRY(pg_bufT(ctx, "mod.bgrp", (size_t)nblk, &d_bgrp));
+        Block *d_blk;
+        int2 *d_state;
+        int *d_no, *d_ng, *d_fb, *d_nb, *d_gid, *d_restart, *d_iters, *d_list;
+        double *d_k, *d_sumbg, *d_Kg, *d_beta, *d_lam, *d_vn, *d_vres, *d_rho;
+        PG_TRY(pg_bufT(ctx, "mod.blk", (size_t)nblk, &d_blk));
         PG_TRY(pg_bufT(ctx, "mod.no", (size_t)G, &d_no));
         PG_TRY(pg_bufT(ctx, "mod.ng", (size_t)G, &d_ng));
         PG_TRY(pg_bufT(ctx, "mod.fb", (size_t)G, &d_fb));
         PG_TRY(pg_bufT(ctx, "mod.nb", (size_t)G, &d_nb));
         PG_TRY(pg_bufT(ctx, "mod.gid", (size_t)nnodes + 1, &d_gid));
-        PG_TRY(pg_bufT(ctx, "mod.srow", (size_t)nnodes + 1, &d_srow));
-        PG_TRY(pg_bufT(ctx, "mod.scol", gn + 1, &d_scol));
-        PG_TRY(pg_bufT(ctx, "mod.sval", gn + 1, &d_sval));
         PG_TRY(pg_bufT(ctx, "mod.k", (size_t)nnodes + 1, &d_k));
         PG_TRY(pg_bufT(ctx, "mod.sumbg", (size_t)nnodes + 1, &d_sumbg));
+        PG_TRY(pg_bufT(ctx, "mod.Kg", (size_t)G, &d_Kg));
         PG_TRY(pg_bufT(ctx, "mod.restart", (size_t)G, &d_restart));
-        PG_TRY(pg_bufT(ctx, "mod.stop", (size_t)G, &d_stop));
+        PG_TRY(pg_bufT(ctx, "mod.state", (size_t)G, &d_state));
         PG_TRY(pg_bufT(ctx, "mod.iters", (size_t)G, &d_iters));
-        PG_TRY(pg_bufT(ctx, "mod.it0", (size_t)G, &d_it0));
         PG_TRY(pg_bufT(ctx, "mod.list", (size_t)G, &d_list));
         PG_TRY(pg_bufT(ctx, "mod.beta", (size_t)G, &d_beta));
-        PG_TRY(pg_bufT(ctx, "mod.vnorm", (size_t)G, &d_vnorm));
         PG_TRY(pg_bufT(ctx, "mod.lam", (size_t)G, &d_lam));
-        PG_TRY(pg_bufT(ctx, "mod.b0", (size_t)nnodes + 1, &d_b0));
-        PG_TRY(pg_bufT(ctx, "mod.b1", (size_t)nnodes + 1, &d_b1));
+        PG_TRY(pg_bufT(ctx, "mod.vn", (size_t)G * 3, &d_vn));
+        PG_TRY(pg_bufT(ctx, "mod.b0", (size_t)nnodes + 1, &w.buf[0]));
+        PG_TRY(pg_bufT(ctx, "mod.b1", (size_t)nnodes + 1, &w.buf[1]));
+        PG_TRY(pg_bufT(ctx, "mod.b2", (size_t)nnodes + 1, &w.buf[2]));
         PG_TRY(pg_bufT(ctx, "mod.vres", (size_t)nnodes + 1, &d_vres));
-        PG_TRY(pg_bufT(ctx, "mod.pdot", (size_t)nblk, &d_pdot));
-        PG_TRY(pg_bufT(ctx, "mod.pss", (size_t)nblk, &d_pss));
-        PG_TRY(pg_bufT(ctx, "mod.pe1", (size_t)nblk, &d_pe1));
-        PG_TRY(pg_bufT(ctx, "mod.pe2", (size_t)nblk, &d_pe2));
-        PG_TRY(pg_bufT(ctx, "mod.pxy", (size_t)nblk, &d_pxy));
-        PG_TRY(pg_bufT(ctx, "mod.pxx", (size_t)nblk, &d_pxx));
+        PG_TRY(pg_bufT(ctx, "mod.part0", (size_t)nblk * NPART, &w.part[0]));
+        PG_TRY(pg_bufT(ctx, "mod.part1", (size_t)nblk * NPART, &w.part[1]));
         PG_TRY(pg_bufT(ctx, "mod.rho", (size_t)G * 2, &d_rho));
         auto h2d = [&](void *dst, const void *src, size_t bytes) -> pg_status {
             if (bytes) PG_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
             return PG_OK;
         };
-        std::vector<int> zeros((size_t)G, 0);
+        std::vector<int2> hstate((size_t)G, make_int2(0, 0));
         std::vector<double> dzeros((size_t)G, 0.0);
-        PG_TRY(h2d(d_bgrp, bgrp.data(), (size_t)nblk * 4));
+        PG_TRY(h2d(d_blk, blk.data(), (size_t)nblk * sizeof(Block)));
         PG_TRY(h2d(d_no, no.data(), (size_t)G * 4));
         PG_TRY(h2d(d_ng, ng.data(), (size_t)G * 4));
         PG_TRY(h2d(d_fb, fb.data(), (size_t)G * 4));
         PG_TRY(h2d(d_nb, nb.data(), (size_t)G * 4));
         PG_TRY(h2d(d_gid, gid.data(), (size_t)nnodes * 4));
-        PG_TRY(h2d(d_srow, srow.data(), ((size_t)nnodes + 1) * 4));
-        PG_TRY(h2d(d_scol, scol.data(), gn * 4));
-        PG_TRY(h2d(d_sval, sval.data(), gn * 4));
-        PG_TRY(h2d(d_k, kw.data(), (size_t)nnodes * 8));
-        PG_TRY(h2d(d_sumbg, sumbg.data(), (size_t)nnodes * 8));
+        PG_TRY(h2d(d_Kg, Kg.data(), (size_t)G * 8));
+        PG_TRY(h2d(d_res, res.data(), (size_t)n * 4));
+        PG_TRY(h2d(d_rloc, rloc.data(), (size_t)n * 4));
+        // the groups' edges, laid out on the device
+        lay.nseg = pgdev::sp_nseg(gmax);
+        lay.cap = pgdev::sp_cap(gmax);
+        pgdev::sp_build<<<(unsigned)pg_cdiv(std::max(nnodes, 1), 4), 256, 0, st>>>(
+            drow, dcol, dval, nnodes, d_gid, d_res, lo, d_no, d_rloc, lay, d_sumbg, kmode == PG_MOD_BINARY_K ? 1 : 0);
+        mod_correction<<<(unsigned)pg_cdiv(std::max(nnodes, 1), 256), 256, 0, st>>>(d_gid, d_res, lo, d_kall, d_Kg, m2,
+                                                                                   nnodes, d_k, d_sumbg);
+        PG_KERNEL_CHECK(ctx);
         std::vector<int> ones((size_t)G, 1);
         PG_TRY(h2d(d_restart, ones.data(), (size_t)G * 4));
-        PG_TRY(h2d(d_stop, zeros.data(), (size_t)G * 4));
-        PG_TRY(h2d(d_it0, zeros.data(), (size_t)G * 4));
+        PG_TRY(h2d(d_state, hstate.data(), (size_t)G * sizeof(int2)));
         PG_TRY(h2d(d_beta, dzeros.data(), (size_t)G * 8));
         w.nnodes = nnodes;
         w.nblk = nblk;
         w.npb = npb;
-        w.bgrp = d_bgrp;
+        w.blk = d_blk;
         w.no = d_no;
         w.ng = d_ng;
         w.fb = d_fb;
         w.nb = d_nb;
         w.gid = d_gid;
-        w.srow = d_srow;
-        w.scol = d_scol;
-        w.sval = d_sval;
+        w.lay = lay;
         w.k = d_k;
         w.sumbg = d_sumbg;
         w.m2 = m2;
@@ -499,44 +473,37 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
         w.tol = tol;
         w.max_iter = max_iter;
         w.ngroups = G;
-        w.stop = d_stop;
+        w.state = d_state;
         w.restart = d_restart;
         w.iters = d_iters;
-        w.it0 = d_it0;
         w.beta = d_beta;
-        w.vnorm = d_vnorm;
         w.lam = d_lam;
-        w.buf[0] = d_b0;
-        w.buf[1] = d_b1;
+        w.vn = d_vn;
         w.vres = d_vres;
-        w.pdot = d_pdot;
-        w.pss = d_pss;
-        w.pe1 = d_pe1;
-        w.pe2 = d_pe2;
-        w.pxy = d_pxy;
-        w.pxx = d_pxx;
         w.rho = d_rho;
 
         // pass state per group: 0 first pass, 1 shifted pass, 2 finished
-        std::vector<int> pass((size_t)G, 0), list, hit0((size_t)G, 0);
+        std::vector<int> pass((size_t)G, 0), list;
         std::vector<double> lam_total((size_t)G, 0.0), hbeta((size_t)G, 0.0);
-        mod_start<<<(unsigned)nblk, TPB, 0, st>>>(w);
+        mod_start<<<(unsigned)nblk, TPB, 0, st>>>(w, 0);
         PG_KERNEL_CHECK(ctx);
+        const size_t lds = pgdev::sp_lds(lay.cap);
+        const void *iter_fn = lay.val ? (const void *)mod_iter<true> : (const void *)mod_iter<false>;
+        PG_HIP(ctx, hipFuncSetAttribute(iter_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         int it = 0, running = G;
-        std::vector<int> hdone((size_t)G);
         std::vector<double> hlam((size_t)G);
         while (running > 0) {
             for (int q = 0; q < BATCH; q++) {
-                mod_phase<0><<<(unsigned)nblk, TPB, 0, st>>>(w, it + q);
-                mod_phase<1><<<(unsigned)nblk, TPB, 0, st>>>(w, it + q);
+                if (lay.val) mod_iter<true><<<(unsigned)nblk, TPB, lds, st>>>(w, it + q);
+                else mod_iter<false><<<(unsigned)nblk, TPB, lds, st>>>(w, it + q);
             }
             it += BATCH;
             PG_KERNEL_CHECK(ctx);
-            PG_HIP(ctx, hipMemcpyAsync(hdone.data(), d_stop, (size_t)G * 4, hipMemcpyDeviceToHost, st));
+            PG_HIP(ctx, hipMemcpyAsync(hstate.data(), d_state, (size_t)G * sizeof(int2), hipMemcpyDeviceToHost, st));
             PG_HIP(ctx, hipStreamSynchronize(st));
             list.clear();
             for (int g = 0; g < G; g++)
-                if (pass[g] < 2 && hdone[g]) list.push_back(g);
+                if (pass[g] < 2 && hstate[g].x) list.push_back(g);
             if (list.empty()) continue;
             const int m = (int)list.size();
             PG_TRY(h2d(d_list, list.data(), (size_t)m * 4));
@@ -566,21 +533,18 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
             }
             if (!restart.empty()) {
                 // second pass on B + beta I, beta = -lambda, from the start vector
-                // no iteration ran since hdone (stop flags) was read: it is
-                // the device state
+                // no iteration ran since hstate was read: it is the device state
                 std::vector<int> rflag((size_t)G, 0);
                 for (int g : restart) {
                     hbeta[g] = -lam_total[g];
-                    hit0[g] = it;
-                    hdone[g] = 0;
+                    hstate[g] = make_int2(0, it);
                     rflag[g] = 1;
                 }
                 PG_TRY(h2d(d_restart, rflag.data(), (size_t)G * 4));
-                mod_start<<<(unsigned)nblk, TPB, 0, st>>>(w);
+                mod_start<<<(unsigned)nblk, TPB, 0, st>>>(w, it);
                 PG_KERNEL_CHECK(ctx);
                 PG_TRY(h2d(d_beta, hbeta.data(), (size_t)G * 8));
-                PG_TRY(h2d(d_it0, hit0.data(), (size_t)G * 4));
-                PG_TRY(h2d(d_stop, hdone.data(), (size_t)G * 4));
+                PG_TRY(h2d(d_state, hstate.data(), (size_t)G * sizeof(int2)));
                 PG_HIP(ctx, hipStreamSynchronize(st));
             }
         }
@@ -596,9 +560,9 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
                 big = std::max(big, ng[g]);
             }
             const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - wave_t0).count();
-            std::fprintf(stderr, "pg_modularity wave %d: rounds %d..%d, %d nodes (largest group %d), %zu edges, "
+            std::fprintf(stderr, "pg_modularity wave %d: rounds %d..%d, %d nodes (largest group %d), "
                          "%d launched iterations, max %d in one pass, %.3f s\n",
-                         nwave, lo, hi - 1, nnodes, big, gn, it, mx, secs);
+                         nwave, lo, hi - 1, nnodes, big, it, mx, secs);
         }
         nwave++;
 
@@ -642,12 +606,19 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
         // W modularity_GPU.cu:500-509 with the same k and m convention
         int maxl = 0;
         for (int i = 0; i < n; i++) maxl = std::max(maxl, lab[i]);
-        std::vector<double> kc((size_t)maxl + 2, 0.0);
+        std::vector<double> kc((size_t)maxl + 2, 0.0), inside((size_t)n);
         double in = 0.0;
+        if (n > 0) {
+            PG_HIP(ctx, hipMemcpyAsync(d_res, lab.data(), (size_t)n * 4, hipMemcpyHostToDevice, st));
+            mod_inside<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, dcol, kmode == PG_MOD_BINARY_K ? nullptr : dval,
+                                                                d_res, n, d_in);
+            PG_KERNEL_CHECK(ctx);
+            PG_HIP(ctx, hipMemcpyAsync(inside.data(), d_in, (size_t)n * 8, hipMemcpyDeviceToHost, st));
+            PG_HIP(ctx, hipStreamSynchronize(st));
+        }
         for (int i = 0; i < n; i++) {
             kc[lab[i]] += k[i];
-            for (int e = R[i]; e < R[i + 1]; e++)
-                if (lab[Cc[e]] == lab[i]) in += (kmode == PG_MOD_BINARY_K || !val) ? 1.0 : (double)V[e];
+            in += inside[i];
         }
         double s2 = 0.0;
         for (double x : kc) s2 += x * x;

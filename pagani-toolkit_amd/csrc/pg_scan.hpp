@@ -1,6 +1,6 @@
 // pg_scan.hpp -- exclusive scan of a short int array by one work-group,
-// shared by the CSR builders of the dense average, the rewiring and the
-// sliced eigenvector-centrality layout.  gfx950 only.
+// shared by the CSR builders of the dense average and the rewiring.  gfx950
+// only.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1,0 +1,248 @@
+// pg_spmv.hpp -- sparse matrix times FP64 vector for the power iterations
+// (modularity, eigenvector centrality), MI355X (gfx950).
+//
+// An FP64 gather straight from L2 costs the texture addresser one line per
+// lane (64 clocks per 64 entries), so the vector is staged in LDS, SP_SEG
+// entries (128 KB of the CU's 160 KB) at a time, and gathered there.  Rows are
+// split by segment into parts, a part's entries stored as 16-bit
+// segment-relative columns (and FP32 weights) in groups of four, its last
+// group filled with the index of a zero LDS slot (weight 0): one 8-byte load
+// (and one of 16) brings a lane four entries, aligned and without bounds.  16
+// lanes take a part, so a work-group of 1,024 threads works on 64 rows at once
+// and a row of up to 256 entries has all its loads in flight.  Row i's parts
+// start at group ceil(row[i] / 4) + i * nseg and follow each other: the
+// fillers always fit before row i + 1's, so the layout needs no scan.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+namespace pgdev {
+
+constexpr int SP_TPB = 1024;     // threads per work-group: 64 rows of 16 lanes
+constexpr int SP_SEG = 16384;    // vector entries per LDS segment
+constexpr int SP_ROWS = 1024;    // most rows per work-group
+constexpr int SP_LOADS = SP_SEG / (2 * SP_TPB);  // 16-byte staging loads per thread
+
+typedef double sp_d2u __attribute__((ext_vector_type(2), aligned(8)));
+
+struct SpLayout {
+    uint16_t *idx;  // groups of 4
+    float *val;     // the same places (NULL: every weight is 1)
+    int2 *part;     // [rows][nseg]: first group, groups
+    int nseg, cap;  // segments of a row's vector; its entries per segment (the zero slot's index)
+};
+
+inline int sp_nseg(long long n) { return (int)std::max<long long>(1, (n + SP_SEG - 1) / SP_SEG); }
+inline int sp_cap(long long n) { return (int)std::max<long long>(1, std::min<long long>(n, SP_SEG)); }
+// entries of idx / val for nnz entries of n rows
+inline size_t sp_room(long long n, long long nnz, int nseg)
+{
+    return 4 * ((size_t)(nnz + 3) / 4 + (size_t)n * nseg + 1);
+}
+// dynamic LDS: the segment, the zero slot
+inline size_t sp_lds(int cap) { return ((size_t)cap + 1) * sizeof(double); }
+
+// Layout of rows a = 0 .. nrows - 1 by one wave each: row i = gid[a] (a itself
+// when gid is NULL), its entries (i, j) with grp[j] == grp[i] (all when grp is
+// NULL) at vector position loc[j] - base[grp[i] - grp0] (j itself).  Columns
+// may come in any order: a pass per segment.  kin[a] (may be NULL): FP64 sum
+// of the kept weights (their count with `count`).
+static __global__ __launch_bounds__(256) void sp_build(const int *__restrict__ row, const int *__restrict__ col,
+                                                const float *__restrict__ val, int nrows,
+                                                const int *__restrict__ gid, const int *__restrict__ grp, int grp0,
+                                                const int *__restrict__ base, const int *__restrict__ loc, SpLayout L,
+                                                double *__restrict__ kin, int count)
+{
+    const int a = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (a >= nrows) return;
+    const int i = gid ? gid[a] : a;
+    const int r0 = row[i], r1 = row[i + 1];
+    const int g = grp ? grp[i] : 0, b0 = grp ? base[g - grp0] : 0;
+    int g0 = (r0 + 3) / 4 + i * L.nseg;
+    double k = 0.0;
+    for (int s = 0; s < L.nseg; s++) {
+        int have = 0;
+        for (int e0 = r0; e0 < r1; e0 += 64) {
+            const int e = e0 + lane;
+            int p = -1;
+            if (e < r1) {
+                const int j = col[e];
+                if (!grp || grp[j] == g) p = (grp ? loc[j] - b0 : j) - s * SP_SEG;
+            }
+            const bool keep = p >= 0 && p < SP_SEG;
+            const unsigned long long m = __ballot(keep);
+            if (keep) {
+                const int at = have + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                const float w = val ? val[e] : 1.0f;
+                L.idx[4ll * g0 + at] = (uint16_t)p;
+                if (L.val) L.val[4ll * g0 + at] = w;
+                k += count ? 1.0 : (double)w;
+            }
+            have += __popcll(m);
+        }
+        const int ng = (have + 3) / 4;
+        if (have + lane < 4 * ng) {
+            L.idx[4ll * g0 + have + lane] = (uint16_t)L.cap;
+            if (L.val) L.val[4ll * g0 + have + lane] = 0.0f;
+        }
+        if (lane == 0) L.part[(long long)a * L.nseg + s] = make_int2(g0, ng);
+        g0 += ng;
+    }
+    if (kin) {
+        for (int o = 32; o > 0; o >>= 1) k += __shfl_xor(k, o);
+        if (lane == 0) kin[a] = k;
+    }
+}
+
+// NB groups of a part per lane (l = 0 .. 15), from group g on: 256 entries, 128
+// where the weights' registers would spill.
+template <bool W>
+struct SpBatch {
+    static constexpr int NB = W ? 2 : 4;
+    uint2 c[NB];
+    float4 w[NB];
+    __device__ __forceinline__ void load(const SpLayout &L, int g, int end)
+    {
+        const uint2 *ix = (const uint2 *)L.idx;
+        const float4 *wx = (const float4 *)L.val;
+        const unsigned pad = (unsigned)L.cap * 0x10001u;
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const bool in = g + 16 * u < end;
+            c[u] = in ? ix[g + 16 * u] : make_uint2(pad, pad);
+            if (W) w[u] = in ? wx[g + 16 * u] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+    }
+    __device__ __forceinline__ double dot(const double *__restrict__ xs, double acc) const
+    {
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const double x0 = xs[c[u].x & 0xffffu], x1 = xs[c[u].x >> 16];
+            const double x2 = xs[c[u].y & 0xffffu], x3 = xs[c[u].y >> 16];
+            if (W) {
+                acc = fma(x0, (double)w[u].x, acc);
+                acc = fma(x1, (double)w[u].y, acc);
+                acc = fma(x2, (double)w[u].z, acc);
+                acc = fma(x3, (double)w[u].w, acc);
+            } else {
+                acc += (x0 + x1) + (x2 + x3);
+            }
+        }
+        return acc;
+    }
+};
+
+// Row sums of rows a0 .. a0 + nr - 1 (nr <= SP_ROWS) against x[0 .. len) into
+// rowv[0 .. nr), behind a barrier.  xs: sp_lds(cap) of LDS; pt: SP_ROWS int2 of
+// LDS.  Latency is what the loop hides: a segment's vector entries and part
+// bounds are loaded into registers under the segment before it (the first
+// under `between`, which the caller's own waits go into; it returns whether to
+// go on, the same in every thread), and a part's entries under the part
+// before it.
+template <bool W, class F>
+__device__ __forceinline__ bool sp_rows(const SpLayout &L, int a0, int nr, const double *__restrict__ x, int len,
+                                        double *__restrict__ xs, int2 *__restrict__ pt, double *__restrict__ rowv,
+                                        F &&between)
+{
+    const int tid = threadIdx.x, l = tid & 15, q = tid >> 4;
+    const int2 *part = L.part + (long long)a0 * L.nseg;
+    sp_d2u v[SP_LOADS];
+    int2 pn = make_int2(0, 0);
+    auto load = [&](int s) {
+        const double *xb = x + (long long)s * SP_SEG;
+        const int m = min(SP_SEG, len - s * SP_SEG);
+#pragma unroll
+        for (int u = 0; u < SP_LOADS; u++) {
+            const int k = 2 * (tid + u * SP_TPB);
+            v[u].x = 0.0;
+            v[u].y = 0.0;
+            if (k + 1 < m) v[u] = *(const sp_d2u *)(xb + k);
+            else if (k < m) v[u].x = xb[k];
+        }
+        if (tid < nr) pn = part[tid * L.nseg + s];
+    };
+    load(0);
+    if (!between()) return false;
+    for (int s = 0; s * SP_SEG < len; s++) {
+        const int m = min(SP_SEG, len - s * SP_SEG);
+        if (s > 0) __syncthreads();  // the previous segment's readers are done
+#pragma unroll
+        for (int u = 0; u < SP_LOADS; u++) {
+            const int k = 2 * (tid + u * SP_TPB);
+            if (k < m) xs[k] = v[u].x;
+            if (k + 1 < m) xs[k + 1] = v[u].y;
+        }
+        if (tid == 0) xs[L.cap] = 0.0;
+        if (tid < nr) pt[tid] = pn;
+        __syncthreads();
+        SpBatch<W> b, c;
+        int2 p = q < nr ? pt[q] : make_int2(0, 0);
+        b.load(L, p.x + l, p.x + p.y);
+        if ((s + 1) * SP_SEG < len) load(s + 1);
+        for (int r = q; r < nr; r += SP_TPB / 16) {
+            const int end = p.x + p.y;
+            double acc = 0.0;
+            int g = p.x + l;
+            constexpr int step = 16 * SpBatch<W>::NB;
+            for (; g - l + step < end; g += step) {  // more of this part to come
+                c.load(L, g + step, end);
+                acc = b.dot(xs, acc);
+                b = c;
+            }
+            p = r + SP_TPB / 16 < nr ? pt[r + SP_TPB / 16] : make_int2(0, 0);
+            c.load(L, p.x + l, p.x + p.y);
+            acc = b.dot(xs, acc);
+            b = c;
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
+            if (l == 0) rowv[r] = s > 0 ? rowv[r] + acc : acc;
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
+// Q sums over the first nr threads of the work-group in a fixed order, written
+// by thread k < Q to out[k]; red: SP_TPB / 64 * Q doubles.
+template <int Q>
+__device__ __forceinline__ void sp_block_sums(double (&v)[Q], int nr, double *__restrict__ red, double *__restrict__ out)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = (nr + 63) >> 6;
+    if (w < nw) {
+#pragma unroll
+        for (int k = 0; k < Q; k++) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o);
+            if (lane == 0) red[w * Q + k] = v[k];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < Q) {
+        double s = 0.0;
+        for (int q = 0; q < nw; q++) s += red[q * Q + threadIdx.x];
+        out[threadIdx.x] = s;
+    }
+}
+
+// Sums of Q per-block partials part[f .. f + m)[Q], one wave per quantity, in
+// a fixed order (every thread gets them); tot: Q doubles.
+template <int Q>
+__device__ __forceinline__ void sp_partials(const double *__restrict__ part, int f, int m, double (&v)[Q],
+                                            double *__restrict__ tot)
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (w < Q) {
+        double s = 0.0;
+        for (int q = lane; q < m; q += 64) s += part[(long long)(f + q) * Q + w];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (lane == 0) tot[w] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < Q; k++) v[k] = tot[k];
+}
+
+}  // namespace pgdev

@@ -87,3 +87,42 @@ def test_clustering_zero_and_negative_weights(ctx):
         np.testing.assert_array_equal(np.isnan(c), np.isnan(oc))
         ok = ~np.isnan(oc)
         np.testing.assert_allclose(c[ok], oc[ok], rtol=1e-12, atol=0)
+
+
+# one, two and three 16,384-entry vector segments with rows that end inside a
+# group; a hub row longer than a batch of 256 entries
+@pytest.mark.parametrize("n,m,hub", [(5, 7, 0), (300, 9000, 299), (16384, 60000, 700), (16385, 60000, 700),
+                                     (33000, 90000, 2000)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_segmented_spmv(ctx, n, m, hub, weighted):
+    """Eigenvector centrality and modularity (both stops) over the segmented
+    SpMV: iteration counts and labels equal to the oracle's."""
+    row, col, val = _graph(n, m, 3 * n + m, hub)
+    v = val if weighted else None
+    say(f"segmented spmv n={n} nnz={col.size} weighted={weighted}")
+    vh, av, lam, it = ctx.eigenvector_centrality(row, col, v)
+    ovh, oav, olam, oit = O.ec(row, col, v)
+    assert it == oit
+    np.testing.assert_allclose(vh, ovh, rtol=1e-9, atol=1e-12)
+    np.testing.assert_allclose(av, oav, rtol=1e-9, atol=1e-12 * max(1.0, abs(olam)))
+    assert abs(lam - olam) <= 1e-9 * abs(olam)
+
+
+@pytest.mark.parametrize("n,m,hub", [(300, 9000, 299), (16385, 60000, 700), (33000, 90000, 2000)])
+@pytest.mark.parametrize("stop", [0, 1])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_segmented_modularity(ctx, n, m, hub, stop, weighted):
+    """One and two bisection levels over segmented groups; with the vector stop
+    the pass ends at the iteration cap (1, 2 and 40), where the launch that
+    stops is not the one after a test."""
+    row, col, val = _graph(n, m, 5 * n + m, hub)
+    v = val if weighted else None
+    for cap in ((1, 2, 40) if stop == 0 else (10000,)):
+        say(f"segmented modularity n={n} stop={stop} weighted={weighted} cap={cap}")
+        got = ctx.modularity(row, col, v, 0, stop=stop, max_iter=cap, max_depth=2)
+        want = O.modularity(row, col, v, 0, stop=stop, max_iter=cap, max_depth=2)
+        np.testing.assert_array_equal(got[0], want[0])
+        assert abs(got[1] - want[1]) <= 1e-9
+        assert abs(got[2] - want[2]) <= 1e-9 * max(1.0, abs(want[2]))
+        np.testing.assert_allclose(got[3], want[3], rtol=1e-7, atol=1e-9)
+        assert got[4] == want[4]
