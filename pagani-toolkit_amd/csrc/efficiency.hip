@@ -10,15 +10,19 @@
 //    pull launch: one wave per (vertex w, 64-word chunk), lane k owns word k of
 //    the chunk and ORs word k of every neighbour's visited set (512 contiguous
 //    bytes per neighbour per wave), stopping as soon as the bits w still lacks
-//    are all found.  New bits are the sources at distance exactly d+1.
+//    are all found.  New bits are the sources at distance exactly d+1.  A
+//    source that reached no vertex at one level is finished: w no longer looks
+//    for it (else every level would scan every row for the sources of other
+//    components).
 //  * Bit-sliced levels.  Bit b of the level at which (w, s) is reached is
 //    OR-ed into plane b, so a batch keeps ceil(log2(depth+1)) planes of S/8
 //    bytes per vertex instead of a byte or a float per pair.  Planes are
 //    allocated as the depth grows.
-//  * Ordered sums.  One lane per source walks j = 0..n-1 in order, rebuilds
-//    d(s, j) from the planes (wave-uniform words) and adds 1.0f / d in FP32
-//    -- the reference's precision and order, so e_s is bit-identical -- and
-//    (double)(1.0f / d) for j > s into the source's FP64 share of the Lp sum.
+//  * Ordered sums.  One lane per source adds 1.0f / d(s, j) in FP32 over j =
+//    0..n-1 in order -- the reference's precision and order, so e_s is
+//    bit-identical -- while other waves of its work-group rebuild the distances
+//    from the planes, and others add (double)(1.0f / d) for j > s into the
+//    source's FP64 share of the Lp sum.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,6 +30,7 @@
 #include <cstdlib>
 #include <vector>
 
+#include "pg_flag.hpp"
 #include "pg_internal.hpp"
 
 namespace {
@@ -40,9 +45,10 @@ struct Planes {
 };
 
 // visited words of a batch: vis[v * W + k]; sources base + 64k + b
-__global__ void eff_init(int n, int W, int base, int nsrc, u64 *__restrict__ vis)
+__global__ void eff_init(int n, int W, int base, int nsrc, u64 *__restrict__ vis, u64 *__restrict__ found)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < W) found[t] = 0ull;
     if (t >= (long long)n * W) return;
     const int v = (int)(t / W), k = (int)(t % W);
     const int lo = 64 * k;
@@ -61,36 +67,69 @@ __global__ void eff_zero(long long count, u64 *__restrict__ p)
     if (t < count) p[t] = 0ull;
 }
 
-// Level d -> d+1.  prog[d] counts waves that found new bits; a launch whose
-// previous level found none returns at once (the BFS has ended).
+// The sources that found a vertex at this level, collected by words; the load
+// keeps most waves' atomics away once a word is full.
+__device__ __forceinline__ void mark_found(u64 *f, u64 nb)
+{
+    if (nb & ~__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) atomicOr(f, nb);
+}
+
+// Level d -> d+1, d >= 1.  found holds three levels' source words: level d's
+// (written by the launch before), level d + 1's (cleared there, collected
+// here), and level d + 2's, cleared here.  chg[d & 1][v][c]: the words of chunk c
+// in which v got new bits at level d + 1; a neighbour matters only if it
+// changed in a word that w still looks for, since w took everything older at
+// the level before (a far source keeps a bit open in almost every row for
+// many levels, and each of those levels read 512 bytes of every neighbour).
+// n = 25,218, 6.4 M entries, depth 10: 8.5 ms over the levels (22.6 ms), of
+// which levels 1 and 2, which read nearly every neighbour, take 2.85 ms each.
+// prog[d] is raised when a wave found
+// new bits; a launch whose previous level found none returns at once (the BFS
+// has ended).
 __global__ __launch_bounds__(256) void eff_level(const int *__restrict__ row, const int *__restrict__ col, int n,
                                                  int W, int d, const u64 *__restrict__ visA,
                                                  u64 *__restrict__ visB, Planes planes, int nplanes,
+                                                 u64 *__restrict__ found, u64 *__restrict__ chg,
                                                  unsigned *__restrict__ prog)
 {
-    if (d > 0 && prog[d - 1] == 0u) return;
+    if (prog[d - 1] == 0u) return;
     const int lane = threadIdx.x & 63;
     const int chunks = W >> 6;
     const long long wid = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (wid < chunks) found[((d + 1) % 3) * W + wid * 64 + lane] = 0ull;
     if (wid >= (long long)n * chunks) return;
     const int w = __builtin_amdgcn_readfirstlane((int)(wid / chunks));
     const int c = __builtin_amdgcn_readfirstlane((int)(wid % chunks));
     const int k = (c << 6) + lane;
     const u64 vis = visA[(size_t)w * W + k];
-    const u64 need = ~vis;
+    const u64 need = ~vis & found[((d - 1) % 3) * W + k];
+    const u64 words = __ballot(need != 0);  // words of the chunk w still looks for
+    const u64 *cin = chg + (size_t)((d - 1) & 1) * n * chunks + c;
     u64 acc = 0;
-    if (need) {
+    if (words) {
         const int a = row[w], b = row[w + 1];
-        int e = a;
-        for (; e + 8 <= b; e += 8) {
-            u64 x = 0;
+        bool done = false;
+        for (int base = a; base < b && !done; base += 64) {
+            int v = 0;
+            u64 m = 0;
+            if (base + lane < b) {
+                v = col[base + lane];
+                m = cin[(size_t)v * chunks] & words;
+            }
+            u64 any = __ballot(m != 0);
+            while (any && !done) {
+                u64 x = 0;
 #pragma unroll
-            for (int q = 0; q < 8; q++) x |= visA[(size_t)col[e + q] * W + k];
-            acc |= x;
-            if ((acc & need) == need) break;
+                for (int q = 0; q < 8; q++) {
+                    if (any == 0) break;
+                    const int vv = __builtin_amdgcn_readlane(v, (int)__builtin_ctzll(any));
+                    any &= any - 1;
+                    if (need) x |= visA[(size_t)vv * W + k];
+                }
+                acc |= x;
+                done = __all((acc & need) == need);
+            }
         }
-        if ((acc & need) != need)
-            for (; e < b; e++) acc |= visA[(size_t)col[e] * W + k];
     }
     const u64 nb = acc & need;
     visB[(size_t)w * W + k] = vis | nb;
@@ -98,8 +137,13 @@ __global__ __launch_bounds__(256) void eff_level(const int *__restrict__ row, co
         const unsigned lv = (unsigned)d + 1u;
         for (int b = 0; b < nplanes; b++)
             if ((lv >> b) & 1u) planes.p[b][(size_t)w * W + k] |= nb;
+        mark_found(&found[(d % 3) * W + k], nb);
     }
-    if (__ballot(nb != 0) != 0 && lane == 0) atomicAdd(&prog[d], 1u);
+    const u64 fresh = __ballot(nb != 0);
+    if (lane == 0) {
+        chg[(size_t)(d & 1) * n * chunks + (size_t)w * chunks + c] = fresh;
+        if (fresh) pgdev::raise(&prog[d]);
+    }
 }
 
 // Level 0 -> 1 from the column indices alone: the sources at distance 1 from
@@ -111,12 +155,14 @@ __global__ __launch_bounds__(256) void eff_level(const int *__restrict__ row, co
 __global__ __launch_bounds__(256) void eff_level0(const int *__restrict__ row, const int *__restrict__ col, int n,
                                                   int W, int base, const u64 *__restrict__ visA,
                                                   u64 *__restrict__ visB, Planes planes,
-                                                  unsigned *__restrict__ prog)
+                                                  u64 *__restrict__ found, u64 *__restrict__ chg,
+                                                 unsigned *__restrict__ prog)
 {
     __shared__ u64 sbits[4][64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int chunks = W >> 6;
     const long long wid = (long long)blockIdx.x * 4 + wv;
+    if (wid < chunks) found[W + wid * 64 + lane] = 0ull;
     if (wid >= (long long)n * chunks) return;
     const int w = __builtin_amdgcn_readfirstlane((int)(wid / chunks));
     const int c = __builtin_amdgcn_readfirstlane((int)(wid % chunks));
@@ -150,68 +196,143 @@ __global__ __launch_bounds__(256) void eff_level0(const int *__restrict__ row, c
     const u64 vis = visA[(size_t)w * W + k];
     const u64 nb = acc & ~vis;
     visB[(size_t)w * W + k] = vis | nb;
-    if (nb) planes.p[0][(size_t)w * W + k] |= nb;
-    if (__ballot(nb != 0) != 0 && lane == 0) atomicAdd(&prog[0], 1u);
+    if (nb) {
+        planes.p[0][(size_t)w * W + k] |= nb;
+        mark_found(&found[k], nb);
+    }
+    const u64 fresh = __ballot(nb != 0);
+    if (lane == 0) {
+        chg[(size_t)w * chunks + c] = fresh;
+        if (fresh) pgdev::raise(&prog[0]);
+    }
 }
 
-// One wave per 64 sources (word k of the batch), one lane per source.  The
-// plane words of 64 consecutive j are fetched by one vector load per plane
-// (lane l holds j0 + l), then j walks them in order through readlane, so the
-// FP32 sums keep the reference's order while the loads are batched.
+// Work-group k sums 64 sources (word k of the batch).  The FP32 sum of a source
+// is a chain of n dependent adds, so one wave does nothing else: it adds
+// values that SUM_PROD waves put into LDS 64 vertices at a time (lane = vertex,
+// the source's bit of each plane -> level -> 1 / level from a table; rows of a
+// tile padded to 68 floats, so that lane = source then reads four in one
+// conflict-free access), and two waves take the FP64 shares of alternate
+// tiles.  Two sets of tiles, one barrier per round of 64 SUM_PROD vertices.
+// n = 25,218, four planes: 0.84 ms (4.4 ms with one wave per 64 sources that
+// did all of it).
+constexpr int SUM_PROD = 4, SUM_TPB = 64 * (3 + SUM_PROD), SUM_LD = 68;
+constexpr size_t SUM_LDS = (size_t)2 * SUM_PROD * 64 * SUM_LD * 4 + 256 * 4;
 template <int NP>
-__global__ __launch_bounds__(64) void eff_sum(int n, int W, int base, int nsrc, Planes planes,
-                                              float *__restrict__ eff, double *__restrict__ lpp,
-                                              int *__restrict__ flags)
+__global__ __launch_bounds__(SUM_TPB) void eff_sum(int n, int W, int base, int nsrc, Planes planes,
+                                                   float *__restrict__ eff, double *__restrict__ lpp,
+                                                   int *__restrict__ flags)
 {
-    const int lane = threadIdx.x;
+    extern __shared__ __align__(16) float sm[];
+    __shared__ double dpart[64];
+    __shared__ int rpart[64];
+    float *rtab = sm + 2 * SUM_PROD * 64 * SUM_LD;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int k = blockIdx.x;
     const int s = base + 64 * k + lane;
+    constexpr bool TAB = NP <= 8;
+    if (TAB && threadIdx.x < (1 << (TAB ? NP : 0))) rtab[threadIdx.x] = threadIdx.x ? 1.0f / (float)(int)threadIdx.x : 0.0f;
+    const int rounds = (n + 64 * SUM_PROD - 1) / (64 * SUM_PROD);
+    const int p = wv - 3;  // producer
+    u64 w[NP];
+    auto fetch = [&](int r) {
+        const int j = (r * SUM_PROD + p) * 64 + lane;
+#pragma unroll
+        for (int b = 0; b < NP; b++) w[b] = j < n ? planes.p[b][(size_t)j * W + k] : 0ull;
+    };
+    if (p >= 0) fetch(0);
     float acc = 0.0f;
     double dacc = 0.0;
     int reached = 0;
-    for (int j0 = 0; j0 < n; j0 += 64) {
-        const int jl = j0 + lane;
-        uint32_t wlo[NP], whi[NP];
+    __syncthreads();
+    for (int r = 0; r <= rounds; r++) {
+        if (p >= 0) {
+            if (r < rounds) {
+                float *t = sm + ((r & 1) * SUM_PROD + p) * 64 * SUM_LD + lane;
+                uint32_t lo[NP], hi[NP];
 #pragma unroll
-        for (int b = 0; b < NP; b++) {
-            const u64 x = jl < n ? planes.p[b][(size_t)jl * W + k] : 0ull;
-            wlo[b] = (uint32_t)x;
-            whi[b] = (uint32_t)(x >> 32);
-        }
-        const int cnt = min(64, n - j0);
-        for (int jj = 0; jj < cnt; jj++) {
-            int lv = 0;
+                for (int b = 0; b < NP; b++) {
+                    lo[b] = (uint32_t)w[b];
+                    hi[b] = (uint32_t)(w[b] >> 32);
+                }
+                if (r + 1 < rounds) fetch(r + 1);
+#pragma unroll 8
+                for (int q = 0; q < 32; q++) {
+                    int l0 = 0, l1 = 0;
 #pragma unroll
-            for (int b = 0; b < NP; b++) {
-                const uint32_t lo = __builtin_amdgcn_readlane(wlo[b], jj);
-                const uint32_t hi = __builtin_amdgcn_readlane(whi[b], jj);
-                const uint32_t word = lane < 32 ? lo : hi;
-                lv |= (int)((word >> (lane & 31)) & 1u) << b;
+                    for (int b = 0; b < NP; b++) {
+                        l0 |= (int)((lo[b] >> q) & 1u) << b;
+                        l1 |= (int)((hi[b] >> q) & 1u) << b;
+                    }
+                    if (TAB) {
+                        t[q * SUM_LD] = rtab[l0];
+                        t[(q + 32) * SUM_LD] = rtab[l1];
+                    } else {
+                        t[q * SUM_LD] = l0 ? 1.0f / (float)l0 : 0.0f;
+                        t[(q + 32) * SUM_LD] = l1 ? 1.0f / (float)l1 : 0.0f;
+                    }
+                }
             }
-            if (lv != 0) {
-                const float r = 1.0f / (float)lv;
-                acc += r;
-                reached++;
-                if (j0 + jj > s) dacc += (double)r;
+        } else if (r > 0) {
+            const float *t0 = sm + ((r - 1) & 1) * SUM_PROD * 64 * SUM_LD + lane * SUM_LD;
+            if (wv == 0) {
+                for (int q = 0; q < SUM_PROD; q++) {
+                    const float4 *t = (const float4 *)(t0 + q * 64 * SUM_LD);
+#pragma unroll
+                    for (int j = 0; j < 16; j++) {
+                        const float4 v = t[j];
+                        acc += v.x;
+                        acc += v.y;
+                        acc += v.z;
+                        acc += v.w;
+                    }
+                }
+            } else {
+                for (int q = wv - 1; q < SUM_PROD; q += 2) {
+                    const float4 *t = (const float4 *)(t0 + q * 64 * SUM_LD);
+                    const int j0 = ((r - 1) * SUM_PROD + q) * 64 - s;  // j > s: j - s > 0
+#pragma unroll 4
+                    for (int j = 0; j < 16; j++) {
+                        const float4 v = t[j];
+                        reached += (v.x != 0.0f) + (v.y != 0.0f) + (v.z != 0.0f) + (v.w != 0.0f);
+                        dacc += j0 + 4 * j > 0 ? (double)v.x : 0.0;
+                        dacc += j0 + 4 * j + 1 > 0 ? (double)v.y : 0.0;
+                        dacc += j0 + 4 * j + 2 > 0 ? (double)v.z : 0.0;
+                        dacc += j0 + 4 * j + 3 > 0 ? (double)v.w : 0.0;
+                    }
+                }
             }
         }
+        __syncthreads();
     }
+    if (wv == 2) {
+        dpart[lane] = dacc;
+        rpart[lane] = reached;
+    }
+    __syncthreads();
     if (64 * k + lane >= nsrc) return;
-    const float e = acc / (float)(n - 1);
-    eff[s] = e;
-    lpp[s] = dacc;
-    if (e == 0.0f) atomicAdd(&flags[0], 1);
-    if (reached < n - 1) atomicOr(&flags[1], 1);
+    if (wv == 0) {
+        const float e = acc / (float)(n - 1);
+        eff[s] = e;
+        if (e == 0.0f) atomicAdd(&flags[0], 1);
+    } else if (wv == 1) {
+        lpp[s] = dacc + dpart[lane];
+        if (reached + rpart[lane] < n - 1) atomicOr(&flags[1], 1);
+    }
 }
 
 template <int NP>
-void launch_sum(hipStream_t st, int n, int W, int base, int nsrc, const Planes &pl, float *eff, double *lpp,
-                int *flags)
+hipError_t launch_sum(hipStream_t st, int n, int W, int base, int nsrc, const Planes &pl, float *eff, double *lpp,
+                      int *flags)
 {
-    eff_sum<NP><<<(unsigned)(W), 64, 0, st>>>(n, W, base, nsrc, pl, eff, lpp, flags);
+    const hipError_t e = hipFuncSetAttribute((const void *)eff_sum<NP>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             (int)SUM_LDS);
+    if (e != hipSuccess) return e;
+    eff_sum<NP><<<(unsigned)((nsrc + 63) / 64), SUM_TPB, SUM_LDS, st>>>(n, W, base, nsrc, pl, eff, lpp, flags);
+    return hipGetLastError();
 }
 
-typedef void (*SumFn)(hipStream_t, int, int, int, int, const Planes &, float *, double *, int *);
+typedef hipError_t (*SumFn)(hipStream_t, int, int, int, int, const Planes &, float *, double *, int *);
 
 SumFn sum_fn(int np)
 {
@@ -266,13 +387,15 @@ extern "C" pg_status pg_bfs_efficiency(pg_ctx *ctx, const int32_t *row, const in
     if (env && std::atoi(env) > 0) S = (int)std::min<long long>(pg_cdiv(std::atoi(env), 4096) * 4096, S);
     const int W = S / 64;
     const size_t words = (size_t)n * W;
-    u64 *va, *vb;
+    u64 *va, *vb, *found, *chg;
     unsigned *prog;
     float *deff;
     double *lpp;
     int *flags;
     PG_TRY(pg_bufT(ctx, "eff.visA", words, &va));
     PG_TRY(pg_bufT(ctx, "eff.visB", words, &vb));
+    PG_TRY(pg_bufT(ctx, "eff.found", (size_t)3 * W, &found));
+    PG_TRY(pg_bufT(ctx, "eff.chg", (size_t)2 * n * (W / 64), &chg));
     PG_TRY(pg_bufT(ctx, "eff.prog", (size_t)n + LEVEL_GROUP + 2, &prog));
     PG_TRY(pg_bufT(ctx, "eff.lpp", (size_t)n, &lpp));
     PG_TRY(pg_bufT(ctx, "eff.flags", 2, &flags));
@@ -298,7 +421,7 @@ extern "C" pg_status pg_bfs_efficiency(pg_ctx *ctx, const int32_t *row, const in
         for (int b = 0; b < nplanes; b++)
             eff_zero<<<(unsigned)pg_cdiv((long long)words, 256), 256, 0, st>>>((long long)words, pl.p[b]);
         PG_HIP(ctx, hipMemsetAsync(prog, 0, ((size_t)n + LEVEL_GROUP + 2) * 4, st));
-        eff_init<<<(unsigned)pg_cdiv((long long)words, 256), 256, 0, st>>>(n, W, base, nsrc, va);
+        eff_init<<<(unsigned)pg_cdiv((long long)words, 256), 256, 0, st>>>(n, W, base, nsrc, va, found);
         PG_KERNEL_CHECK(ctx);
         const unsigned blocks = (unsigned)pg_cdiv((long long)n * (W / 64), 4);
         int depth = -1;
@@ -309,9 +432,9 @@ extern "C" pg_status pg_bfs_efficiency(pg_ctx *ctx, const int32_t *row, const in
             PG_TRY(grow(bit_width((unsigned)top)));
             for (int q = 0; q < LEVEL_GROUP; q++) {
                 if (d + q == 0)
-                    eff_level0<<<blocks, 256, 0, st>>>(drow, dcol, n, W, base, va, vb, pl, prog);
+                    eff_level0<<<blocks, 256, 0, st>>>(drow, dcol, n, W, base, va, vb, pl, found, chg, prog);
                 else
-                    eff_level<<<blocks, 256, 0, st>>>(drow, dcol, n, W, d + q, va, vb, pl, nplanes, prog);
+                    eff_level<<<blocks, 256, 0, st>>>(drow, dcol, n, W, d + q, va, vb, pl, nplanes, found, chg, prog);
                 std::swap(va, vb);
             }
             PG_KERNEL_CHECK(ctx);
@@ -322,8 +445,7 @@ extern "C" pg_status pg_bfs_efficiency(pg_ctx *ctx, const int32_t *row, const in
                 if (h[q] == 0) depth = d + q;  // deepest level present
         }
         const int np = std::max(1, bit_width((unsigned)depth));
-        sum_fn(np)(st, n, W, base, nsrc, pl, deff, lpp, flags);
-        PG_KERNEL_CHECK(ctx);
+        PG_HIP(ctx, sum_fn(np)(st, n, W, base, nsrc, pl, deff, lpp, flags));
     }
     PG_TRY(pg_out_finish(ctx, eff, deff, (size_t)n));
     std::vector<double> h((size_t)n);

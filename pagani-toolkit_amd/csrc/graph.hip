@@ -20,6 +20,7 @@
 #include <mutex>
 #include <vector>
 
+#include "pg_flag.hpp"
 #include "pg_internal.hpp"
 
 namespace {
@@ -450,8 +451,8 @@ struct BatchBufs {
     u64 *sigma, *visA, *visB, *p0, *p1;
     int *lev, *srcs;
     double *coef, *bcpart;
-    unsigned *prog;        // [nb][lcap]: waves that found new vertices at level d + 1
-    unsigned *tot;         // [lcap]: the same summed over the batches
+    unsigned *prog;        // [nb][lcap]: 1 when some wave found new vertices at level d + 1
+    unsigned *tot;         // [lcap]: the same over all batches
 };
 
 __global__ void bfs_init(int n, BatchBufs B)
@@ -560,8 +561,8 @@ __global__ __launch_bounds__(256) void bfs_forward(const int *__restrict__ row, 
         if (nbits) {
             if ((d + 1) & 1) B.p0[vb0 + w] |= nbits;
             if ((d + 1) & 2) B.p1[vb0 + w] |= nbits;
-            atomicAdd(&prog[d], 1u);
-            atomicAdd(&B.tot[d], 1u);
+            pgdev::raise(&prog[d]);
+            pgdev::raise(&B.tot[d]);
         }
     }
 }

@@ -126,3 +126,32 @@ def test_segmented_modularity(ctx, n, m, hub, stop, weighted):
         assert abs(got[2] - want[2]) <= 1e-9 * max(1.0, abs(want[2]))
         np.testing.assert_allclose(got[3], want[3], rtol=1e-7, atol=1e-9)
         assert got[4] == want[4]
+
+
+# one and two 4,096-source chunks; work-groups whose last round of 256 vertices
+# is whole (512, 4,096) or ragged
+@pytest.mark.parametrize("n,m,tail", [(70, 200, 10), (512, 3000, 20), (4096, 30000, 3), (4500, 40000, 300)])
+def test_efficiency_components_and_tails(ctx, n, m, tail):
+    """A random part, a chain hanging off it (sources that stay active for many
+    levels), a separate triangle and isolated vertices."""
+    rng = np.random.default_rng(n)
+    core = n - tail - 8
+    a, b = rng.integers(0, core, m), rng.integers(0, core, m)
+    c = np.arange(core, core + tail)
+    t = core + tail
+    a = np.concatenate([a, [0], c[:-1], [t, t + 1, t + 2]])
+    b = np.concatenate([b, [c[0]], c[1:], [t + 1, t + 2, t]])
+    perm = rng.permutation(n)  # t + 3 .. n - 1 stay isolated
+    a, b = perm[a], perm[b]
+    lo, hi = np.minimum(a, b), np.maximum(a, b)
+    key = np.unique(lo[lo != hi] * np.int64(n) + hi[lo != hi])
+    lo, hi = key // n, key % n
+    both = np.sort(np.concatenate([key, hi * n + lo]))
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(both // n, minlength=n))
+    col = (both % n).astype(np.int32)
+    say(f"efficiency components n={n} tail={tail}")
+    e, lp, iso, unc = ctx.bfs_efficiency(row, col)
+    oe, olp, oiso, ounc = O.bfs_efficiency(row, col)
+    np.testing.assert_array_equal(e.view(np.uint32), oe.view(np.uint32))
+    assert abs(lp - olp) <= 1e-12 * abs(olp) and (iso, unc) == (oiso, ounc)
