@@ -26,10 +26,8 @@
 // thresholds as the reference applies them to the averaged matrix: r-mode
 // keeps a > thr; s-mode keeps the k largest with the earliest (row-major) ties
 // at the k-th value, found by a 3-pass radix select over the M1 values.  The
-// CSR is built in order without sorting: a per-pair keep byte in packed order,
-// then one work-group per 64 CSR rows that reads the lower part of its rows as
-// 64-byte slices of the packed rows above it (column order for free) and the
-// upper part from the rows' own packed segments.
+// kept pairs are listed row by row and go through the construction's counting
+// sort (pg_csr_pairs).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -370,28 +368,30 @@ __global__ __launch_bounds__(1024) void cm_scan(const int *__restrict__ in, int 
     pgdev::block_scan_1024(in, n, out, 1);
 }
 
-// Keep byte per pair in packed order; ties at the bound are kept while their
-// row-major rank (tbase[i] + rank inside the row) is below ntie.  cu[i] = kept
-// pairs of packed row i.
-__global__ __launch_bounds__(256) void cm_keep(const float *__restrict__ a, int n, float bound, int ties,
-                                               const long long *__restrict__ tbase, long long ntie,
-                                               uint8_t *__restrict__ keep, int *__restrict__ cu)
+// The kept pairs (and values) of packed row i at base[i] on: values above the
+// bound, and ties at it while their row-major rank (tbase[i] + rank inside the
+// row) is below ntie; with ties the kept ties of earlier rows shift base[i],
+// which counts the values above only.
+__global__ __launch_bounds__(256) void cm_pairs(const float *__restrict__ a, int n, float bound, int ties,
+                                                const long long *__restrict__ base, const long long *__restrict__ tbase,
+                                                long long ntie, int2 *__restrict__ pairs, float *__restrict__ w)
 {
     // one packed row per wave, 64 pairs per step and four steps in flight; tie
     // ranks advance in column order by ballot, with no block barriers
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const int i = blockIdx.x * 4 + wv;
     if (i >= n) return;
-    const long long base = pidx(i, i + 1, n);
+    const long long b = pidx(i, i + 1, n);
     const int len = n - 1 - i;
+    const u64 below = (1ull << lane) - 1ull;
     long long rank = ties ? tbase[i] : 0;
-    int nk = 0;
+    long long at = base[i] + (ties ? min(rank, ntie) : 0);
     for (int q0 = 0; q0 < len; q0 += 4 * 64) {
         float x[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
             const int q = q0 + 64 * u + lane;
-            x[u] = q < len ? a[base + q] : 0.0f;
+            x[u] = q < len ? a[b + q] : 0.0f;
         }
 #pragma unroll
         for (int u = 0; u < 4; u++) {
@@ -399,125 +399,17 @@ __global__ __launch_bounds__(256) void cm_keep(const float *__restrict__ a, int 
             const bool in = q < len;
             const bool gt = in && x[u] > bound, tie = in && ties && x[u] == bound;
             const u64 tm = __ballot(tie);
-            const long long r = rank + __popcll(tm & ((1ull << lane) - 1ull));
-            const bool k = gt || (tie && r < ntie);
-            if (in) keep[base + q] = k ? 1 : 0;
-            nk += __popcll(__ballot(k));
+            const bool k = gt || (tie && rank + __popcll(tm & below) < ntie);
+            const u64 km = __ballot(k);
+            if (k) {
+                const long long p = at + __popcll(km & below);
+                pairs[p] = make_int2(i, i + 1 + q);
+                if (w) w[p] = x[u];
+            }
             rank += __popcll(tm);
+            at += __popcll(km);
         }
     }
-    if (lane == 0) cu[i] = nk;
-}
-
-// One work-group per 64 CSR rows [i0, i0 + 64).  Count pass (rowptr == NULL):
-// cl[i] = kept pairs (j, i) with j < i.  Fill pass: writes row i as its lower
-// part (ascending j < i) followed by its upper part (ascending j > i).
-__global__ __launch_bounds__(256) void cm_csr_group(const uint8_t *__restrict__ keep, const float *__restrict__ a,
-                                                    int n, const long long *__restrict__ rowptr,
-                                                    int *__restrict__ cl, int *__restrict__ col,
-                                                    float *__restrict__ val)
-{
-    __shared__ int run[64];
-    __shared__ int wcnt[4][64];
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const int i0 = blockIdx.x * 64;
-    const int nr = min(64, n - i0);
-    if (tid < 64) run[tid] = 0;
-    __syncthreads();
-    // lower parts: packed rows j = 0 .. i0 + nr - 2
-    const int jend = i0 + nr - 1;
-    for (int j0 = 0; j0 < jend; j0 += 256) {
-        const int j = j0 + tid;
-        u64 mask = 0;
-        if (j < jend) {
-            // rows r with i0 + r > j; their bytes are contiguous in packed row j:
-            // fetched as at most five aligned 16-byte words (only those that
-            // overlap [b, b + cnt), so no read passes b + cnt + 15), then
-            // unpacked by compile-time byte position
-            const int r0 = j >= i0 ? j - i0 + 1 : 0;
-            const long long b = pidx(j, i0 + r0, n);
-            const long long b16 = b & ~15ll;
-            const int off = (int)(b - b16), cnt = nr - r0;
-            uint4 wd[5];
-#pragma unroll
-            for (int q = 0; q < 5; q++)
-                wd[q] = 16 * q < off + cnt ? *(const uint4 *)(keep + b16 + 16 * q) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int q = 0; q < 5; q++) {
-                const unsigned w4[4] = {wd[q].x, wd[q].y, wd[q].z, wd[q].w};
-#pragma unroll
-                for (int p = 0; p < 16; p++) {
-                    const int r = 16 * q + p - off + r0;  // row of byte 16q + p
-                    const bool set = ((w4[p >> 2] >> (8 * (p & 3))) & 0xffu) != 0u;
-                    if (set && r >= r0 && r < nr) mask |= 1ull << r;
-                }
-            }
-        }
-        for (int r = 0; r < nr; r++) {
-            const u64 bm = __ballot((mask >> r) & 1ull);
-            if (lane == 0) wcnt[wv][r] = __popcll(bm);
-        }
-        __syncthreads();
-        if (rowptr) {
-            for (int r = 0; r < nr; r++) {
-                const u64 bm = __ballot((mask >> r) & 1ull);
-                if ((mask >> r) & 1ull) {
-                    int pos = run[r] + __popcll(bm & ((1ull << lane) - 1ull));
-                    for (int w = 0; w < wv; w++) pos += wcnt[w][r];
-                    const long long at = rowptr[i0 + r] + pos;
-                    col[at] = j;
-                    if (val) val[at] = a[pidx(j, i0 + r, n)];
-                }
-            }
-        }
-        __syncthreads();
-        if (tid < nr) run[tid] += wcnt[0][tid] + wcnt[1][tid] + wcnt[2][tid] + wcnt[3][tid];
-        __syncthreads();
-    }
-    if (!rowptr) {
-        if (tid < nr) cl[i0 + tid] = run[tid];
-        return;
-    }
-    // upper parts: packed segment of row i, j = i+1 .. n-1, one row per wave
-    // (no block barriers), 64 bytes per step and four steps in flight, each
-    // kept column placed by its rank in the step's ballot
-    for (int r = wv; r < nr; r += 4) {
-        const int i = i0 + r;
-        const long long b = pidx(i, i + 1, n);
-        const int len = n - 1 - i;
-        long long pos = rowptr[i] + cl[i];
-        for (int q0 = 0; q0 < len; q0 += 4 * 64) {
-            bool k[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const int q = q0 + 64 * u + lane;
-                k[u] = q < len && keep[b + q];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const u64 bm = __ballot(k[u]);
-                if (k[u]) {
-                    const int q = q0 + 64 * u + lane;
-                    const long long at = pos + __popcll(bm & ((1ull << lane) - 1ull));
-                    col[at] = i + 1 + q;
-                    if (val) val[at] = a[b + q];
-                }
-                pos += __popcll(bm);
-            }
-        }
-    }
-}
-
-__global__ void cm_degrees(int n, const int *__restrict__ cl, const int *__restrict__ cu, int *__restrict__ deg)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) deg[i] = cl[i] + cu[i];
-}
-
-__global__ void cm_rowptr(int n, const long long *__restrict__ p, int *__restrict__ row)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i <= n) row[i] = (int)p[i];
 }
 
 pg_status need_matrix(pg_ctx *ctx)
@@ -639,13 +531,12 @@ extern "C" pg_status pg_cormat_threshold(pg_ctx *ctx, int32_t thr_kind, float th
     inf.n = n;
     float bound = thr;
     long long kwant = 0, ntie = 0;
-    int *cgt, *ctie, *cu, *cl, *deg;
+    if (!pg_csr_pairs_ok(ctx, n)) return pg_fail(ctx, PG_ENOTSUP, "n=%d exceeds the row-sort LDS", n);
+    const bool smode = thr_kind == PG_THR_SPARSITY;
+    int *cgt, *ctie;
     long long *tbase, *rp;
     PG_TRY(pg_bufT(ctx, "cm.cgt", (size_t)n, &cgt));
     PG_TRY(pg_bufT(ctx, "cm.ctie", (size_t)n, &ctie));
-    PG_TRY(pg_bufT(ctx, "cm.cu", (size_t)n, &cu));
-    PG_TRY(pg_bufT(ctx, "cm.cl", (size_t)n, &cl));
-    PG_TRY(pg_bufT(ctx, "cm.deg", (size_t)n, &deg));
     PG_TRY(pg_bufT(ctx, "cm.tbase", (size_t)n + 1, &tbase));
     PG_TRY(pg_bufT(ctx, "cm.rp", (size_t)n + 1, &rp));
     if (thr_kind == PG_THR_SPARSITY) {
@@ -672,14 +563,16 @@ extern "C" pg_status pg_cormat_threshold(pg_ctx *ctx, int32_t thr_kind, float th
         PG_HIP(ctx, hipMemcpyAsync(&hs, ss, sizeof hs, hipMemcpyDeviceToHost, st));
         PG_HIP(ctx, hipStreamSynchronize(st));
         bound = key_float(hs.prefix);
-        cm_row_counts<<<(unsigned)n, 256, 0, st>>>(a, n, bound, cgt, ctie);
-        cm_scan<<<1, 1024, 0, st>>>(cgt, n, rp);
-        cm_scan<<<1, 1024, 0, st>>>(ctie, n, tbase);
-        PG_KERNEL_CHECK(ctx);
-        long long totgt = 0, tottie = 0;
-        PG_HIP(ctx, hipMemcpyAsync(&totgt, rp + n, 8, hipMemcpyDeviceToHost, st));
-        PG_HIP(ctx, hipMemcpyAsync(&tottie, tbase + n, 8, hipMemcpyDeviceToHost, st));
-        PG_HIP(ctx, hipStreamSynchronize(st));
+    }
+    cm_row_counts<<<(unsigned)n, 256, 0, st>>>(a, n, bound, cgt, ctie);
+    cm_scan<<<1, 1024, 0, st>>>(cgt, n, rp);
+    if (smode) cm_scan<<<1, 1024, 0, st>>>(ctie, n, tbase);
+    PG_KERNEL_CHECK(ctx);
+    long long totgt = 0, tottie = 0;
+    PG_HIP(ctx, hipMemcpyAsync(&totgt, rp + n, 8, hipMemcpyDeviceToHost, st));
+    if (smode) PG_HIP(ctx, hipMemcpyAsync(&tottie, tbase + n, 8, hipMemcpyDeviceToHost, st));
+    PG_HIP(ctx, hipStreamSynchronize(st));
+    if (smode) {
         ntie = kwant - totgt;
         if (ntie < 1 || ntie > tottie)
             return pg_fail(ctx, PG_ETHRESH, "selection mismatch: %lld above, %lld ties, %lld wanted", totgt, tottie,
@@ -691,30 +584,28 @@ extern "C" pg_status pg_cormat_threshold(pg_ctx *ctx, int32_t thr_kind, float th
         inf.r_thresh = thr;
         inf.t_star = (double)thr;
     }
-    uint8_t *keep;
-    PG_TRY(pg_bufT(ctx, "cm.keep", (size_t)m1, &keep));
-    cm_keep<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(a, n, bound, thr_kind == PG_THR_SPARSITY, tbase, ntie, keep,
-                                                      cu);
-    const int ng = (int)pg_cdiv(n, 64);
-    cm_csr_group<<<(unsigned)ng, 256, 0, st>>>(keep, a, n, nullptr, cl, nullptr, nullptr);
-    cm_degrees<<<(unsigned)pg_cdiv(n, 256), 256, 0, st>>>(n, cl, cu, deg);
-    cm_scan<<<1, 1024, 0, st>>>(deg, n, rp);
-    PG_KERNEL_CHECK(ctx);
-    long long nnz = 0;
-    PG_HIP(ctx, hipMemcpyAsync(&nnz, rp + n, 8, hipMemcpyDeviceToHost, st));
-    PG_HIP(ctx, hipStreamSynchronize(st));
+    const long long kept = totgt + ntie, nnz = 2 * kept;
     if (nnz > INT32_MAX) return pg_fail(ctx, PG_ENOTSUP, "nnz %lld exceeds int32 CSR", nnz);
-    if (thr_kind == PG_THR_SPARSITY && nnz != 2 * kwant)
-        return pg_fail(ctx, PG_ETHRESH, "CSR holds %lld entries, %lld wanted", nnz, 2 * kwant);
+    // kept pairs, then the construction's counting sort (the row groups that
+    // picked each row's lower part out of keep bytes took 1.06 ms of 4.6 at n =
+    // 12,011: 188 work-groups, twice)
+    int2 *pairs;
     int *row, *col;
-    float *val = nullptr;
+    float *val = nullptr, *w = nullptr;
+    PG_TRY(pg_bufT(ctx, "cm.pairs", (size_t)std::max<long long>(kept, 1), &pairs));
     PG_TRY(pg_bufT(ctx, "cm.row", (size_t)n + 1, &row));
     PG_TRY(pg_bufT(ctx, "cm.col", (size_t)std::max<long long>(nnz, 1), &col));
-    if (weighted) PG_TRY(pg_bufT(ctx, "cm.val", (size_t)std::max<long long>(nnz, 1), &val));
-    cm_rowptr<<<(unsigned)pg_cdiv(n + 1, 256), 256, 0, st>>>(n, rp, row);
-    cm_csr_group<<<(unsigned)ng, 256, 0, st>>>(keep, a, n, rp, cl, col, val);
+    if (weighted) {
+        PG_TRY(pg_bufT(ctx, "cm.w", (size_t)std::max<long long>(kept, 1), &w));
+        PG_TRY(pg_bufT(ctx, "cm.val", (size_t)std::max<long long>(nnz, 1), &val));
+    }
+    cm_pairs<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(a, n, bound, smode, rp, tbase, ntie, pairs, w);
     PG_KERNEL_CHECK(ctx);
+    PG_TRY(pg_csr_pairs(ctx, "cm.", pairs, w, kept, n, row, col, val));
+    int rn = 0;
+    PG_HIP(ctx, hipMemcpyAsync(&rn, row + n, 4, hipMemcpyDeviceToHost, st));
     PG_HIP(ctx, hipStreamSynchronize(st));
+    if (rn != nnz) return pg_fail(ctx, PG_ETHRESH, "CSR holds %d entries, %lld wanted", rn, nnz);
     if (thr_kind == PG_THR_R) inf.s_thresh = (float)(100.0 * nnz / m1 / 2);
     inf.nnz = nnz;
     ctx->cn = n;

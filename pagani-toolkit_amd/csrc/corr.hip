@@ -3450,6 +3450,76 @@ __global__ __launch_bounds__(256) void sp_report(const unsigned long long *__res
     }
 }
 
+// The CSR of n vertices from the nsrc sources of src (nnz entries; weights
+// beside the lists when weighted), launched without a host check; row[n]
+// reports the entries found.  Work buffers are named pfx + ...
+pg_status csr_launch(pg_ctx *ctx, const char *pfx, const EdgeSrc &src, int n, int nsrc, bool weighted, long long nnz,
+                     bool seg_counted, int *row, int *col, float *val)
+{
+    hipStream_t st = ctx->stream;
+    const std::string p = pfx;
+    const size_t nnzs = (size_t)std::max<long long>(nnz, 1);
+    const int nbk = (int)pg_cdiv(n, BROWS);
+    unsigned *bcnt, *ent;
+    long long *boff, *bstart, *btot;
+    int *ctmp = nullptr;
+    float *entv = nullptr, *vtmp = nullptr;
+    PG_TRY(pg_bufT(ctx, (p + "bcnt").c_str(), (size_t)nsrc * nbk, &bcnt));
+    PG_TRY(pg_bufT(ctx, (p + "boff").c_str(), (size_t)nsrc * nbk, &boff));
+    PG_TRY(pg_bufT(ctx, (p + "bstart").c_str(), (size_t)nbk + 1, &bstart));
+    PG_TRY(pg_bufT(ctx, (p + "btot").c_str(), (size_t)nbk + 1, &btot));
+    PG_TRY(pg_bufT(ctx, (p + "ent").c_str(), nnzs, &ent));
+    const BitsPlan bp = weighted ? BitsPlan() : rows_bits_plan(n, ctx->lds_per_block);
+    const size_t lbits = bp.lds;
+    if (!lbits) PG_TRY(pg_bufT(ctx, (p + "ctmp").c_str(), nnzs, &ctmp));
+    if (weighted) {
+        PG_TRY(pg_bufT(ctx, (p + "entv").c_str(), nnzs, &entv));
+        PG_TRY(pg_bufT(ctx, (p + "vtmp").c_str(), nnzs, &vtmp));
+    }
+    const size_t shb = (size_t)nbk * 4;
+    if (!seg_counted) {
+        if (shb > 64 * 1024) PG_HIP(ctx, set_shared_limit(ctx, (const void *)bucket_count, shb));
+        bucket_count<<<(unsigned)nsrc, SEG_THREADS, shb, st>>>(src, nbk, 0, nsrc, bcnt);
+    }
+    bucket_scan_local<<<(unsigned)pg_cdiv(nbk, SCAN_BK), SCAN_BK * SCAN_SG, 0, st>>>(bcnt, nsrc, nbk, boff, btot);
+    bucket_scan_global<<<1, 1024, 0, st>>>(btot, nbk, bstart);
+    const size_t shs = (size_t)nbk * (4 + 4);  // bases + cursors
+    const void *scatter_fn = weighted ? (const void *)bucket_scatter<true> : (const void *)bucket_scatter<false>;
+    if (shs > 64 * 1024) PG_HIP(ctx, set_shared_limit(ctx, scatter_fn, shs));
+    if (weighted)
+        bucket_scatter<true><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, entv,
+                                                                       (long long)nnzs);
+    else
+        bucket_scatter<false><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, nullptr,
+                                                                        (long long)nnzs);
+    if (lbits) {
+        PG_HIP(ctx, set_shared_limit(ctx, rows_bits_fn(bp.rank), (int)lbits));
+        launch_rows_bits(ctx, bp, st, bstart, ent, n, nbk, row, col, (long long)nnzs);
+        PG_KERNEL_CHECK(ctx);
+        return PG_OK;
+    }
+    const RowsPlan rp = rows_plan(n, ctx->lds_per_block);
+    if (rp.nbm == 0) return pg_fail(ctx, PG_ENOTSUP, "n = %d: the row bitmap does not fit LDS", n);
+    const void *rows_fn = weighted ? (const void *)bucket_rows<true> : (const void *)bucket_rows<false>;
+    PG_HIP(ctx, set_shared_limit(ctx, rows_fn, rp.lds));
+    if (weighted)
+        bucket_rows<true><<<(unsigned)nbk, ROWS_THREADS, rp.lds, st>>>(bstart, ent, entv, n, nbk, rp.nbm, rp.dbit, row,
+                                                                       ctmp, vtmp, col, val, (long long)nnzs);
+    else
+        bucket_rows<false><<<(unsigned)nbk, ROWS_THREADS, rp.lds, st>>>(bstart, ent, nullptr, n, nbk, rp.nbm, rp.dbit,
+                                                                        row, ctmp, nullptr, col, nullptr,
+                                                                        (long long)nnzs);
+    PG_KERNEL_CHECK(ctx);
+    return PG_OK;
+}
+
+// cnt[g] = entries of segment g of a list of m cut every cap entries
+__global__ void slice_counts(long long m, long long cap, int nseg, unsigned long long *__restrict__ cnt)
+{
+    const int g = blockIdx.x * blockDim.x + threadIdx.x;
+    if (g < nseg) cnt[g] = (unsigned long long)max(0ll, min(cap, m - g * cap));
+}
+
 struct CorrRun {
     pg_ctx *ctx = nullptr;
     hipStream_t st = nullptr;
@@ -3741,65 +3811,16 @@ struct CorrRun {
     {
         if (nnz > INT32_MAX) return pg_fail(ctx, PG_ENOTSUP, "nnz %lld exceeds int32 CSR", (long long)nnz);
         const size_t nnzs = (size_t)std::max<long long>(nnz, 1);
-        unsigned *bcnt, *ent;
-        long long *boff, *bstart, *btot;
-        int *ctmp = nullptr;
-        float *entv = nullptr, *vtmp = nullptr;
-        PG_TRY(pg_bufT(ctx, "corr.bcnt", (size_t)nsrc * nbk, &bcnt));
-        PG_TRY(pg_bufT(ctx, "corr.boff", (size_t)nsrc * nbk, &boff));
-        PG_TRY(pg_bufT(ctx, "corr.bstart", (size_t)nbk + 1, &bstart));
-        PG_TRY(pg_bufT(ctx, "corr.btot", (size_t)nbk + 1, &btot));
-        PG_TRY(pg_bufT(ctx, "corr.ent", nnzs, &ent));
         PG_TRY(pg_bufT(ctx, "corr.row", (size_t)n + 2, &row));
         PG_TRY(pg_bufT(ctx, "corr.col", nnzs, &col));
-        const BitsPlan bp = weighted ? BitsPlan() : rows_bits_plan(n, ctx->lds_per_block);
-        const size_t lbits = bp.lds;
-        if (!lbits) PG_TRY(pg_bufT(ctx, "corr.ctmp", nnzs, &ctmp));
         val = nullptr;
-        if (weighted) {
-            PG_TRY(pg_bufT(ctx, "corr.entv", nnzs, &entv));
-            PG_TRY(pg_bufT(ctx, "corr.vtmp", nnzs, &vtmp));
-            PG_TRY(pg_bufT(ctx, "corr.val", nnzs, &val));
-        }
-        if (n > 0) {
-            const size_t shb = (size_t)nbk * 4;
-            if (!seg_counted) bucket_count<<<(unsigned)nsrc, SEG_THREADS, shb, st>>>(src, nbk, 0, nsrc, bcnt);
-            bucket_scan_local<<<(unsigned)pg_cdiv(nbk, SCAN_BK), SCAN_BK * SCAN_SG, 0, st>>>(bcnt, nsrc, nbk, boff,
-                                                                                          btot);
-            bucket_scan_global<<<1, 1024, 0, st>>>(btot, nbk, bstart);
-            const size_t shs = (size_t)nbk * (4 + 4);  // bases + cursors
-            const void *scatter_fn = weighted ? (const void *)bucket_scatter<true> : (const void *)bucket_scatter<false>;
-            if (shs > 64 * 1024)
-                PG_HIP(ctx, set_shared_limit(ctx, scatter_fn, shs));
-            if (weighted) {
-                PG_TRY(launch_edge_values(src));
-                bucket_scatter<true><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, entv,
-                                                                               (long long)nnzs);
-            } else {
-                bucket_scatter<false><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, nullptr,
-                                                                                (long long)nnzs);
-            }
-            if (lbits) {
-                PG_HIP(ctx, set_shared_limit(ctx, rows_bits_fn(bp.rank), (int)lbits));
-                launch_rows_bits(ctx, bp, st, bstart, ent, n, nbk, row, col, (long long)nnzs);
-                PG_KERNEL_CHECK(ctx);
-                return PG_OK;
-            }
-            const RowsPlan rp = rows_plan(n, ctx->lds_per_block);
-            if (rp.nbm == 0) return pg_fail(ctx, PG_ENOTSUP, "n = %d: the row bitmap does not fit LDS", n);
-            const void *rows_fn = weighted ? (const void *)bucket_rows<true> : (const void *)bucket_rows<false>;
-            PG_HIP(ctx, set_shared_limit(ctx, rows_fn, rp.lds));
-            if (weighted)
-                bucket_rows<true><<<(unsigned)nbk, ROWS_THREADS, rp.lds, st>>>(
-                    bstart, ent, entv, n, nbk, rp.nbm, rp.dbit, row, ctmp, vtmp, col, val, (long long)nnzs);
-            else
-                bucket_rows<false><<<(unsigned)nbk, ROWS_THREADS, rp.lds, st>>>(
-                    bstart, ent, nullptr, n, nbk, rp.nbm, rp.dbit, row, ctmp, nullptr, col, nullptr, (long long)nnzs);
-            PG_KERNEL_CHECK(ctx);
-        } else {
+        if (weighted) PG_TRY(pg_bufT(ctx, "corr.val", nnzs, &val));
+        if (n == 0) {
             PG_HIP(ctx, hipMemsetAsync(row, 0, 4, st));
+            return PG_OK;
         }
-        return PG_OK;
+        if (weighted) PG_TRY(launch_edge_values(src));
+        return csr_launch(ctx, "corr.", src, n, nsrc, weighted, nnz, seg_counted, row, col, val);
     }
 
     // launch, wait, and check row[n]
@@ -4505,6 +4526,34 @@ extern "C" pg_status pg_corr_select(pg_ctx *ctx, float thr, pg_corr_info *info)
     ctx->c_z64 = R.z64;
     if (info) *info = inf;
     return PG_OK;
+}
+
+// ------------------------------------------------------- CSR of a pair list
+
+bool pg_csr_pairs_ok(const pg_ctx *ctx, int n)
+{
+    // the scatter's two words per bucket and one row bitmap have to fit LDS
+    return n >= 1 && pg_cdiv(n, BROWS) * 8 <= 159 * 1024 && rows_plan(n, ctx->lds_per_block).nbm > 0;
+}
+
+pg_status pg_csr_pairs(pg_ctx *ctx, const char *pfx, const int2 *pairs, const float *w, long long m, int n,
+                       int32_t *row, int32_t *col, float *val)
+{
+    // at most as many segments as CUs hold scatter work-groups, 4,096 pairs
+    // (half a batch per thread) at least
+    const int nseg = (int)std::max<long long>(1, std::min<long long>(2LL * std::max(ctx->num_cu, 1), pg_cdiv(m, 4096)));
+    EdgeSrc src;
+    std::memset(&src, 0, sizeof src);
+    unsigned long long *cnt;
+    PG_TRY(pg_bufT(ctx, (std::string(pfx) + "segcnt").c_str(), (size_t)nseg, &cnt));
+    src.seg = pairs;
+    src.seg_cap = std::max<long long>(1, pg_cdiv(m, nseg));
+    src.seg_cnt = cnt;
+    src.nseg = nseg;
+    src.seg_w = const_cast<float *>(w);
+    src.w_cap = src.seg_cap;
+    slice_counts<<<(unsigned)pg_cdiv(nseg, 256), 256, 0, ctx->stream>>>(m, src.seg_cap, nseg, cnt);
+    return csr_launch(ctx, pfx, src, n, nseg, val != nullptr, 2 * m, false, row, col, val);
 }
 
 // ------------------------------------------- captured cohort: construction

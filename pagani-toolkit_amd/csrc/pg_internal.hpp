@@ -151,6 +151,14 @@ pg_status pg_validate_csr_flag(pg_ctx *ctx, const int32_t *drow, const int32_t *
 // with the device current.
 pg_status pg_static_scratch(pg_ctx *ctx, void **ptr);
 
+// Symmetric CSR (columns ascending) of n vertices from m distinct pairs i != j
+// in device memory, by the bucketed counting sort of the construction
+// (corr.hip); with val, w holds the pairs' weights.  Launches only; row[n] = 2 m.
+// Work buffers are named pfx + ...  pg_csr_pairs_ok: n fits the sort's LDS.
+bool pg_csr_pairs_ok(const pg_ctx *ctx, int n);
+pg_status pg_csr_pairs(pg_ctx *ctx, const char *pfx, const int2 *pairs, const float *w, long long m, int n,
+                       int32_t *row, int32_t *col, float *val);
+
 // pg_corr_emit state: dropped by any build that reuses its buffers, freed
 // with the context.
 void pg_emit_invalidate(pg_ctx *ctx);

@@ -18,11 +18,11 @@
 // edges through a keyed bijection of [0, M) (a 4-round Feistel network on the
 // next even power of two, cycle-walked into range): attempt t takes edges
 // perm(2t) and perm(2t+1), so no edge is in two attempts of one round.  The
-// round-start edges sit in an open-addressing hash (linear probing, 64-bit
-// keys) with owner 0.  Kernel rw_propose finds or inserts each attempt's two
-// new-edge keys and, when neither is an existing edge, takes both with an
-// atomicMin of its attempt id; kernel rw_commit applies the swaps whose
-// attempt owns both keys.  The winners are a function of the seed alone (no
+// round-start edges are bits of a lower-triangular bitmap (n <= BM_MAX_N) or
+// sit in an open-addressing hash (linear probing, 64-bit keys) with owner 0.
+// rw_propose / rw_propose_bits look each attempt's two new edges up and, when
+// neither exists, take both keys in a hash with an atomicMin of the attempt
+// id; rw_commit / rw_commit_bits apply the swaps whose attempt owns both keys.  The winners are a function of the seed alone (no
 // dependence on thread timing), every applied swap is valid for the graph at
 // the end of the round, and degrees, symmetry and the absence of self-loops
 // and multi-edges hold after every round.  Deviations from the sequential
@@ -135,29 +135,27 @@ __global__ __launch_bounds__(1024) void rw_scan(const int *__restrict__ in, int 
 // One wave per row: the row's upper entries into E at base[u], in column order.
 __global__ __launch_bounds__(256) void rw_extract(const int *__restrict__ row, const int *__restrict__ col,
                                                   const float *__restrict__ val, const int *__restrict__ cnt,
-                                                  const long long *__restrict__ base, int n, int *__restrict__ eu,
-                                                  int *__restrict__ ev, float *__restrict__ ew)
+                                                  const long long *__restrict__ base, int n, int2 *__restrict__ E,
+                                                  float *__restrict__ ew)
 {
     const int u = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (u >= n) return;
     const int b = row[u + 1], c = cnt[u], a = b - c;
     const long long o = base[u];
     for (int k = lane; k < c; k += 64) {
-        eu[o + k] = u;
-        ev[o + k] = col[a + k];
+        E[o + k] = make_int2(u, col[a + k]);
         if (ew) ew[o + k] = val[a + k];
     }
 }
 
 // Every upper entry (u, v) must have its mirror (v, u), with the same weight.
 __global__ void rw_check_mirror(const int *__restrict__ row, const int *__restrict__ col,
-                                const float *__restrict__ val, const int *__restrict__ eu,
-                                const int *__restrict__ ev, const float *__restrict__ ew, int m,
-                                int *__restrict__ flags)
+                                const float *__restrict__ val, const int2 *__restrict__ E,
+                                const float *__restrict__ ew, int m, int *__restrict__ flags)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= m) return;
-    const int u = eu[e], v = ev[e];
+    const int u = E[e].x, v = E[e].y;
     int lo = row[v], hi = row[v + 1];
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
@@ -178,13 +176,12 @@ __global__ void rw_clear(unsigned long long *__restrict__ tab, unsigned *__restr
 }
 
 // The current edges, owner 0.
-__global__ void rw_insert_edges(const int *__restrict__ eu, const int *__restrict__ ev, int m,
-                                unsigned long long *__restrict__ tab, unsigned *__restrict__ own,
-                                unsigned long long mask)
+__global__ void rw_insert_edges(const int2 *__restrict__ E, int m, unsigned long long *__restrict__ tab,
+                                unsigned *__restrict__ own, unsigned long long mask)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= m) return;
-    const unsigned long long s = hs_find_or_insert(tab, mask, edge_key(eu[e], ev[e]));
+    const unsigned long long s = hs_find_or_insert(tab, mask, edge_key(E[e].x, E[e].y));
     own[s] = 0u;
 }
 
@@ -194,30 +191,37 @@ struct Attempt {
     bool disjoint;
 };
 
-__device__ __forceinline__ Attempt rw_attempt(long long t, const RwRound &r, const int *__restrict__ eu,
-                                              const int *__restrict__ ev)
+__device__ __forceinline__ Attempt rw_attempt(long long t, const RwRound &r, const int2 *__restrict__ E)
 {
     Attempt a;
     a.i = (int)rw_perm((unsigned)(2 * t), r);
     a.j = (int)rw_perm((unsigned)(2 * t + 1), r);
-    a.v1 = eu[a.i];
-    a.v2 = ev[a.i];
-    a.v3 = eu[a.j];
-    a.v4 = ev[a.j];
+    const int2 x = E[a.i], y = E[a.j];
+    a.v1 = x.x;
+    a.v2 = x.y;
+    a.v3 = y.x;
+    a.v4 = y.y;
     a.disjoint = !(a.v1 == a.v3 || a.v1 == a.v4 || a.v2 == a.v3 || a.v2 == a.v4);
     a.form13 = (mix64(r.ckey ^ (unsigned long long)t) & 1ull) != 0;
     return a;
 }
 
+// The two edges after the swap (each slot keeps its orientation rules: 1-3,2-4
+// or 1-4,3-2).
+__device__ __forceinline__ void rw_swap(const Attempt &a, int2 &x, int2 &y)
+{
+    x = make_int2(a.v1, a.form13 ? a.v3 : a.v4);
+    y = a.form13 ? make_int2(a.v2, a.v4) : make_int2(a.v3, a.v2);
+}
+
 // Attempt t (id t + 1) proposes its two new edges: both slots are found or
 // inserted; unless one is an existing edge, both are claimed by atomicMin.
-__global__ void rw_propose(RwRound r, const int *__restrict__ eu, const int *__restrict__ ev,
-                           unsigned long long *__restrict__ tab, unsigned *__restrict__ own,
-                           uint2 *__restrict__ slots)
+__global__ void rw_propose(RwRound r, const int2 *__restrict__ E, unsigned long long *__restrict__ tab,
+                           unsigned *__restrict__ own, uint2 *__restrict__ slots)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= r.p) return;
-    const Attempt a = rw_attempt(t, r, eu, ev);
+    const Attempt a = rw_attempt(t, r, E);
     uint2 sl = make_uint2(NO_OWNER, NO_OWNER);
     if (a.disjoint) {
         const int x = a.form13 ? a.v3 : a.v4, y = a.form13 ? a.v4 : a.v3;
@@ -235,8 +239,7 @@ __global__ void rw_propose(RwRound r, const int *__restrict__ eu, const int *__r
 }
 
 // Apply the swaps whose attempt owns both of its keys; count them.
-__global__ __launch_bounds__(256) void rw_commit(RwRound r, int *__restrict__ eu, int *__restrict__ ev,
-                                                 const unsigned *__restrict__ own, const uint2 *__restrict__ slots,
+__global__ __launch_bounds__(256) void rw_commit(RwRound r, int2 *__restrict__ E, const unsigned *__restrict__ own, const uint2 *__restrict__ slots,
                                                  unsigned long long *__restrict__ swaps)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -245,19 +248,145 @@ __global__ __launch_bounds__(256) void rw_commit(RwRound r, int *__restrict__ eu
         const uint2 sl = slots[t];
         const unsigned id = (unsigned)(t + 1);
         if (sl.x != NO_OWNER && own[sl.x] == id && own[sl.y] == id) {
-            const Attempt a = rw_attempt(t, r, eu, ev);
-            if (a.form13) {
-                ev[a.i] = a.v3;
-                eu[a.j] = a.v2;
-            } else {
-                ev[a.i] = a.v4;
-                ev[a.j] = a.v2;
-            }
+            const Attempt a = rw_attempt(t, r, E);
+            rw_swap(a, E[a.i], E[a.j]);
             done = true;
         }
     }
     const unsigned long long b = __ballot(done);
     if ((threadIdx.x & 63) == 0 && b) atomicAdd(swaps, (unsigned long long)__popcll(b));
+}
+
+// ---- edges as bits (n <= BM_MAX_N)
+//
+// Bit lo of row hi is set when {lo, hi}, lo < hi, is an edge; rows of nw words.
+// A look-up is one 4-byte read of a table of n^2 / 16 bytes in use (210 MB at n
+// = 58,000, the size of the last-level cache) where the hash with its owners
+// takes 1.6 GB, and the keys that attempts claim have a table to themselves:
+// key and smallest attempt id in one 64-bit word.
+constexpr int BM_MAX_N = 1 << 17;  // 1.1 GB in use; keys of 34 bits
+constexpr int ID_BITS = 30;        // attempt ids: at most m / 2 <= 2^28
+
+__device__ __forceinline__ bool rw_bit(const unsigned *__restrict__ bm, int nw, int a, int b)
+{
+    const int lo = min(a, b), hi = max(a, b);
+    return (bm[(long long)hi * nw + (lo >> 5)] >> (lo & 31)) & 1u;
+}
+
+// Rows of the bitmap from the sorted CSR, one work-group per vertex, no atomics
+// on memory: the words up to the diagonal.
+__global__ __launch_bounds__(256) void rw_bits_rows(const int *__restrict__ row, const int *__restrict__ col, int nw,
+                                                    unsigned *__restrict__ bm)
+{
+    extern __shared__ uint32_t sm[];
+    const int v = blockIdx.x, used = (v >> 5) + 1;
+    for (int q = threadIdx.x; q < used; q += 256) sm[q] = 0u;
+    __syncthreads();
+    for (int e = row[v] + (int)threadIdx.x; e < row[v + 1]; e += 256) {
+        const int c = col[e];
+        if (c >= v) break;  // ascending: the rest lies above the diagonal
+        atomicOr(&sm[c >> 5], 1u << (c & 31));
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < used; q += 256) bm[(long long)v * nw + q] = sm[q];
+}
+
+// Every upper entry's mirror is the bit of a lower one; with as many lower
+// entries as upper ones the network is symmetric.
+__global__ void rw_check_bits(const int2 *__restrict__ E, int m, const unsigned *__restrict__ bm, int nw,
+                              int *__restrict__ flags)
+{
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < m && !rw_bit(bm, nw, E[e].x, E[e].y)) atomicOr(flags, 4);
+}
+
+__global__ __launch_bounds__(256) void rw_bits_clear(int nw, unsigned *__restrict__ bm)
+{
+    const int v = blockIdx.x, used = (v >> 5) + 1;
+    for (int q = threadIdx.x; q < used; q += 256) bm[(long long)v * nw + q] = 0u;
+}
+
+__global__ void rw_bits_edges(const int2 *__restrict__ E, int m, int nw, unsigned *__restrict__ bm)
+{
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= m) return;
+    const int lo = min(E[e].x, E[e].y), hi = max(E[e].x, E[e].y);
+    atomicOr(&bm[(long long)hi * nw + (lo >> 5)], 1u << (lo & 31));
+}
+
+__global__ void rw_claims_clear(unsigned long long *__restrict__ tab, unsigned long long cap)
+{
+    const unsigned long long s = 2ull * ((unsigned long long)blockIdx.x * blockDim.x + threadIdx.x);
+    if (s < cap) *(ulonglong2 *)(tab + s) = make_ulonglong2(EMPTY, EMPTY);
+}
+
+// Claim key a-b for attempt id: the slot, holding the smallest id of its key.
+__device__ __forceinline__ unsigned rw_claim(unsigned long long *tab, unsigned long long mask, int a, int b, unsigned id)
+{
+    const unsigned long long key = ((unsigned long long)(unsigned)min(a, b) << 17) | (unsigned)max(a, b);
+    const unsigned long long w = (key << ID_BITS) | id;
+    unsigned long long s = mix64(key) & mask;
+    for (;;) {
+        const unsigned long long prev = atomicCAS(&tab[s], EMPTY, w);
+        if (prev == EMPTY) return (unsigned)s;
+        if ((prev >> ID_BITS) == key) {
+            if (prev > w) atomicMin(&tab[s], w);
+            return (unsigned)s;
+        }
+        s = (s + 1) & mask;
+    }
+}
+
+struct RwRec {
+    int i, j;
+    unsigned sa, sb;
+    int2 x, y;  // the edges after the swap
+};
+
+// As rw_propose; the record spares rw_commit_bits the permutation and the
+// random reads of both edges.
+__global__ __launch_bounds__(256) void rw_propose_bits(RwRound r, const int2 *__restrict__ E, const unsigned *__restrict__ bm, int nw,
+                                unsigned long long *__restrict__ tab, RwRec *__restrict__ rec)
+{
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= r.p) return;
+    const Attempt a = rw_attempt(t, r, E);
+    RwRec c;
+    c.i = a.i;
+    c.j = a.j;
+    c.sa = c.sb = NO_OWNER;
+    rw_swap(a, c.x, c.y);
+    if (a.disjoint && !rw_bit(bm, nw, c.x.x, c.x.y) && !rw_bit(bm, nw, c.y.x, c.y.y)) {
+        const unsigned id = (unsigned)(t + 1);
+        c.sa = rw_claim(tab, r.mask, c.x.x, c.x.y, id);
+        c.sb = rw_claim(tab, r.mask, c.y.x, c.y.y, id);
+    }
+    rec[t] = c;
+}
+
+__global__ __launch_bounds__(256) void rw_commit_bits(RwRound r, int2 *__restrict__ E, const unsigned long long *__restrict__ tab,
+                               const RwRec *__restrict__ rec, unsigned long long *__restrict__ swaps)
+{
+    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    bool done = false;
+    if (t < r.p) {
+        const RwRec c = rec[t];
+        const unsigned long long id = (unsigned long long)(t + 1), idm = (1ull << ID_BITS) - 1;
+        if (c.sa != NO_OWNER && (tab[c.sa] & idm) == id && (tab[c.sb] & idm) == id) {
+            E[c.i] = c.x;
+            E[c.j] = c.y;
+            done = true;
+        }
+    }
+    const unsigned long long b = __ballot(done);
+    if ((threadIdx.x & 63) == 0 && b) atomicAdd(swaps, (unsigned long long)__popcll(b));
+}
+
+// Swaps preserve degrees: the rebuilt offsets are the input's (else bit 3).
+__global__ void rw_check_rows(const int *__restrict__ row, const int *__restrict__ nrow, int n, int *__restrict__ flags)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i <= n && row[i] != nrow[i]) atomicOr(flags, 8);
 }
 
 __global__ void rw_cursor_init(const int *__restrict__ row, int n, int *__restrict__ cur)
@@ -269,13 +398,12 @@ __global__ void rw_cursor_init(const int *__restrict__ row, int n, int *__restri
 // Both directions of every edge into their rows (unordered inside a row).
 // Swaps preserve degrees, so each row receives exactly its length; a write
 // that would leave its row is dropped and flagged (bit 3), and the call fails.
-__global__ void rw_fill(const int *__restrict__ row, const int *__restrict__ eu, const int *__restrict__ ev,
-                        const float *__restrict__ ew, int m, int *__restrict__ cur, int *__restrict__ ctmp,
+__global__ void rw_fill(const int *__restrict__ row, const int2 *__restrict__ E, const float *__restrict__ ew, int m, int *__restrict__ cur, int *__restrict__ ctmp,
                         float *__restrict__ vtmp, int *__restrict__ flags)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= m) return;
-    const int u = eu[e], v = ev[e];
+    const int u = E[e].x, v = E[e].y;
     const int pu = atomicAdd(&cur[u], 1), pv = atomicAdd(&cur[v], 1);
     const float w = ew ? ew[e] : 0.0f;
     if (pu < row[u + 1]) {
@@ -395,7 +523,8 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
     // hash slots are 32-bit with 0xffffffff reserved: capacity 4M <= 2^31
     if (m64 > (1ll << 29)) return pg_fail(ctx, PG_ENOTSUP, "%lld edges: at most 2^29 are supported", m64);
     const int m = (int)m64;
-    const bool long_rows = (fl & 2) != 0;
+    const bool by_sort = pg_csr_pairs_ok(ctx, n);  // else row by row
+    const bool long_rows = (fl & 2) != 0 && !by_sort;
     const size_t long_lds = 2 * (size_t)((n + 31) / 32) * 4;  // bitmap + prefix words
     constexpr size_t LDS_MAX = 159 * 1024;                     // 160 KB less the static scan array
     if (long_rows && long_lds > LDS_MAX)
@@ -403,13 +532,24 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
     if (long_rows)
         PG_HIP(ctx, hipFuncSetAttribute((const void *)rw_sort_long, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)long_lds));
-    int *eu, *ev;
+    int2 *E;
     float *ew = nullptr;
-    PG_TRY(pg_bufT(ctx, "rw.eu", (size_t)m, &eu));
-    PG_TRY(pg_bufT(ctx, "rw.ev", (size_t)m, &ev));
+    PG_TRY(pg_bufT(ctx, "rw.edges", (size_t)m, &E));
     if (weighted) PG_TRY(pg_bufT(ctx, "rw.ew", (size_t)m, &ew));
-    rw_extract<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, dcol, dval, cnt, base, n, eu, ev, ew);
-    rw_check_mirror<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(drow, dcol, dval, eu, ev, ew, m, flags);
+    rw_extract<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, dcol, dval, cnt, base, n, E, ew);
+    // the bitmap pays while its rows are no emptier than a hash would be
+    // (n^2 / 16 bytes in use against 48 per edge, or a size that any cache holds)
+    const int nw = (n + 31) / 32;
+    const bool bits = n <= BM_MAX_N && (long long)n * n / 16 <= std::max<long long>(48ll * m, 64ll << 20);
+    unsigned *bm = nullptr;
+    if (bits) {
+        PG_TRY(pg_bufT(ctx, "rw.bits", (size_t)n * nw, &bm));
+        rw_bits_rows<<<(unsigned)n, 256, (size_t)nw * 4, st>>>(drow, dcol, nw, bm);
+    }
+    if (bits && !ew)
+        rw_check_bits<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(E, m, bm, nw, flags);
+    else
+        rw_check_mirror<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(drow, dcol, dval, E, ew, m, flags);
     PG_KERNEL_CHECK(ctx);
     PG_HIP(ctx, hipMemcpyAsync(&fl, flags, 4, hipMemcpyDeviceToHost, st));
     PG_HIP(ctx, hipStreamSynchronize(st));
@@ -425,19 +565,26 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
     PG_TRY(pg_bufT(ctx, "rw.swaps", 1, &dswaps));
     PG_HIP(ctx, hipMemsetAsync(dswaps, 0, 8, st));
     if (per_round > 0 && total > 0) {
+        // hash: edges and proposals, at most half full; claims alone: at most m
+        // proposals
         unsigned long long cap = 1024;
-        while (cap < 4ull * (unsigned long long)m) cap <<= 1;
+        while (cap < (bits ? 2ull : 4ull) * (unsigned long long)m) cap <<= 1;
         unsigned long long *tab;
-        unsigned *own;
-        uint2 *slots;
+        unsigned *own = nullptr;
+        uint2 *slots = nullptr;
+        RwRec *rec = nullptr;
         PG_TRY(pg_bufT(ctx, "rw.tab", (size_t)cap, &tab));
-        PG_TRY(pg_bufT(ctx, "rw.own", (size_t)cap, &own));
-        PG_TRY(pg_bufT(ctx, "rw.slots", (size_t)per_round, &slots));
-        int bits = 0;
-        while ((1ll << bits) < m) bits++;
-        bits += bits & 1;
+        if (bits) {
+            PG_TRY(pg_bufT(ctx, "rw.rec", (size_t)per_round, &rec));
+        } else {
+            PG_TRY(pg_bufT(ctx, "rw.own", (size_t)cap, &own));
+            PG_TRY(pg_bufT(ctx, "rw.slots", (size_t)per_round, &slots));
+        }
+        int pbits = 0;
+        while ((1ll << pbits) < m) pbits++;
+        pbits += pbits & 1;
         RwRound r;
-        r.half_bits = bits / 2;
+        r.half_bits = pbits / 2;
         r.half_mask = (1u << r.half_bits) - 1u;
         r.m = m;
         r.mask = cap - 1;
@@ -447,10 +594,20 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
             key = mix64(key + 0x9e3779b97f4a7c15ull);
             r.pkey = key;
             r.ckey = mix64(key ^ 0xd1b54a32d192ed03ull);
+            if (bits) {
+                if (done > 0) {  // the first round's bits are the input's
+                    rw_bits_clear<<<(unsigned)n, 256, 0, st>>>(nw, bm);
+                    rw_bits_edges<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(E, m, nw, bm);
+                }
+                rw_claims_clear<<<(unsigned)pg_cdiv((long long)cap, 512), 256, 0, st>>>(tab, cap);
+                rw_propose_bits<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, bm, nw, tab, rec);
+                rw_commit_bits<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, tab, rec, dswaps);
+                continue;
+            }
             rw_clear<<<(unsigned)pg_cdiv((long long)cap, 256), 256, 0, st>>>(tab, own, cap);
-            rw_insert_edges<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(eu, ev, m, tab, own, r.mask);
-            rw_propose<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, eu, ev, tab, own, slots);
-            rw_commit<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, eu, ev, own, slots, dswaps);
+            rw_insert_edges<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(E, m, tab, own, r.mask);
+            rw_propose<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, tab, own, slots);
+            rw_commit<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, own, slots, dswaps);
         }
         PG_KERNEL_CHECK(ctx);
     }
@@ -460,13 +617,20 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
     float *dvout = nullptr, *vtmp = nullptr;
     PG_TRY(pg_out(ctx, out_col, (size_t)nnz, "out.rwcol", &dout));
     if (weighted) PG_TRY(pg_out(ctx, out_val, (size_t)nnz, "out.rwval", &dvout));
-    PG_TRY(pg_bufT(ctx, "rw.cur", (size_t)n, &cur));
-    PG_TRY(pg_bufT(ctx, "rw.ctmp", (size_t)nnz, &ctmp));
-    if (weighted) PG_TRY(pg_bufT(ctx, "rw.vtmp", (size_t)nnz, &vtmp));
-    rw_cursor_init<<<(unsigned)pg_cdiv(n, 256), 256, 0, st>>>(drow, n, cur);
-    rw_fill<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(drow, eu, ev, ew, m, cur, ctmp, vtmp, flags);
-    rw_sort_short<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, n, ctmp, vtmp, dout, dvout);
-    if (long_rows) rw_sort_long<<<(unsigned)n, 256, long_lds, st>>>(drow, n, ctmp, vtmp, dout, dvout);
+    if (by_sort) {
+        int *nrow;
+        PG_TRY(pg_bufT(ctx, "rw.row", (size_t)n + 1, &nrow));
+        PG_TRY(pg_csr_pairs(ctx, "rw.", E, ew, m, n, nrow, dout, dvout));
+        rw_check_rows<<<(unsigned)pg_cdiv(n + 1, 256), 256, 0, st>>>(drow, nrow, n, flags);
+    } else {
+        PG_TRY(pg_bufT(ctx, "rw.cur", (size_t)n, &cur));
+        PG_TRY(pg_bufT(ctx, "rw.ctmp", (size_t)nnz, &ctmp));
+        if (weighted) PG_TRY(pg_bufT(ctx, "rw.vtmp", (size_t)nnz, &vtmp));
+        rw_cursor_init<<<(unsigned)pg_cdiv(n, 256), 256, 0, st>>>(drow, n, cur);
+        rw_fill<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(drow, E, ew, m, cur, ctmp, vtmp, flags);
+        rw_sort_short<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, n, ctmp, vtmp, dout, dvout);
+        if (long_rows) rw_sort_long<<<(unsigned)n, 256, long_lds, st>>>(drow, n, ctmp, vtmp, dout, dvout);
+    }
     PG_KERNEL_CHECK(ctx);
     PG_TRY(pg_out_finish(ctx, out_col, dout, (size_t)nnz));
     if (weighted) PG_TRY(pg_out_finish(ctx, out_val, dvout, (size_t)nnz));

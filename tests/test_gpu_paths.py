@@ -155,3 +155,27 @@ def test_efficiency_components_and_tails(ctx, n, m, tail):
     oe, olp, oiso, ounc = O.bfs_efficiency(row, col)
     np.testing.assert_array_equal(e.view(np.uint32), oe.view(np.uint32))
     assert abs(lp - olp) <= 1e-12 * abs(olp) and (iso, unc) == (oiso, ounc)
+
+
+# bitmap of the edges (n^2 / 16 bytes up to 64 MB or 48 per edge), the hash
+# beyond; a hub row longer than the registers sort
+@pytest.mark.parametrize("n,m,hub", [(31, 200, 0), (32, 300, 0), (33, 200, 20), (2000, 30000, 1500),
+                                     (32000, 100000, 1500), (40000, 100000, 1500)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_rewire_paths(ctx, n, m, hub, weighted):
+    from helpers import check_rewired
+    row, col, val = _graph(n, m, 7 * n + m, hub)
+    v = val if weighted else None
+    say(f"rewire paths n={n} nnz={col.size} weighted={weighted}")
+    oc, ov, sw = ctx.rewire(row, col, v, seed=9)
+    check_rewired(row, col, v, oc, ov)
+    oc2, ov2, sw2 = ctx.rewire(row, col, v, seed=9)
+    assert sw == sw2 and np.array_equal(oc, oc2) and (v is None or np.array_equal(ov, ov2))
+    # an entry without its mirror is refused on either path
+    bad = col.copy()
+    bad[row[1] - 1] = bad[row[1] - 1] + 1 if bad[row[1] - 1] + 1 < n else 1
+    if not np.array_equal(bad, col):
+        import pagani_amd
+        with pytest.raises(pagani_amd.PgError) as ex:
+            ctx.rewire(row, bad, v, seed=9)
+        assert ex.value.status == 4
