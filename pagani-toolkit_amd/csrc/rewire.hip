@@ -22,7 +22,7 @@
 // sit in an open-addressing hash (linear probing, 64-bit keys) with owner 0.
 // rw_propose / rw_propose_bits look each attempt's two new edges up and, when
 // neither exists, take both keys in a hash with an atomicMin of the attempt
-// id; rw_commit / rw_commit_bits apply the swaps whose attempt owns both keys.  The winners are a function of the seed alone (no
+// id; rw_commit / rw_restore keep the swaps whose attempt owns both keys.  The winners are a function of the seed alone (no
 // dependence on thread timing), every applied swap is valid for the graph at
 // the end of the round, and degrees, symmetry and the absence of self-loops
 // and multi-edges hold after every round.  Deviations from the sequential
@@ -63,6 +63,7 @@ __device__ __forceinline__ unsigned long long edge_key(int a, int b)
 
 struct RwRound {
     unsigned long long pkey;  // permutation key
+    unsigned long long prev;  // the round before's (bitmap rounds)
     unsigned long long ckey;  // coin key
     unsigned half_mask;       // Feistel half: h bits
     int half_bits;
@@ -82,6 +83,23 @@ __device__ __forceinline__ unsigned rw_perm(unsigned x, const RwRound &r)
             const unsigned t = L ^ f;
             L = R;
             R = t;
+        }
+        x = (L << r.half_bits) | R;
+    } while (x >= (unsigned)r.m);
+    return x;
+}
+
+// The inverse of rw_perm.
+__device__ __forceinline__ unsigned rw_perm_inv(unsigned x, const RwRound &r, unsigned long long key)
+{
+    do {
+        unsigned L = x >> r.half_bits, R = x & r.half_mask;
+#pragma unroll
+        for (int q = 3; q >= 0; q--) {
+            const unsigned f = (unsigned)mix64(key ^ ((unsigned long long)q << 56) ^ L) & r.half_mask;
+            const unsigned t = R ^ f;
+            R = L;
+            L = t;
         }
         x = (L << r.half_bits) | R;
     } while (x >= (unsigned)r.m);
@@ -191,11 +209,18 @@ struct Attempt {
     bool disjoint;
 };
 
+// MOVED: E is the list the round before left in its attempts' order, edge slot
+// x at place rw_perm_inv(x).
+template <bool MOVED = false>
 __device__ __forceinline__ Attempt rw_attempt(long long t, const RwRound &r, const int2 *__restrict__ E)
 {
     Attempt a;
     a.i = (int)rw_perm((unsigned)(2 * t), r);
     a.j = (int)rw_perm((unsigned)(2 * t + 1), r);
+    if (MOVED) {
+        a.i = (int)rw_perm_inv((unsigned)a.i, r, r.prev);
+        a.j = (int)rw_perm_inv((unsigned)a.j, r, r.prev);
+    }
     const int2 x = E[a.i], y = E[a.j];
     a.v1 = x.x;
     a.v2 = x.y;
@@ -314,72 +339,120 @@ __global__ void rw_bits_edges(const int2 *__restrict__ E, int m, int nw, unsigne
     atomicOr(&bm[(long long)hi * nw + (lo >> 5)], 1u << (lo & 31));
 }
 
-__global__ void rw_claims_clear(unsigned long long *__restrict__ tab, unsigned long long cap)
+__global__ void rw_claims_clear(unsigned long long *__restrict__ tab, unsigned long long cap,
+                                unsigned *__restrict__ lost, unsigned long long nlost)
 {
     const unsigned long long s = 2ull * ((unsigned long long)blockIdx.x * blockDim.x + threadIdx.x);
     if (s < cap) *(ulonglong2 *)(tab + s) = make_ulonglong2(EMPTY, EMPTY);
+    if (s < nlost) lost[s] = 0u;
+    if (s + 1 < nlost) lost[s + 1] = 0u;
 }
 
-// Claim key a-b for attempt id: the slot, holding the smallest id of its key.
-__device__ __forceinline__ unsigned rw_claim(unsigned long long *tab, unsigned long long mask, int a, int b, unsigned id)
+// Claim key a-b for attempt id.  The key's slot keeps the smallest id; every
+// other claimer is marked lost, by itself when it finds a smaller id or by the
+// one that displaces it.
+__device__ __forceinline__ void rw_claim(unsigned long long *tab, unsigned long long mask, int a, int b, unsigned id,
+                                         uint8_t *lost)
 {
     const unsigned long long key = ((unsigned long long)(unsigned)min(a, b) << 17) | (unsigned)max(a, b);
     const unsigned long long w = (key << ID_BITS) | id;
     unsigned long long s = mix64(key) & mask;
     for (;;) {
-        const unsigned long long prev = atomicCAS(&tab[s], EMPTY, w);
-        if (prev == EMPTY) return (unsigned)s;
+        unsigned long long prev = atomicCAS(&tab[s], EMPTY, w);
+        if (prev == EMPTY) return;
         if ((prev >> ID_BITS) == key) {
-            if (prev > w) atomicMin(&tab[s], w);
-            return (unsigned)s;
+            prev = atomicMin(&tab[s], w);
+            lost[(prev > w ? (unsigned)(prev & ((1ull << ID_BITS) - 1)) : id) - 1] = 1;
+            return;
         }
         s = (s + 1) & mask;
     }
 }
 
-struct RwRec {
-    int i, j;
-    unsigned sa, sb;
-    int2 x, y;  // the edges after the swap
-};
-
-// As rw_propose; the record spares rw_commit_bits the permutation and the
-// random reads of both edges.
-__global__ __launch_bounds__(256) void rw_propose_bits(RwRound r, const int2 *__restrict__ E, const unsigned *__restrict__ bm, int nw,
-                                unsigned long long *__restrict__ tab, RwRec *__restrict__ rec)
+// Attempts 0 .. p - 1 as rw_propose; thread t also carries the edges at places
+// 2t and 2t + 1 of the round's order into F: the swapped ones if both keys were
+// claimed (rw_restore takes back the attempts that lost one), else unchanged.
+// So the list is written in order, the next round finds slot x at
+// rw_perm_inv(x), and a round's random traffic is the reads of two edges and
+// two bits and the two claims.  Per work-group the claiming attempts are added
+// to part (one address for all waves cost more than the rest of the commit).
+template <bool MOVED>
+__global__ __launch_bounds__(256) void rw_propose_bits(RwRound r, const int2 *__restrict__ E,
+                                                       const unsigned *__restrict__ bm, int nw,
+                                                       unsigned long long *__restrict__ tab,
+                                                       uint8_t *__restrict__ lost, int2 *__restrict__ F,
+                                                       int *__restrict__ part)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= r.p) return;
-    const Attempt a = rw_attempt(t, r, E);
-    RwRec c;
-    c.i = a.i;
-    c.j = a.j;
-    c.sa = c.sb = NO_OWNER;
-    rw_swap(a, c.x, c.y);
-    if (a.disjoint && !rw_bit(bm, nw, c.x.x, c.x.y) && !rw_bit(bm, nw, c.y.x, c.y.y)) {
-        const unsigned id = (unsigned)(t + 1);
-        c.sa = rw_claim(tab, r.mask, c.x.x, c.x.y, id);
-        c.sb = rw_claim(tab, r.mask, c.y.x, c.y.y, id);
+    bool claimed = false;
+    if (2 * t + 1 < r.m) {
+        const Attempt a = rw_attempt<MOVED>(t, r, E);
+        int2 x = make_int2(a.v1, a.v2), y = make_int2(a.v3, a.v4);
+        if (t < r.p && a.disjoint) {
+            int2 sx, sy;
+            rw_swap(a, sx, sy);
+            if (!rw_bit(bm, nw, sx.x, sx.y) && !rw_bit(bm, nw, sy.x, sy.y)) {
+                const unsigned id = (unsigned)(t + 1);
+                rw_claim(tab, r.mask, sx.x, sx.y, id, lost);
+                rw_claim(tab, r.mask, sy.x, sy.y, id, lost);
+                x = sx;
+                y = sy;
+                claimed = true;
+            }
+        }
+        *(int4 *)(F + 2 * t) = make_int4(x.x, x.y, y.x, y.y);
+    } else if (2 * t < r.m) {
+        unsigned p = rw_perm((unsigned)(2 * t), r);
+        if (MOVED) p = rw_perm_inv(p, r, r.prev);
+        F[2 * t] = E[p];
     }
-    rec[t] = c;
+    const int k = __syncthreads_count(claimed);
+    if (threadIdx.x == 0) part[blockIdx.x] += k;
 }
 
-__global__ __launch_bounds__(256) void rw_commit_bits(RwRound r, int2 *__restrict__ E, const unsigned long long *__restrict__ tab,
-                               const RwRec *__restrict__ rec, unsigned long long *__restrict__ swaps)
+// The attempts that lost a key take their edges back.
+template <bool MOVED>
+__global__ __launch_bounds__(256) void rw_restore(RwRound r, const int2 *__restrict__ E,
+                                                  const uint8_t *__restrict__ lost, int2 *__restrict__ F,
+                                                  int *__restrict__ part)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    bool done = false;
-    if (t < r.p) {
-        const RwRec c = rec[t];
-        const unsigned long long id = (unsigned long long)(t + 1), idm = (1ull << ID_BITS) - 1;
-        if (c.sa != NO_OWNER && (tab[c.sa] & idm) == id && (tab[c.sb] & idm) == id) {
-            E[c.i] = c.x;
-            E[c.j] = c.y;
-            done = true;
-        }
+    const bool back = t < r.p && lost[t] != 0;
+    if (back) {
+        const Attempt a = rw_attempt<MOVED>(t, r, E);
+        *(int4 *)(F + 2 * t) = make_int4(a.v1, a.v2, a.v3, a.v4);
     }
-    const unsigned long long b = __ballot(done);
-    if ((threadIdx.x & 63) == 0 && b) atomicAdd(swaps, (unsigned long long)__popcll(b));
+    const int k = __syncthreads_count(back);
+    if (threadIdx.x == 0 && k) part[blockIdx.x] -= k;
+}
+
+// swaps = the sum of the work-groups' counts (one work-group)
+__global__ __launch_bounds__(1024) void rw_count(const int *__restrict__ part, int np, unsigned long long *__restrict__ swaps)
+{
+    __shared__ unsigned long long red[16];
+    unsigned long long s = 0;
+    for (int q = threadIdx.x; q < np; q += 1024) s += (unsigned long long)part[q];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        s = 0;
+        for (int q = 0; q < 16; q++) s += red[q];
+        *swaps = s;
+    }
+}
+
+// Weights of the list in the last round's order.
+__global__ void rw_weights(RwRound r, const float *__restrict__ ew, float *__restrict__ fw)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < r.m) fw[p] = ew[rw_perm((unsigned)p, r)];
+}
+
+__global__ void rw_zero(int *__restrict__ p, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
 }
 
 // Swaps preserve degrees: the rebuilt offsets are the input's (else bit 3).
@@ -532,9 +605,9 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
     if (long_rows)
         PG_HIP(ctx, hipFuncSetAttribute((const void *)rw_sort_long, hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)long_lds));
-    int2 *E;
+    int2 *E, *F = nullptr;
     float *ew = nullptr;
-    PG_TRY(pg_bufT(ctx, "rw.edges", (size_t)m, &E));
+    PG_TRY(pg_bufT(ctx, "rw.edges", (size_t)m + 1, &E));
     if (weighted) PG_TRY(pg_bufT(ctx, "rw.ew", (size_t)m, &ew));
     rw_extract<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, dcol, dval, cnt, base, n, E, ew);
     // the bitmap pays while its rows are no emptier than a hash would be
@@ -572,10 +645,16 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
         unsigned long long *tab;
         unsigned *own = nullptr;
         uint2 *slots = nullptr;
-        RwRec *rec = nullptr;
+        unsigned *lost = nullptr;  // a byte per attempt
+        const long long half = (m + 1) / 2, nlost = (per_round + 3) / 4;
+        const int np = (int)pg_cdiv(half, 256);
+        int *part = nullptr;
         PG_TRY(pg_bufT(ctx, "rw.tab", (size_t)cap, &tab));
         if (bits) {
-            PG_TRY(pg_bufT(ctx, "rw.rec", (size_t)per_round, &rec));
+            PG_TRY(pg_bufT(ctx, "rw.lost", (size_t)nlost, &lost));
+            PG_TRY(pg_bufT(ctx, "rw.part", (size_t)np, &part));
+            PG_TRY(pg_bufT(ctx, "rw.edges2", (size_t)m + 1, &F));
+            rw_zero<<<(unsigned)pg_cdiv(np, 256), 256, 0, st>>>(part, np);
         } else {
             PG_TRY(pg_bufT(ctx, "rw.own", (size_t)cap, &own));
             PG_TRY(pg_bufT(ctx, "rw.slots", (size_t)per_round, &slots));
@@ -583,7 +662,7 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
         int pbits = 0;
         while ((1ll << pbits) < m) pbits++;
         pbits += pbits & 1;
-        RwRound r;
+        RwRound r{};
         r.half_bits = pbits / 2;
         r.half_mask = (1u << r.half_bits) - 1u;
         r.m = m;
@@ -599,15 +678,34 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
                     rw_bits_clear<<<(unsigned)n, 256, 0, st>>>(nw, bm);
                     rw_bits_edges<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(E, m, nw, bm);
                 }
-                rw_claims_clear<<<(unsigned)pg_cdiv((long long)cap, 512), 256, 0, st>>>(tab, cap);
-                rw_propose_bits<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, bm, nw, tab, rec);
-                rw_commit_bits<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, tab, rec, dswaps);
+                uint8_t *lb = (uint8_t *)lost;
+                rw_claims_clear<<<(unsigned)pg_cdiv(std::max<long long>((long long)cap, nlost), 512), 256, 0, st>>>(
+                    tab, cap, lost, (unsigned long long)nlost);
+                const unsigned gp = (unsigned)np, gr = (unsigned)pg_cdiv(r.p, 256);
+                if (done > 0) {
+                    rw_propose_bits<true><<<gp, 256, 0, st>>>(r, E, bm, nw, tab, lb, F, part);
+                    rw_restore<true><<<gr, 256, 0, st>>>(r, E, lb, F, part);
+                } else {
+                    rw_propose_bits<false><<<gp, 256, 0, st>>>(r, E, bm, nw, tab, lb, F, part);
+                    rw_restore<false><<<gr, 256, 0, st>>>(r, E, lb, F, part);
+                }
+                std::swap(E, F);
+                r.prev = r.pkey;
                 continue;
             }
             rw_clear<<<(unsigned)pg_cdiv((long long)cap, 256), 256, 0, st>>>(tab, own, cap);
             rw_insert_edges<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(E, m, tab, own, r.mask);
             rw_propose<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, tab, own, slots);
             rw_commit<<<(unsigned)pg_cdiv(r.p, 256), 256, 0, st>>>(r, E, own, slots, dswaps);
+        }
+        if (bits) {
+            rw_count<<<1, 1024, 0, st>>>(part, np, dswaps);
+            if (ew) {
+                float *fw;
+                PG_TRY(pg_bufT(ctx, "rw.ew2", (size_t)m, &fw));
+                rw_weights<<<(unsigned)pg_cdiv(m, 256), 256, 0, st>>>(r, ew, fw);
+                ew = fw;
+            }
         }
         PG_KERNEL_CHECK(ctx);
     }
