@@ -281,13 +281,33 @@ __global__ __launch_bounds__(256) void zscore_fused(const float *__restrict__ x,
     }
     __syncthreads();
     if (tid < ZV) {
+        // in time order; eight LDS reads ahead of the chain of adds (one at a
+        // time, the 2 t reads' latency was the kernel: 17 us at n = 1,024)
         double s1 = 0.0;
-        for (int l = 0; l < t; l++) s1 += (double)zt[l * LD + tid];
+        int l = 0;
+        for (; l + 8 <= t; l += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = zt[(l + u) * LD + tid];
+#pragma unroll
+            for (int u = 0; u < 8; u++) s1 += (double)v[u];
+        }
+        for (; l < t; l++) s1 += (double)zt[l * LD + tid];
         s1 /= t;
         double s2 = 0.0;
-        for (int l = 0; l < t; l++) {
-            double d = (double)zt[l * LD + tid] - s1;
-            double p = d * d;
+        for (l = 0; l + 8 <= t; l += 8) {
+            double p[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const double d = (double)zt[(l + u) * LD + tid] - s1;
+                p[u] = d * d;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; u++) s2 += p[u];
+        }
+        for (; l < t; l++) {
+            const double d = (double)zt[l * LD + tid] - s1;
+            const double p = d * d;
             s2 += p;
         }
         smu[tid] = s1;
@@ -3415,10 +3435,11 @@ float thr_effective(float thr, bool weighted) { return weighted ? (float)((doubl
 
 // One construction's geometry, device buffers and launch helpers, shared by
 // pg_corr_build and the pg_corr_emit / pg_corr_select pair.
-// What the host checks after the single sparsity pass, gathered on the
-// device so that one small copy into pinned memory brings it back.
+// What the host checks after a pass, gathered by one work-group straight into
+// the context's pinned memory: no copy, one wait.
 struct SpReport {
     unsigned long long seg_max;      // the fullest segment's count
+    unsigned long long seg_sum;      // all segments' counts
     unsigned long long counters[16]; // the pass's counters
     SelCtl ctl;
     double tstar;
@@ -3432,20 +3453,29 @@ __global__ __launch_bounds__(256) void sp_report(const unsigned long long *__res
                                                  const SelCtl *__restrict__ ctl, const double *__restrict__ tstar,
                                                  const int *__restrict__ rown, SpReport *__restrict__ out)
 {
-    __shared__ unsigned long long part[256];
-    unsigned long long m = 0;
-    for (int g = threadIdx.x; g < nseg; g += 256) m = seg_cnt[g] > m ? seg_cnt[g] : m;
+    __shared__ unsigned long long part[256], sums[256];
+    unsigned long long m = 0, s = 0;
+    for (int g = threadIdx.x; g < nseg; g += 256) {
+        const unsigned long long c = seg_cnt[g];
+        m = c > m ? c : m;
+        s += c;
+    }
     part[threadIdx.x] = m;
+    sums[threadIdx.x] = s;
     __syncthreads();
     for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o && part[threadIdx.x + o] > part[threadIdx.x]) part[threadIdx.x] = part[threadIdx.x + o];
+        if ((int)threadIdx.x < o) {
+            if (part[threadIdx.x + o] > part[threadIdx.x]) part[threadIdx.x] = part[threadIdx.x + o];
+            sums[threadIdx.x] += sums[threadIdx.x + o];
+        }
         __syncthreads();
     }
     if (threadIdx.x < 16) out->counters[threadIdx.x] = counters[threadIdx.x];
     if (threadIdx.x == 0) {
         out->seg_max = part[0];
-        out->ctl = *ctl;
-        out->tstar = *tstar;
+        out->seg_sum = sums[0];
+        if (ctl) out->ctl = *ctl;
+        if (tstar) out->tstar = *tstar;
         out->rn = rown ? *rown : -1;
     }
 }
@@ -3547,6 +3577,7 @@ struct CorrRun {
     bool dedic = false;
     long long gram_passes = 0;
     std::vector<unsigned long long> hseg;
+    long long seg_sum = 0;  // entries of all segments (emit_pass)
     unsigned long long hcnt[16] = {};
 
     // z-score and MFMA panels of the series (events ev[0], ev[1] around it),
@@ -3719,17 +3750,20 @@ struct CorrRun {
         return PG_OK;
     }
 
-    // The same with a host check of the segment and band counts (hseg, hcnt),
+    // The same with a host check of the segment and band counts (seg_sum, hcnt),
     // re-run with larger buffers on overflow.
     pg_status emit_pass(long long seg_cap0, long long band_cap0, bool store_r)
     {
         long long sc = seg_cap0, bcap = band_cap0;
         for (int attempt = 0; attempt < 3; attempt++) {
             PG_TRY(emit_launch(sc, bcap, store_r));
-            PG_HIP(ctx, hipMemcpyAsync(hseg.data(), seg_cnt, nwg * 8, hipMemcpyDeviceToHost, st));
-            PG_HIP(ctx, hipMemcpyAsync(hcnt, counters, sizeof hcnt, hipMemcpyDeviceToHost, st));
+            SpReport *rep = (SpReport *)ctx->h_report;
+            sp_report<<<1, 256, 0, st>>>(seg_cnt, (int)nwg, counters, nullptr, nullptr, nullptr, rep);
+            PG_KERNEL_CHECK(ctx);
             PG_HIP(ctx, hipStreamSynchronize(st));
-            const long long mx = max_segment();
+            const long long mx = (long long)rep->seg_max;
+            seg_sum = (long long)rep->seg_sum;
+            std::memcpy(hcnt, rep->counters, sizeof hcnt);
             if (mx <= seg_cap && (long long)hcnt[0] <= band_cap) {
                 seg_used = (mx + 31) / 32 * 32;
                 return PG_OK;
@@ -3829,9 +3863,9 @@ struct CorrRun {
         PG_HIP(ctx, stage_event(ctx, 4, st));
         PG_TRY(launch_csr(src, nnz));
         PG_HIP(ctx, stage_event(ctx, 5, st));
-        PG_HIP(ctx, hipStreamSynchronize(st));
         int rn = 0;
-        PG_HIP(ctx, hipMemcpy(&rn, row + n, 4, hipMemcpyDeviceToHost));
+        PG_HIP(ctx, hipMemcpyAsync(&rn, row + n, 4, hipMemcpyDeviceToHost, st));
+        PG_HIP(ctx, hipStreamSynchronize(st));
         if ((long long)rn != nnz)
             return pg_fail(ctx, PG_EFORMAT, "CSR build mismatch: row[n]=%d nnz=%lld", rn, (long long)nnz);
         return PG_OK;
@@ -4049,8 +4083,7 @@ extern "C" pg_status pg_corr_build(pg_ctx *ctx, const float *bold, int32_t n, in
         const long long seg0 = pg_cdiv(std::max<long long>((long long)(m1 * 0.03), 1 << 20), nwg) + 4096;
         PG_TRY(R.emit_pass(seg0, 1 << 22, false));
         PG_HIP(ctx, stage_event(ctx, 3, st));
-        long long definite = 0;
-        for (auto c : R.hseg) definite += (long long)c;
+        const long long definite = R.seg_sum;
         const long long nband = (long long)hcnt[0];
         inf.band_pairs = nband;
         double *band64;
@@ -4063,13 +4096,29 @@ extern "C" pg_status pg_corr_build(pg_ctx *ctx, const float *bold, int32_t n, in
                 R.bandl, R.band_r, band64, counters + 0, R.band_cap, (double)thr_eff, extra, extra_cnt, flips);
         }
         PG_KERNEL_CHECK(ctx);
-        PG_HIP(ctx, hipMemcpyAsync(hcnt, counters, sizeof R.hcnt, hipMemcpyDeviceToHost, st));
+        // the CSR is built for every rechecked pair's room and its size read
+        // back with the counters; an overflowing bound waits for the counters
+        long long room = 2 * (definite + nband);
+        SpReport *rep = (SpReport *)ctx->h_report;
+        if (room > INT32_MAX) {
+            sp_report<<<1, 256, 0, st>>>(R.seg_cnt, (int)nwg, counters, nullptr, nullptr, nullptr, rep);
+            PG_KERNEL_CHECK(ctx);
+            PG_HIP(ctx, hipStreamSynchronize(st));
+            room = 2 * (definite + (long long)rep->counters[1]);
+        }
+        PG_HIP(ctx, stage_event(ctx, 4, st));
+        PG_TRY(R.launch_csr(R.edges(extra, extra_cnt, std::max<long long>(nband, 1)), room));
+        PG_HIP(ctx, stage_event(ctx, 5, st));
+        sp_report<<<1, 256, 0, st>>>(R.seg_cnt, (int)nwg, counters, nullptr, nullptr, R.row + n, rep);
+        PG_KERNEL_CHECK(ctx);
         PG_HIP(ctx, hipStreamSynchronize(st));
+        std::memcpy(hcnt, rep->counters, sizeof R.hcnt);
         inf.band_flips = (long long)hcnt[2];
         inf.band_max_err = host_err(hcnt[5]);
         inf.nnz = 2 * (definite + (long long)hcnt[1]);
         inf.s_thresh = (float)(m1 > 0 ? 100.0 * (double)inf.nnz / (double)m1 / 2.0 : 0.0);
-        PG_TRY(R.finish_csr(R.edges(extra, extra_cnt, std::max<long long>(nband, 1)), inf.nnz));
+        if ((long long)rep->rn != inf.nnz)
+            return pg_fail(ctx, PG_EFORMAT, "CSR build mismatch: row[n]=%d nnz=%lld", rep->rn, (long long)inf.nnz);
     } else if (kwant == 0 || n < 2) {
         // ---------------------------------------------------- nothing asked
         PG_HIP(ctx, stage_event(ctx, 2, st));
@@ -4132,13 +4181,10 @@ extern "C" pg_status pg_corr_build(pg_ctx *ctx, const float *bold, int32_t n, in
             PG_HIP(ctx, stage_event(ctx, 4, st));
             PG_TRY(R.launch_csr(es, 2 * kwant, true));
             PG_HIP(ctx, stage_event(ctx, 5, st));
-            // every check's inputs gathered on the device, one small copy back
-            SpReport *rep_d;
-            PG_TRY(pg_bufT(ctx, "corr.report", 1, &rep_d));
+            // every check's inputs
             sp_report<<<1, 256, 0, st>>>(R.seg_cnt, (int)nwg, counters, ctl, tstar_d, n > 0 ? R.row + n : nullptr,
-                                         rep_d);
+                                         (SpReport *)ctx->h_report);
             PG_KERNEL_CHECK(ctx);
-            PG_HIP(ctx, hipMemcpyAsync(ctx->h_report, rep_d, sizeof(SpReport), hipMemcpyDeviceToHost, st));
             PG_HIP(ctx, hipStreamSynchronize(st));
             const SpReport &rep = *(const SpReport *)ctx->h_report;
             std::memcpy(hcnt, rep.counters, sizeof R.hcnt);
@@ -4877,16 +4923,59 @@ pg_status pg_zscore64(pg_ctx *ctx, const float *dbold, int layout, int n, int t,
     return PG_OK;
 }
 
+namespace {
+// m words of a to b, four per thread and step when both are 16-byte aligned
+// (a caller's array may start at any word).
+__device__ __forceinline__ void copy_words(const int *__restrict__ a, long long m, int *__restrict__ b)
+{
+    const long long t0 = (long long)blockIdx.x * 256 + threadIdx.x, step = (long long)gridDim.x * 256;
+    long long done = 0;
+    if ((((uintptr_t)a | (uintptr_t)b) & 15) == 0) {
+        const int4 *a4 = (const int4 *)a;
+        int4 *b4 = (int4 *)b;
+        long long k = t0;
+        for (; k + 3 * step < m / 4; k += 4 * step) {
+            int4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = a4[k + u * step];
+#pragma unroll
+            for (int u = 0; u < 4; u++) b4[k + u * step] = v[u];
+        }
+        for (; k < m / 4; k += step) b4[k] = a4[k];
+        done = m / 4 * 4;
+    }
+    for (long long k = done + t0; k < m; k += step) b[k] = a[k];
+}
+__global__ __launch_bounds__(256) void csr_copy(const int *__restrict__ row, long long nrow,
+                                                const int *__restrict__ col, const int *__restrict__ val,
+                                                long long nnz, int *__restrict__ orow, int *__restrict__ ocol,
+                                                int *__restrict__ oval)
+{
+    copy_words(row, nrow, orow);
+    copy_words(col, nnz, ocol);
+    if (val) copy_words(val, nnz, oval);
+}
+}  // namespace
+
 extern "C" pg_status pg_corr_csr(pg_ctx *ctx, int32_t *row, int32_t *col, float *val)
 {
     if (!ctx) return PG_EINVAL;
     if (ctx->cnnz < 0) return pg_fail(ctx, PG_ESTATE, "no CSR built yet");
+    const long long nrow = (long long)ctx->cn + 1, nnz = ctx->cnnz;
+    const bool want_val = val && ctx->cweighted;
+    if (row && col && (!want_val || pg_is_device_ptr(val)) && pg_is_device_ptr(row) && pg_is_device_ptr(col)) {
+        // to device memory: the arrays in one launch
+        const long long most = std::max(nrow, nnz);
+        csr_copy<<<(unsigned)std::min<long long>(pg_cdiv(most, 1024), 8LL * std::max(ctx->num_cu, 1)), 256, 0, ctx->stream>>>(
+            ctx->c_row, nrow, ctx->c_col, want_val ? (const int *)ctx->c_val : nullptr, nnz, row, col, (int *)val);
+        PG_KERNEL_CHECK(ctx);
+        PG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        return PG_OK;
+    }
     auto kind = [](void *p) { return pg_is_device_ptr(p) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost; };
-    if (row) PG_HIP(ctx, hipMemcpyAsync(row, ctx->c_row, ((size_t)ctx->cn + 1) * 4, kind(row), ctx->stream));
-    if (col && ctx->cnnz > 0)
-        PG_HIP(ctx, hipMemcpyAsync(col, ctx->c_col, (size_t)ctx->cnnz * 4, kind(col), ctx->stream));
-    if (val && ctx->cweighted && ctx->cnnz > 0)
-        PG_HIP(ctx, hipMemcpyAsync(val, ctx->c_val, (size_t)ctx->cnnz * 4, kind(val), ctx->stream));
+    if (row) PG_HIP(ctx, hipMemcpyAsync(row, ctx->c_row, (size_t)nrow * 4, kind(row), ctx->stream));
+    if (col && nnz > 0) PG_HIP(ctx, hipMemcpyAsync(col, ctx->c_col, (size_t)nnz * 4, kind(col), ctx->stream));
+    if (want_val && nnz > 0) PG_HIP(ctx, hipMemcpyAsync(val, ctx->c_val, (size_t)nnz * 4, kind(val), ctx->stream));
     PG_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return PG_OK;
 }

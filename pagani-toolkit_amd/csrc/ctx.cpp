@@ -116,7 +116,9 @@ pg_status pg_create(pg_ctx **out, int device)
         delete ctx;
         return PG_EDEVICE;
     }
-    for (auto &e : ctx->ev) (void)hipEventCreate(&e);
+    // timing only: no cache flush around the recorded point
+    for (auto &e : ctx->ev)
+        if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) (void)hipEventCreate(&e);
     if (hipHostMalloc(&ctx->h_report, PG_REPORT_BYTES, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
         ctx->h_report = nullptr;

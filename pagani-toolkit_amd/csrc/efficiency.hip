@@ -26,6 +26,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
@@ -480,42 +481,54 @@ __global__ __launch_bounds__(256) void csr_validate(const int *__restrict__ row,
     if (w < n) {
         const long long a = row[w], b = row[w + 1];
         ok = a >= 0 && a <= b && b <= nnz;
-        if (ok && col)
-            for (long long e = a + lane; e < b; e += 64) {
-                const int c = col[e];
-                ok = ok && c >= 0 && c < n && !(sorted && e > a && col[e - 1] >= c);
+        if (ok && col) {
+            // four loads in flight; a column's left neighbour comes from the
+            // lane before, the batch before, or nowhere at the row's start
+            int prev = -1;  // last column of the batch before
+            for (long long e0 = a; e0 < b; e0 += 256) {
+                int c[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const long long e = e0 + 64 * u + lane;
+                    c[u] = e < b ? col[e] : INT_MAX;
+                }
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const bool in = e0 + 64 * u + lane < b;
+                    int left = __shfl_up(c[u], 1);
+                    if (lane == 0) left = prev;
+                    ok = ok && (!in || (c[u] >= 0 && c[u] < n && !(sorted && left >= c[u])));
+                    prev = __shfl(c[u], 63);
+                }
             }
+        }
     }
     if (w == 0 && lane == 0) ok = ok && row[0] == 0 && (long long)row[n] == nnz;
-    if (!ok) atomicOr(bad, 1);
+    if (!ok) *(volatile int *)bad = 1;
 }
 }  // namespace
 
-namespace {
-__global__ void flag_clear(int *f) { *f = 0; }
-}  // namespace
-
-pg_status pg_validate_csr_flag(pg_ctx *ctx, const int32_t *drow, const int32_t *dcol, int32_t n, int64_t nnz,
-                               bool sorted, int *bad)
+void pg_validate_launch(pg_ctx *ctx, const int32_t *drow, const int32_t *dcol, int32_t n, int64_t nnz, bool sorted,
+                        int *bad)
 {
-    hipStream_t st = ctx->stream;
-    int hbad = 0;
-    flag_clear<<<1, 1, 0, st>>>(bad);
     const long long waves = std::max<long long>(n, 1);
-    csr_validate<<<(unsigned)pg_cdiv(waves, 4), 256, 0, st>>>(drow, dcol, n, nnz, sorted ? 1 : 0, bad);
-    PG_KERNEL_CHECK(ctx);
-    PG_HIP(ctx, hipMemcpyAsync(&hbad, bad, 4, hipMemcpyDeviceToHost, st));
-    PG_HIP(ctx, hipStreamSynchronize(st));
-    if (hbad)
-        return pg_fail(ctx, PG_EFORMAT, "malformed CSR (row not 0..nnz non-decreasing, col out of range%s)",
-                       sorted ? " or columns not ascending in a row" : "");
-    return PG_OK;
+    csr_validate<<<(unsigned)pg_cdiv(waves, 4), 256, 0, ctx->stream>>>(drow, dcol, n, nnz, sorted ? 1 : 0, bad);
+}
+
+pg_status pg_malformed(pg_ctx *ctx, bool sorted)
+{
+    return pg_fail(ctx, PG_EFORMAT, "malformed CSR (row not 0..nnz non-decreasing, col out of range%s)",
+                   sorted ? " or columns not ascending in a row" : "");
 }
 
 pg_status pg_validate_csr(pg_ctx *ctx, const int32_t *drow, const int32_t *dcol, int32_t n, int64_t nnz,
                           bool sorted)
 {
-    int *bad;
-    PG_TRY(pg_bufT(ctx, "csr.bad", 1, &bad));
-    return pg_validate_csr_flag(ctx, drow, dcol, n, nnz, sorted, bad);
+    // the flag is the context's pinned word: no clearing launch, no copy
+    volatile int *bad = &pg_check(ctx)->bad;
+    *bad = 0;
+    pg_validate_launch(ctx, drow, dcol, n, nnz, sorted, (int *)bad);
+    PG_KERNEL_CHECK(ctx);
+    PG_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return *bad ? pg_malformed(ctx, sorted) : PG_OK;
 }

@@ -287,11 +287,22 @@ __global__ __launch_bounds__(256) void triangles_lists(const int *__restrict__ r
 // Fixed-order mean by one work-group, eight loads in flight per thread (58,000
 // floats: 18 us, 54 us with 256 threads and one load in flight).
 constexpr int MEAN_TPB = 1024;
+// With chk (pinned) the mean and the CSR check's flag go there and the device
+// flag is left clear for the next call.
 template <class T>
-__global__ __launch_bounds__(MEAN_TPB) void mean_kernel(const T *__restrict__ x, int n, double *__restrict__ out)
+__global__ __launch_bounds__(MEAN_TPB) void mean_kernel(const T *__restrict__ x, int n, double *__restrict__ out,
+                                                        PgCheck *__restrict__ chk = nullptr, int *bad = nullptr)
 {
     __shared__ double red[MEAN_TPB];
     const int tid = threadIdx.x;
+    if (bad && *bad) {
+        __syncthreads();
+        if (tid == 0) {
+            chk->bad = 1;
+            *bad = 0;
+        }
+        return;
+    }
     double s = 0.0;
     for (int i0 = tid; i0 < n; i0 += 8 * MEAN_TPB) {
         T v[8];
@@ -306,7 +317,14 @@ __global__ __launch_bounds__(MEAN_TPB) void mean_kernel(const T *__restrict__ x,
         if (tid < off) red[tid] += red[tid + off];
         __syncthreads();
     }
-    if (tid == 0) *out = n > 0 ? red[0] / (double)n : 0.0;
+    if (tid == 0) {
+        const double m = n > 0 ? red[0] / (double)n : 0.0;
+        if (out) *out = m;
+        if (chk) {
+            chk->bad = 0;
+            chk->mean = m;
+        }
+    }
 }
 
 // Largest of m floats in two launches: MAX_WG work-groups take the part maxima
@@ -803,14 +821,15 @@ void launch_triangles(hipStream_t st, const int *row, const int *col, int n, voi
                                                                             skip);
 }
 
-pg_status run_triangles(pg_ctx *ctx, const int *row, const int *col, int n, int64_t nnz, long long *tri, float *cp)
+pg_status run_triangles(pg_ctx *ctx, const int *row, const int *col, int n, int64_t nnz, long long *tri, float *cp,
+                        const unsigned *skip = nullptr)
 {
     unsigned char *up;
     int4 *meta;
     PG_TRY(pg_bufT(ctx, "cp.up", upper_room(n, nnz) * (upper16(n) ? 2 : 4), &up));
     PG_TRY(pg_bufT(ctx, "cp.meta", (size_t)n, &meta));
-    if (upper16(n)) launch_triangles<uint16_t>(ctx->stream, row, col, n, up, meta, tri, cp);
-    else launch_triangles<uint32_t>(ctx->stream, row, col, n, up, meta, tri, cp);
+    if (upper16(n)) launch_triangles<uint16_t>(ctx->stream, row, col, n, up, meta, tri, cp, skip);
+    else launch_triangles<uint32_t>(ctx->stream, row, col, n, up, meta, tri, cp, skip);
     PG_KERNEL_CHECK(ctx);
     return PG_OK;
 }
@@ -842,20 +861,42 @@ extern "C" pg_status pg_cp_binary(pg_ctx *ctx, const int32_t *row, const int32_t
     if (!cp) return pg_fail(ctx, PG_EINVAL, "cp is NULL");
     PG_HIP(ctx, hipSetDevice(ctx->device));
     const int *drow, *dcol;
-    PG_TRY(stage_csr(ctx, row, col, nullptr, n, nnz, true, &drow, &dcol, nullptr));
+    PG_TRY(pg_check_csr_args(ctx, row, col, n, nnz));
+    PG_TRY(pg_in(ctx, row, (size_t)n + 1, "in.row", &drow));
+    PG_TRY(pg_in(ctx, col, (size_t)nnz, "in.col", &dcol));
     const int nw = (n + 31) / 32;
-    if ((size_t)nw * 4 + 4096 > ctx->lds_per_block) return pg_fail(ctx, PG_ENOTSUP, "n too large for LDS bitmap");
+    if ((size_t)nw * 4 + 4096 > ctx->lds_per_block) {
+        PG_TRY(pg_validate_csr(ctx, drow, dcol, n, nnz, true));  // a malformed CSR is reported first
+        return pg_fail(ctx, PG_ENOTSUP, "n too large for LDS bitmap");
+    }
+    // one wait: the check raises a device flag that the kernels behind it look
+    // at before they index with the CSR, and the mean's launch reports both
     float *dcp;
-    double *dmean;
-    PG_TRY(pg_bufT(ctx, "cp.mean", 1, &dmean));
+    int *bad;
+    const bool fresh = ctx->bufs.find("cp.bad") == ctx->bufs.end();
+    PG_TRY(pg_bufT(ctx, "cp.bad", 1, &bad));
     PG_TRY(pg_out(ctx, cp, (size_t)n, "out.cp", &dcp));
     hipStream_t st = ctx->stream;
-    if (n > 0) PG_TRY(run_triangles(ctx, drow, dcol, n, nnz, nullptr, dcp));
-    mean_kernel<float><<<1, MEAN_TPB, 0, st>>>(dcp, n, dmean);
+    if (fresh) PG_HIP(ctx, hipMemsetAsync(bad, 0, 4, st));
+    pg_validate_launch(ctx, drow, dcol, n, nnz, true, bad);
+    if (n > 0) {
+        const pg_status rs = run_triangles(ctx, drow, dcol, n, nnz, nullptr, dcp, (const unsigned *)bad);
+        if (rs != PG_OK) {
+            (void)hipMemsetAsync(bad, 0, 4, st);  // as the mean's launch would have left it
+            return rs;
+        }
+    }
+    PgCheck *chk = pg_check(ctx);
+    mean_kernel<float><<<1, MEAN_TPB, 0, st>>>(dcp, n, nullptr, chk, bad);
     PG_KERNEL_CHECK(ctx);
-    PG_TRY(pg_out_finish(ctx, cp, dcp, (size_t)n));
-    if (mean) PG_HIP(ctx, hipMemcpyAsync(mean, dmean, 8, pg_is_device_ptr(mean) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, st));
     PG_HIP(ctx, hipStreamSynchronize(st));
+    if (*(volatile int *)&chk->bad) return pg_malformed(ctx, true);
+    const double m = *(volatile double *)&chk->mean;
+    PG_TRY(pg_out_finish(ctx, cp, dcp, (size_t)n));
+    const bool dmean = mean && pg_is_device_ptr(mean);
+    if (dmean) PG_HIP(ctx, hipMemcpyAsync(mean, &m, 8, hipMemcpyHostToDevice, st));
+    else if (mean) *mean = m;
+    if (dcp != cp || dmean) PG_HIP(ctx, hipStreamSynchronize(st));
     return PG_OK;
 }
 
@@ -947,7 +988,7 @@ void pg_cohort_metrics_free(PgCohortMetrics *M) { delete M; }
 
 namespace {
 // Fixed scratch of pg_cp_binary_static: triangle counts of up to
-// PG_CP_STATIC_MAX_N vertices, then the FP64 mean, then the CSR check flag.
+// PG_CP_STATIC_MAX_N vertices, then the FP64 mean.
 // One copy per GPU, held while the library is loaded; host code reaches it
 // only through the address pg_static_scratch looks up per device.
 constexpr size_t STATIC_TRI_BYTES = (size_t)PG_CP_STATIC_MAX_N * 8;
@@ -990,8 +1031,7 @@ extern "C" pg_status pg_cp_binary_static(pg_ctx *ctx, const int32_t *row, const 
     unsigned char *base = (unsigned char *)ctx->static_scratch;
     long long *dtri = (long long *)base;
     double *dmean = (double *)(base + STATIC_TRI_BYTES);
-    int *bad = (int *)(base + STATIC_TRI_BYTES + 64);
-    PG_TRY(pg_validate_csr_flag(ctx, row, col, n, nnz, true, bad));
+    PG_TRY(pg_validate_csr(ctx, row, col, n, nnz, true));
     const int nw = (n + 31) / 32;
     if ((size_t)nw * 4 + 4096 > ctx->lds_per_block) return pg_fail(ctx, PG_ENOTSUP, "n too large for LDS bitmap");
     hipStream_t st = ctx->stream;

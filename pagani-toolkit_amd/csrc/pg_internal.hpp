@@ -59,8 +59,14 @@ struct pg_ctx {
 
 pg_status pg_fail(pg_ctx *ctx, pg_status st, const char *fmt, ...);
 
-// size of pg_ctx::h_report
+// size of pg_ctx::h_report; its last bytes are the CSR checks' words
 constexpr size_t PG_REPORT_BYTES = 4096;
+struct PgCheck {
+    int bad;
+    int pad;
+    double mean;  // pg_cp_binary's result, beside the check it waited for
+};
+inline PgCheck *pg_check(pg_ctx *ctx) { return (PgCheck *)((char *)ctx->h_report + PG_REPORT_BYTES - sizeof(PgCheck)); }
 
 #define PG_HIP(ctx, expr)                                                                  \
     do {                                                                                   \
@@ -142,9 +148,11 @@ pg_status pg_zscore64(pg_ctx *ctx, const float *dbold, int layout, int n, int t,
 // each row.  PG_EFORMAT otherwise.  Synchronises the stream.
 pg_status pg_validate_csr(pg_ctx *ctx, const int32_t *drow, const int32_t *dcol, int32_t n, int64_t nnz,
                           bool sorted);
-// The same check with a caller-provided device flag (no allocation).
-pg_status pg_validate_csr_flag(pg_ctx *ctx, const int32_t *drow, const int32_t *dcol, int32_t n, int64_t nnz,
-                               bool sorted, int *bad);
+// The check's launch alone: *bad = 1 (device or pinned memory) on a malformed
+// CSR, else unchanged.
+void pg_validate_launch(pg_ctx *ctx, const int32_t *drow, const int32_t *dcol, int32_t n, int64_t nnz, bool sorted,
+                        int *bad);
+pg_status pg_malformed(pg_ctx *ctx, bool sorted);
 
 // Device address of this device's fixed scratch array of the allocation-free
 // entry points (graph.hip), looked up once per device; called by pg_create
