@@ -17,10 +17,9 @@
 //    that a second kernel recomputes in the oracle's sequential order, one
 //    thread per pair (a lane stalling its wave for a 240-step dependent sum
 //    would idle the matrix cores).
-//  * The epilogue writes every pair's FP32 r into a per-subject packed buffer
-//    straight from the MFMA result registers (16 consecutive columns of a row
-//    per 16 lanes); a streaming kernel then adds r, or its Fisher z, to the
-//    packed accumulator (the first subject without Fisher is written in place).
+//  * The epilogue adds every pair's FP32 r, or its Fisher z, to the packed
+//    accumulator straight from the MFMA result registers (16 consecutive
+//    columns of a row per 16 lanes); the first subject is written.
 //
 // After the last subject: divide by the subject count, inverse Fisher.  Then
 // thresholds as the reference applies them to the averaged matrix: r-mode
@@ -37,6 +36,7 @@
 #include <vector>
 
 #include "pg_internal.hpp"
+#include "pg_pairsum.hpp"
 #include "pg_scan.hpp"
 
 namespace {
@@ -108,6 +108,19 @@ constexpr int GTHREADS = 512;
 constexpr int GLDS = 2 * 2 * GT * GLD;      // doubles: 2 buffers x (A, B)
 constexpr int GNLD = GT * GKC / GTHREADS;   // doubles per thread per panel and step
 
+// What a pair's r becomes in the accumulator: r itself (the first subject of a
+// plain average), += r, = its Fisher z (the first subject: the accumulator
+// needs no clearing), += its Fisher z.
+enum { CM_SET, CM_ADD, CM_SET_Z, CM_ADD_Z };
+template <int MODE>
+__device__ __forceinline__ float cm_value(float r, float acc)
+{
+#pragma clang fp contract(off)
+    const float x = MODE == CM_SET_Z || MODE == CM_ADD_Z ? fisher_f(r) : r;
+    return MODE == CM_SET ? x : (MODE == CM_SET_Z ? 0.0f + x : acc + x);
+}
+
+template <int MODE>
 __global__ __launch_bounds__(GTHREADS) __attribute__((amdgpu_waves_per_eu(4))) void gram64_r(const double *__restrict__ z, int n, int t, int tp,
                                                      double delta, float *__restrict__ out, int2 *__restrict__ amb,
                                                      unsigned *__restrict__ namb, unsigned cap)
@@ -165,14 +178,26 @@ __global__ __launch_bounds__(GTHREADS) __attribute__((amdgpu_waves_per_eu(4))) v
         __syncthreads();
     }
     // every pair's FP32 r, straight from the MFMA registers (16 consecutive
-    // columns of a row per 16 lanes)
+    // columns of a row per 16 lanes), into the accumulator.  The logarithms
+    // share the FP64 unit with the MFMAs, so this kernel takes as long as the
+    // Gram and a pass of its own did (1,065 against 793 + 237 us at n =
+    // 12,011), but the subject buffer and its 576 MB of traffic are gone:
+    // three subjects and a threshold 3.45 against 3.53 ms
 #pragma unroll
     for (int m = 0; m < 2; m++)
 #pragma unroll
-        for (int q = 0; q < 4; q++)
+        for (int v = 0; v < 4; v++) {
+            const int i = i0 + wr * 32 + m * 16 + (lane >> 4) + 4 * v;
+            float *row = out + pidx(i, 0, n);  // row[j], j > i
+            float x[4];
+            if (MODE == CM_ADD || MODE == CM_ADD_Z)
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int i = i0 + wr * 32 + m * 16 + (lane >> 4) + 4 * v;
+                for (int q = 0; q < 4; q++) {
+                    const int j = j0 + wc * 64 + q * 16 + (lane & 15);
+                    x[q] = i < j && j < n ? row[j] : 0.0f;
+                }
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
                 const int j = j0 + wc * 64 + q * 16 + (lane & 15);
                 if (i < j && j < n) {
                     bool a;
@@ -186,45 +211,45 @@ __global__ __launch_bounds__(GTHREADS) __attribute__((amdgpu_waves_per_eu(4))) v
                         }
                         f = seq_r(z + (long long)i * tp, z + (long long)j * tp, t);
                     }
-                    out[pidx(i, j, n)] = f;
+                    row[j] = cm_value<MODE>(f, x[q]);
                 }
             }
+        }
 }
 
-// The pairs whose rounding the Gram left open: one thread each, the oracle's
-// sequential sum.
-__global__ void gram64_recheck(const double *__restrict__ z, int n, int t, int tp, float *__restrict__ out,
-                               const int2 *__restrict__ amb, const unsigned *__restrict__ namb, unsigned cap)
+// The pairs whose rounding the Gram left open: the oracle's sequential sum, 16
+// pairs per wave (a thread per pair waited for 2 t loads of 64 rows each: 57
+// against 10.5 us at n = 12,011, t = 210).
+template <int MODE>
+__global__ __launch_bounds__(256) void gram64_recheck(const double *__restrict__ z, int n, int t, int tp,
+                                                      float *__restrict__ out, const int2 *__restrict__ amb,
+                                                      const unsigned *__restrict__ namb, unsigned cap)
+{
+    __shared__ __align__(16) double prod[4][pgdev::PairSum<16>::LDS_DOUBLES];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const unsigned m = min(*namb, cap);
+    for (unsigned b0 = (blockIdx.x * 4 + w) * 16; b0 < m; b0 += gridDim.x * 64) {
+        const bool own = lane < 16 && b0 + lane < m;
+        const int2 e = own ? amb[b0 + lane] : make_int2(0, 0);
+        const double r = pgdev::clamp_r(pgdev::PairSum<16>::run(e, z, tp, t, 0.0, lane, prod[w]));
+        if (own) {
+            float *p = out + pidx(e.x, e.y, n);
+            *p = cm_value<MODE>((float)r, MODE == CM_ADD || MODE == CM_ADD_Z ? *p : 0.0f);
+        }
+    }
+}
+
+// The same, a thread per pair, for rows beyond 32-bit offsets.
+template <int MODE>
+__global__ void gram64_recheck_wide(const double *__restrict__ z, int n, int t, int tp, float *__restrict__ out,
+                                    const int2 *__restrict__ amb, const unsigned *__restrict__ namb, unsigned cap)
 {
     const unsigned k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= min(*namb, cap)) return;
     const int2 p = amb[k];
-    out[pidx(p.x, p.y, n)] = seq_r(z + (long long)p.x * tp, z + (long long)p.y * tp, t);
-}
-
-// post_block (U CorMat.cpp:806-838): acc += r, or its Fisher z
-// 16-byte accesses (4 pairs per thread and step), the last m % 4 pairs one by
-// one; the buffers are device allocations, so 16-byte aligned.
-__global__ void cm_accumulate(long long m, const float *__restrict__ r, int fisher, float *__restrict__ acc)
-{
-#pragma clang fp contract(off)
-    const long long m4 = m >> 2, stride = (long long)gridDim.x * blockDim.x;
-    const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const float4 *r4 = (const float4 *)r;
-    float4 *a4 = (float4 *)acc;
-    for (long long q = t0; q < m4; q += stride) {
-        const float4 x = r4[q];
-        float4 y = a4[q];
-        y.x = y.x + (fisher ? fisher_f(x.x) : x.x);
-        y.y = y.y + (fisher ? fisher_f(x.y) : x.y);
-        y.z = y.z + (fisher ? fisher_f(x.z) : x.z);
-        y.w = y.w + (fisher ? fisher_f(x.w) : x.w);
-        a4[q] = y;
-    }
-    for (long long q = 4 * m4 + t0; q < m; q += stride) {
-        const float x = r[q];
-        acc[q] = acc[q] + (fisher ? fisher_f(x) : x);
-    }
+    float *o = out + pidx(p.x, p.y, n);
+    *o = cm_value<MODE>(seq_r(z + (long long)p.x * tp, z + (long long)p.y * tp, t),
+                        MODE == CM_ADD || MODE == CM_ADD_Z ? *o : 0.0f);
 }
 
 // z rows padded with zeros to [npad][tp]: exact zeros leave every FP64 sum
@@ -237,6 +262,8 @@ __global__ void cm_pad(const double *__restrict__ z, int n, int t, int npad, int
     zp[q] = (i < n && l < t) ? z[(long long)i * t + l] : 0.0;
 }
 
+// The accumulator of no subjects (only read by a caller that adds none: the
+// first subject overwrites it).
 __global__ void cm_zero(long long m, float *__restrict__ a)
 {
     for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < m; q += (long long)gridDim.x * blockDim.x)
@@ -427,8 +454,6 @@ extern "C" pg_status pg_cormat_begin(pg_ctx *ctx, int32_t n, int32_t fisher)
     PG_HIP(ctx, hipSetDevice(ctx->device));
     const long long m1 = (long long)n * (n - 1) / 2;
     PG_TRY(pg_bufT(ctx, "cm.acc", (size_t)m1, &ctx->cm_acc));
-    cm_zero<<<(unsigned)std::min<long long>(pg_cdiv(m1, 256), 65536), 256, 0, ctx->stream>>>(m1, ctx->cm_acc);
-    PG_KERNEL_CHECK(ctx);
     ctx->cm_n = n;
     ctx->cm_nsub = 0;
     ctx->cm_fisher = fisher ? 1 : 0;
@@ -458,7 +483,6 @@ extern "C" pg_status pg_cormat_add(pg_ctx *ctx, const float *bold, int32_t t, in
     cm_pad<<<(unsigned)pg_cdiv((long long)npad * tp, 256), 256, 0, st>>>(z64, n, t, npad, tp, zp);
     const double delta = 2.5 * (double)t * std::ldexp(1.0, -53);
     const size_t shm = (size_t)GLDS * sizeof(double);
-    PG_HIP(ctx, hipFuncSetAttribute((const void *)gram64_r, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
     // ambiguous-rounding list: about one pair in 10^4 is expected
     const long long m1 = (long long)n * (n - 1) / 2;
     unsigned cap = (unsigned)std::min<long long>(std::max<long long>(m1 / 256, 1 << 16), 1 << 26);
@@ -468,18 +492,22 @@ extern "C" pg_status pg_cormat_add(pg_ctx *ctx, const float *bold, int32_t t, in
     PG_TRY(pg_bufT(ctx, "cm.amb", std::max(cap, 1u), &amb));
     PG_TRY(pg_bufT(ctx, "cm.namb", 1, &namb));
     PG_HIP(ctx, hipMemsetAsync(namb, 0, 4, st));
-    // the first subject without Fisher is its own sum (0 + r = r): written in
-    // place; otherwise into the subject buffer, then accumulated
-    const bool direct = ctx->cm_nsub == 0 && !ctx->cm_fisher;
-    float *r = ctx->cm_acc;
-    if (!direct) PG_TRY(pg_bufT(ctx, "cm.r", (size_t)m1, &r));
-    gram64_r<<<dim3((unsigned)nt, (unsigned)nt), GTHREADS, shm, st>>>(zp, n, t, tp, delta, r, amb, namb, cap);
-    if (cap > 0)
-        gram64_recheck<<<(unsigned)pg_cdiv(cap, 256), 256, 0, st>>>(zp, n, t, tp, r, amb, namb, cap);
-    if (!direct)
-        cm_accumulate<<<(unsigned)std::min<long long>(pg_cdiv(m1, 256), 65536), 256, 0, st>>>(
-            m1, r, ctx->cm_fisher, ctx->cm_acc);
-    PG_KERNEL_CHECK(ctx);
+    auto run = [&](auto gram, auto recheck, auto recheck_wide) -> pg_status {
+        PG_HIP(ctx, hipFuncSetAttribute((const void *)gram, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+        gram<<<dim3((unsigned)nt, (unsigned)nt), GTHREADS, shm, st>>>(zp, n, t, tp, delta, ctx->cm_acc, amb, namb, cap);
+        if (cap > 0 && (unsigned long long)npad * tp < (1ull << 32))
+            recheck<<<(unsigned)std::min<long long>(pg_cdiv(cap, 64), 4LL * std::max(ctx->num_cu, 1)), 256, 0, st>>>(
+                zp, n, t, tp, ctx->cm_acc, amb, namb, cap);
+        else if (cap > 0)
+            recheck_wide<<<(unsigned)pg_cdiv(cap, 256), 256, 0, st>>>(zp, n, t, tp, ctx->cm_acc, amb, namb, cap);
+        PG_KERNEL_CHECK(ctx);
+        return PG_OK;
+    };
+    const bool first = ctx->cm_nsub == 0;
+    if (!ctx->cm_fisher && first) PG_TRY(run(gram64_r<CM_SET>, gram64_recheck<CM_SET>, gram64_recheck_wide<CM_SET>));
+    else if (!ctx->cm_fisher) PG_TRY(run(gram64_r<CM_ADD>, gram64_recheck<CM_ADD>, gram64_recheck_wide<CM_ADD>));
+    else if (first) PG_TRY(run(gram64_r<CM_SET_Z>, gram64_recheck<CM_SET_Z>, gram64_recheck_wide<CM_SET_Z>));
+    else PG_TRY(run(gram64_r<CM_ADD_Z>, gram64_recheck<CM_ADD_Z>, gram64_recheck_wide<CM_ADD_Z>));
     PG_HIP(ctx, hipStreamSynchronize(st));
     ctx->cm_nsub++;
     return PG_OK;
@@ -508,6 +536,10 @@ extern "C" pg_status pg_cormat_read(pg_ctx *ctx, int64_t offset, int64_t count, 
     const long long m1 = (long long)ctx->cm_n * (ctx->cm_n - 1) / 2;
     if (!dst || offset < 0 || count < 0 || offset + count > m1) return pg_fail(ctx, PG_EINVAL, "bad range");
     PG_HIP(ctx, hipSetDevice(ctx->device));
+    if (ctx->cm_nsub == 0) {
+        cm_zero<<<(unsigned)std::min<long long>(pg_cdiv(m1, 256), 65536), 256, 0, ctx->stream>>>(m1, ctx->cm_acc);
+        PG_KERNEL_CHECK(ctx);
+    }
     const hipMemcpyKind kind = pg_is_device_ptr(dst) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
     PG_HIP(ctx, hipMemcpyAsync(dst, ctx->cm_acc + offset, (size_t)count * 4, kind, ctx->stream));
     PG_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "pg_internal.hpp"
+#include "pg_pairsum.hpp"
 #include "pg_rowsort.hpp"
 
 namespace {
@@ -36,6 +37,11 @@ namespace {
 #ifndef PG_GRAM_KC
 #define PG_GRAM_KC 64
 #endif
+using pgdev::clamp_r;
+using pgdev::d2a;
+using pgdev::PAIR_LDS;
+using pgdev::PairSum;
+
 constexpr int TM = PG_GRAM_TM;  // Gram tile rows (128 or 256)
 constexpr int TN = 128;         // Gram tile columns
 constexpr int RT = TM / TN;     // tile aspect ratio
@@ -1446,96 +1452,6 @@ __global__ void accept_kernel(const int2 *__restrict__ pairs, const float *__res
     }
 }
 
-// FP64 r of P pairs by one wave, exactly as r64_pair forms it (lane p < P holds
-// pair p in e and gets its unclamped sum).  The wave walks the pairs' rows TC
-// time points at a time: TC / 2 lanes read one row's run of TC * 8 bytes, 16
-// bytes each, so a load covers whole runs of a few rows (a thread per pair
-// touches 64 rows per load and is bound by the texture addresser: 64 lines
-// for 512 bytes).  The rounded products go through LDS and lane p adds pair
-// p's in time order; the next run's loads are in flight under the sums.
-// P * TC = 1024 keeps 16 loads of 16 bytes per lane in flight.  P = 64 sums
-// on every lane (bulk); P = 16 takes t / 64 dependent rounds instead of t / 16
-// (lists that do not fill the chip with 64 pairs per wave).
-// Two layouts.  Rows: z[i * t + l], l = 0 .. t - 1; a row starts at a multiple
-// of 8 bytes only (odd t): d2u has that alignment, and a global 16-byte load
-// needs no more than 4; the run past t is read at the row's last two points
-// and masked to zero (a zero product leaves the sum: it starts at +0); n * t <
-// 2^32 and t >= 2, checked by the caller.  CHUNKS (P = 64): zchunk_copy's
-// z[(c * n + i) * 16 + l % 16], zero past t, so every run is one 128-byte line
-// (a row's run straddles two); c counts the chunks from the caller's first.
-// prod: this wave's P * (TC + 2) doubles of LDS; the padding of two keeps the
-// 16-byte row reads off each other's banks.
-typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
-typedef double d2a __attribute__((ext_vector_type(2)));
-template <int P, bool CHUNKS = false>
-struct PairSum {
-    static constexpr int TC = 1024 / P, LPR = TC / 2, RPL = 64 / LPR, M = P / RPL, LDP = TC + 2;
-    static constexpr int LDS_DOUBLES = P * LDP;
-    static_assert(!CHUNKS || TC == 16, "a chunk is one run");
-    // rows: t points per row (n unused); chunks: len / 16 chunks of n rows
-    static __device__ __forceinline__ double run(int2 e, const double *__restrict__ z, int n, int len, double sum,
-                                                 int lane, double *__restrict__ prod)
-    {
-#pragma clang fp contract(off)
-        const int rl = lane / LPR, cl = 2 * (lane % LPR);
-        const unsigned stride = CHUNKS ? (unsigned)TC : (unsigned)len;
-        unsigned oa[M], ob[M];
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            oa[m] = (unsigned)__shfl(e.x, m * RPL + rl) * stride;
-            ob[m] = (unsigned)__shfl(e.y, m * RPL + rl) * stride;
-        }
-        d2a x[M], y[M];
-        auto load = [&](int l0) {
-            if (CHUNKS) {
-                const double *zc = z + (long long)l0 * n + cl;  // chunk l0 / 16
-#pragma unroll
-                for (int m = 0; m < M; m++) {
-                    x[m] = *(const d2a *)(zc + oa[m]);
-                    y[m] = *(const d2a *)(zc + ob[m]);
-                }
-            } else {
-                const unsigned l = (unsigned)min(l0 + cl, len - 2);
-#pragma unroll
-                for (int m = 0; m < M; m++) {
-                    x[m] = *(const d2u *)(z + (oa[m] + l));
-                    y[m] = *(const d2u *)(z + (ob[m] + l));
-                }
-            }
-        };
-        load(0);
-        for (int l0 = 0; l0 < len; l0 += TC) {
-            const int l = l0 + cl;
-            const bool both = CHUNKS || l + 1 < len, last = !CHUNKS && l + 1 == len;  // last: point len - 1, read as .y
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                const double p0 = x[m].x * y[m].x, p1 = x[m].y * y[m].y;
-                d2a w;
-                w.x = both ? p0 : (last ? p1 : 0.0);
-                w.y = both ? p1 : 0.0;
-                *(d2a *)(prod + (m * RPL + rl) * LDP + cl) = w;
-            }
-            __builtin_amdgcn_wave_barrier();
-            if (l0 + TC < len) load(l0 + TC);
-            if (P == 64 || lane < P) {
-#pragma unroll
-                for (int k = 0; k < TC; k += 2) {
-                    const d2a w = *(const d2a *)(prod + lane * LDP + k);
-                    sum += w.x;
-                    sum += w.y;
-                }
-            }
-            __builtin_amdgcn_wave_barrier();
-        }
-        return sum;
-    }
-};
-constexpr int PAIR_LDS = PairSum<64>::LDS_DOUBLES > PairSum<16>::LDS_DOUBLES ? PairSum<64>::LDS_DOUBLES
-                                                                             : PairSum<16>::LDS_DOUBLES;
-static_assert(PAIR_LDS % 2 == 0, "each wave's products start 16-byte aligned");
-
-__device__ __forceinline__ double clamp_r(double r) { return r > 1.0 ? 1.0 : (r < -1.0 ? -1.0 : r); }
-
 // The same FP64 r of a list of pairs.  A list that gives every wave of the
 // grid 64 pairs takes 64 per wave, a shorter one 16.
 template <int P>
@@ -1549,7 +1465,7 @@ __device__ __forceinline__ double recheck_list(const int2 *__restrict__ pairs, l
         const long long q = b0 + lane;
         const bool own = lane < P && q < c;
         const int2 e = own ? pairs[q] : make_int2(0, 0);
-        const double r = clamp_r(PairSum<P>::run(e, z, 0, t, 0.0, lane, prod));
+        const double r = clamp_r(PairSum<P>::run(e, z, t, t, 0.0, lane, prod));
         if (own) {
             r_out[q] = r;
             if (rfast) err = fmax(err, fabs((double)rfast[q] - r));
@@ -1577,7 +1493,9 @@ __global__ __launch_bounds__(256) void recheck_rows(const int2 *__restrict__ pai
                      : recheck_list<16>(pairs, c, z, t, r_out, rfast, sh, lane, w, prod[w]);
     if (!rfast) return;
     for (int o = 32; o > 0; o >>= 1) err = fmax(err, __shfl_xor(err, o));
-    if (lane == 0 && err > 0.0) atomicMax(errmax, (unsigned long long)__double_as_longlong(err));
+    // thousands of waves on one address: only those that raise it
+    const unsigned long long eb = (unsigned long long)__double_as_longlong(err);
+    if (lane == 0 && eb > __hip_atomic_load(errmax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(errmax, eb);
 }
 
 // FP64 r of the first min(cap, *cnt) listed pairs (recheck_rows when the row
