@@ -466,13 +466,20 @@ constexpr int MAX_BATCHES = 16;  // batches per launch (blockIdx.y)
 struct BatchBufs {
     int nb = 1;            // batches per launch
     int lcap = 0;          // level counters per batch
-    u64 *sigma, *visA, *visB, *p0, *p1;
+    void *sigma;           // path counts, u64 or (while they fit) uint32
+    u64 *visA, *visB, *p0, *p1;
     int *lev, *srcs;
     double *coef, *bcpart;
     unsigned *prog;        // [nb][lcap]: 1 when some wave found new vertices at level d + 1
     unsigned *tot;         // [lcap]: the same over all batches
+    unsigned *big;         // 1 once a path count left 32 bits (NULL: not looked at)
 };
 
+// ST: the path counts' storage.  The level that reaches most vertices is bound
+// by the reads of its neighbours' counts (12.7 TB/s out of the caches at N =
+// 58,000), so they are kept in 32 bits, summed in 64, and a group of batches
+// whose counts outgrow 32 bits (big) is run again in 64.
+template <class ST>
 __global__ void bfs_init(int n, BatchBufs B)
 {
     const long long ns = (long long)n * S;
@@ -480,7 +487,7 @@ __global__ void bfs_init(int n, BatchBufs B)
     if (k >= ns) return;  // ns is a multiple of 64: whole waves return
     const int bb = blockIdx.y, lane = threadIdx.x & 63;
     const long long o = (long long)bb * ns + k;
-    B.sigma[o] = 0;
+    ((ST *)B.sigma)[o] = 0;
     B.lev[o] = -1;
     // absent lanes count as visited
     const u64 absent = __ballot(B.srcs[bb * S + lane] < 0);
@@ -495,15 +502,17 @@ __global__ void bfs_init(int n, BatchBufs B)
         B.prog[(long long)bb * B.lcap + k] = 0u;
         if (bb == 0) B.tot[k] = 0u;
     }
+    if (k == 0 && bb == 0 && B.big) *B.big = 0u;
 }
 
+template <class ST>
 __global__ void bfs_seed(int n, BatchBufs B)
 {
     const int s = threadIdx.x, bb = blockIdx.y;
     const int v = B.srcs[bb * S + s];
     if (v < 0) return;
     const long long o = (long long)bb * n * S + (long long)v * S + s;
-    B.sigma[o] = 1;
+    ((ST *)B.sigma)[o] = 1;
     B.lev[o] = 0;
     atomicOr(&B.visA[(long long)bb * n + v], 1ull << s);
 }
@@ -512,6 +521,7 @@ __global__ void bfs_seed(int n, BatchBufs B)
 // collects sigma[w][s] = sum of sigma[v][s] over neighbours v reached from s;
 // in an undirected graph those are exactly its level-d neighbours.  A batch
 // whose level d is empty (no progress at d - 1) returns at once.
+template <class ST>
 __global__ __launch_bounds__(256) void bfs_forward(const int *__restrict__ row, const int *__restrict__ col, int n,
                                                    int d, int flip, BatchBufs B)
 {
@@ -524,7 +534,7 @@ __global__ __launch_bounds__(256) void bfs_forward(const int *__restrict__ row, 
     const long long vb0 = (long long)bb * n;
     const u64 *__restrict__ visA = (flip ? B.visB : B.visA) + vb0;
     u64 *__restrict__ visB = (flip ? B.visA : B.visB) + vb0;
-    u64 *__restrict__ sigma = B.sigma + vb0 * S;
+    ST *__restrict__ sigma = (ST *)B.sigma + vb0 * S;
     const u64 vis = visA[w];
     const u64 need = ~vis;
     if (need == 0) {
@@ -544,7 +554,7 @@ __global__ __launch_bounds__(256) void bfs_forward(const int *__restrict__ row, 
         }
         u64 any = __ballot(m != 0);
         while (any) {
-            u64 g[GATHER];
+            ST g[GATHER];
             bool gh[GATHER];
 #pragma unroll
             for (int q = 0; q < GATHER; q++) {
@@ -571,8 +581,9 @@ __global__ __launch_bounds__(256) void bfs_forward(const int *__restrict__ row, 
     const bool fresh = ((need >> lane) & 1ull) && hit;
     const u64 nbits = __ballot(fresh);
     if (fresh) {
-        sigma[(long long)w * S + lane] = acc;
+        sigma[(long long)w * S + lane] = (ST)acc;
         B.lev[(vb0 + w) * S + lane] = d + 1;
+        if (sizeof(ST) == 4 && B.big && (acc >> 32)) pgdev::raise(B.big);
     }
     if (lane == 0) {
         visB[w] = vis | nbits;
@@ -585,11 +596,12 @@ __global__ __launch_bounds__(256) void bfs_forward(const int *__restrict__ row, 
     }
 }
 
-__global__ void bc_coef_init(long long total, const u64 *__restrict__ sigma, double *__restrict__ coef)
+template <class ST>
+__global__ void bc_coef_init(long long total, const ST *__restrict__ sigma, double *__restrict__ coef)
 {
     long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= total) return;
-    u64 s = sigma[k];
+    const ST s = sigma[k];
     coef[k] = s ? 1.0 / (double)s : 0.0;
 }
 
@@ -599,6 +611,7 @@ __global__ void bc_coef_init(long long total, const u64 *__restrict__ sigma, dou
 // delta[v][s] (fixed lane order).  A batch without level d + 1 returns.  vis:
 // the final visited masks (either ping-pong buffer holds them once the
 // batch's BFS has ended).
+template <class ST>
 __global__ __launch_bounds__(256) void bc_backward(const int *__restrict__ row, const int *__restrict__ col, int n,
                                                    int d, BatchBufs B)
 {
@@ -611,7 +624,7 @@ __global__ __launch_bounds__(256) void bc_backward(const int *__restrict__ row, 
     const u64 *__restrict__ vis = B.visA + vb0;
     const u64 *__restrict__ p0 = B.p0 + vb0;
     const u64 *__restrict__ p1 = B.p1 + vb0;
-    const u64 *__restrict__ sigma = B.sigma + vb0 * S;
+    const ST *__restrict__ sigma = (const ST *)B.sigma + vb0 * S;
     double *__restrict__ coef = B.coef + vb0 * S;
     const bool own = B.lev[(vb0 + v) * S + lane] == d;
     const u64 ownm = __ballot(own);
@@ -692,7 +705,8 @@ pg_status batch_bufs(pg_ctx *ctx, int n, int nb, int lcap, BatchBufs &B, bool ne
     const size_t ns = (size_t)n * S * nb, nv = (size_t)n * nb + 1;
     B.nb = nb;
     B.lcap = lcap;
-    PG_TRY(pg_bufT(ctx, "bc.sigma", ns, &B.sigma));
+    PG_TRY(pg_buf(ctx, "bc.sigma", ns * 8, &B.sigma));
+    PG_TRY(pg_bufT(ctx, "bc.big", 1, &B.big));
     PG_TRY(pg_bufT(ctx, "bc.lev", ns, &B.lev));
     PG_TRY(pg_bufT(ctx, "bc.visA", nv, &B.visA));
     PG_TRY(pg_bufT(ctx, "bc.visB", nv, &B.visB));
@@ -707,26 +721,41 @@ pg_status batch_bufs(pg_ctx *ctx, int n, int nb, int lcap, BatchBufs &B, bool ne
     return PG_OK;
 }
 
+__global__ void level_report(const unsigned *__restrict__ tot, const unsigned *__restrict__ big,
+                             PgCheck *__restrict__ chk)
+{
+    chk->level = (int)*tot;
+    chk->big = big ? (int)*big : 0;
+}
+
 // Forward sweep of one group of batches (sources already in B.srcs), host
 // driven: a level is launched while some batch progressed at the previous
 // one.  Returns the number of levels launched after level 0; the final
-// visited masks are in B.visA (and B.visB).
-pg_status run_forward(pg_ctx *ctx, const int *row, const int *col, int n, BatchBufs &B, int *maxlev)
+// visited masks are in B.visA (and B.visB).  *big: a path count left ST's 32
+// bits; the sweep stopped there.
+template <class ST>
+pg_status run_forward(pg_ctx *ctx, const int *row, const int *col, int n, BatchBufs &B, int *maxlev, bool *big)
 {
     hipStream_t st = ctx->stream;
     const long long ns = (long long)n * S;
-    bfs_init<<<dim3((unsigned)pg_cdiv(ns, 256), (unsigned)B.nb), 256, 0, st>>>(n, B);
-    bfs_seed<<<dim3(1, (unsigned)B.nb), S, 0, st>>>(n, B);
+    bfs_init<ST><<<dim3((unsigned)pg_cdiv(ns, 256), (unsigned)B.nb), 256, 0, st>>>(n, B);
+    bfs_seed<ST><<<dim3(1, (unsigned)B.nb), S, 0, st>>>(n, B);
     PG_KERNEL_CHECK(ctx);
+    *big = false;
     int d = 0;
     for (;; d++) {
         if (d + 1 >= B.lcap) return pg_fail(ctx, PG_ENOTSUP, "BFS deeper than %d levels", B.lcap - 1);
-        bfs_forward<<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)B.nb), 256, 0, st>>>(row, col, n, d, d & 1, B);
+        bfs_forward<ST><<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)B.nb), 256, 0, st>>>(row, col, n, d, d & 1, B);
+        // the level's flag and the overflow's, into pinned memory
+        volatile PgCheck *chk = pg_check(ctx);
+        level_report<<<1, 1, 0, st>>>(B.tot + d, B.big, (PgCheck *)chk);
         PG_KERNEL_CHECK(ctx);
-        unsigned prog = 0;
-        PG_HIP(ctx, hipMemcpyAsync(&prog, B.tot + d, 4, hipMemcpyDeviceToHost, st));
         PG_HIP(ctx, hipStreamSynchronize(st));
-        if (prog == 0) break;
+        if (chk->big) {
+            *big = true;
+            break;
+        }
+        if (chk->level == 0) break;
     }
     *maxlev = d;  // levels 0..d hold vertices
     return PG_OK;
@@ -967,14 +996,16 @@ pg_status pg_cohort_metrics_enqueue(PgCohortMetrics *M, const int32_t *row, cons
         fill_f64<<<(unsigned)pg_cdiv((long long)nb * n, 256), 256, 0, st>>>(B.bcpart, (long long)nb * n);
         for (long long g0 = 0; g0 < nsrc; g0 += (long long)nb * S) {
             B.srcs = const_cast<int32_t *>(srcs) + g0;
-            bfs_init<<<dim3((unsigned)pg_cdiv(ns, 256), (unsigned)nb), 256, 0, st>>>(n, B);
-            bfs_seed<<<dim3(1, (unsigned)nb), S, 0, st>>>(n, B);
+            // nothing on the device re-runs a group: 64-bit path counts
+            B.big = nullptr;
+            bfs_init<u64><<<dim3((unsigned)pg_cdiv(ns, 256), (unsigned)nb), 256, 0, st>>>(n, B);
+            bfs_seed<u64><<<dim3(1, (unsigned)nb), S, 0, st>>>(n, B);
             for (int d = 0; d < L; d++)
-                bfs_forward<<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)nb), 256, 0, st>>>(row, col, n, d, d & 1, B);
+                bfs_forward<u64><<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)nb), 256, 0, st>>>(row, col, n, d, d & 1, B);
             bc_depth_check<<<1, 64, 0, st>>>(B.tot, L, status);
-            bc_coef_init<<<(unsigned)pg_cdiv(ns * nb, 256), 256, 0, st>>>(ns * nb, B.sigma, B.coef);
+            bc_coef_init<u64><<<(unsigned)pg_cdiv(ns * nb, 256), 256, 0, st>>>(ns * nb, (const u64 *)B.sigma, B.coef);
             for (int d = L - 1; d >= 1; d--)
-                bc_backward<<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)nb), 256, 0, st>>>(row, col, n, d, B);
+                bc_backward<u64><<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)nb), 256, 0, st>>>(row, col, n, d, B);
         }
         bc_reduce<<<(unsigned)pg_cdiv(n, 256), 256, 0, st>>>(B.bcpart, nb, n, bc);
     }
@@ -1110,6 +1141,25 @@ extern "C" pg_status pg_cp_weighted(pg_ctx *ctx, const int32_t *row, const int32
     return PG_OK;
 }
 
+namespace {
+// Forward and backward sweep of the group of batches in B.srcs; *big: its path
+// counts do not fit ST, nothing was added to the BC shares.
+template <class ST>
+pg_status bc_group(pg_ctx *ctx, const int *row, const int *col, int n, BatchBufs &B, bool *big)
+{
+    hipStream_t st = ctx->stream;
+    const long long total = (long long)n * S * B.nb;
+    int maxlev = 0;
+    PG_TRY(run_forward<ST>(ctx, row, col, n, B, &maxlev, big));
+    if (*big) return PG_OK;
+    bc_coef_init<ST><<<(unsigned)pg_cdiv(total, 256), 256, 0, st>>>(total, (const ST *)B.sigma, B.coef);
+    for (int d = maxlev - 1; d >= 1; d--)
+        bc_backward<ST><<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)B.nb), 256, 0, st>>>(row, col, n, d, B);
+    PG_KERNEL_CHECK(ctx);
+    return PG_OK;
+}
+}  // namespace
+
 extern "C" pg_status pg_bc(pg_ctx *ctx, const int32_t *row, const int32_t *col, int32_t n, int64_t nnz,
                            const int32_t *sources, int64_t nsrc, double *bc)
 {
@@ -1145,17 +1195,19 @@ extern "C" pg_status pg_bc(pg_ctx *ctx, const int32_t *row, const int32_t *col, 
     BatchBufs B;
     PG_TRY(batch_bufs(ctx, n, nb, n + 2, B, true));
     fill_f64<<<(unsigned)pg_cdiv((long long)nb * n, 256), 256, 0, st>>>(B.bcpart, (long long)nb * n);
-    const long long ns = (long long)n * S;
     std::vector<int32_t> pad((size_t)nb * S);
+    bool wide = std::getenv("PAGANI_BC_WIDE") != nullptr;  // 64-bit path counts from the start
     for (long long g0 = 0; g0 < nsrc; g0 += (long long)nb * S) {
         for (int s = 0; s < nb * S; s++) pad[s] = g0 + s < nsrc ? hsrc[g0 + s] : -1;
         PG_HIP(ctx, hipMemcpyAsync(B.srcs, pad.data(), pad.size() * 4, hipMemcpyHostToDevice, st));
-        int maxlev = 0;
-        PG_TRY(run_forward(ctx, drow, dcol, n, B, &maxlev));
-        bc_coef_init<<<(unsigned)pg_cdiv(ns * nb, 256), 256, 0, st>>>(ns * nb, B.sigma, B.coef);
-        for (int d = maxlev - 1; d >= 1; d--)
-            bc_backward<<<dim3((unsigned)pg_cdiv(n, 4), (unsigned)nb), 256, 0, st>>>(drow, dcol, n, d, B);
-        PG_KERNEL_CHECK(ctx);
+        if (!wide) {
+            bool big = false;
+            PG_TRY(bc_group<uint32_t>(ctx, drow, dcol, n, B, &big));
+            wide = big;  // the groups to come as well
+            if (!big) continue;
+        }
+        bool big = false;
+        PG_TRY(bc_group<u64>(ctx, drow, dcol, n, B, &big));
     }
     bc_reduce<<<(unsigned)pg_cdiv(n, 256), 256, 0, st>>>(B.bcpart, nb, n, dbc);
     PG_KERNEL_CHECK(ctx);
@@ -1215,7 +1267,9 @@ extern "C" pg_status pg_bfs(pg_ctx *ctx, const int32_t *row, const int32_t *col,
             for (int s = 0; s < nb * S; s++) pad[s] = g0 + s < nsrc ? hsrc[g0 + s] : -1;
             PG_HIP(ctx, hipMemcpyAsync(B.srcs, pad.data(), pad.size() * 4, hipMemcpyHostToDevice, st));
             int maxlev = 0;
-            PG_TRY(run_forward(ctx, drow, dcol, n, B, &maxlev));
+            bool big = false;
+            B.big = nullptr;  // only the levels are wanted
+            PG_TRY(run_forward<uint32_t>(ctx, drow, dcol, n, B, &maxlev, &big));
             const int nvalid = (int)std::min<long long>((long long)nb * S, nsrc - g0);
             bfs_export<<<dim3((unsigned)pg_cdiv((long long)n * S, 256), (unsigned)nb), 256, 0, st>>>(n, nvalid, B.lev,
                                                                                                  dlev + g0 * n);

@@ -62,7 +62,9 @@ pg_status pg_fail(pg_ctx *ctx, pg_status st, const char *fmt, ...);
 // size of pg_ctx::h_report; its last bytes are the CSR checks' words
 constexpr size_t PG_REPORT_BYTES = 4096;
 struct PgCheck {
-    int bad;
+    int bad;      // the CSR check's flag
+    int level;    // a BFS level's flag, and its path counts' (graph.hip)
+    int big;
     int pad;
     double mean;  // pg_cp_binary's result, beside the check it waited for
 };

@@ -179,3 +179,29 @@ def test_rewire_paths(ctx, n, m, hub, weighted):
         with pytest.raises(pagani_amd.PgError) as ex:
             ctx.rewire(row, bad, v, seed=9)
         assert ex.value.status == 4
+
+
+def _ladder(stages, width):
+    """Layers of `width` vertices, every layer joined to the next: width^k
+    shortest paths over k layers."""
+    edges = [(0, 1 + j) for j in range(width)]
+    for k in range(stages - 1):
+        a, b = 1 + k * width, 1 + (k + 1) * width
+        edges += [(a + i, b + j) for i in range(width) for j in range(width)]
+    return 1 + stages * width, edges
+
+
+# path counts below, at and above 2^32 (16^8): the last stay in 32 bits, the
+# others run again in 64, with more groups of sources behind them
+@pytest.mark.parametrize("stages,width", [(7, 16), (9, 16), (10, 16), (40, 2)])
+def test_bc_path_counts_beyond_32_bits(ctx, stages, width, monkeypatch):
+    from helpers import csr_from_edges
+    n, edges = _ladder(stages, width)
+    row, col, _ = csr_from_edges(n, edges)
+    monkeypatch.setenv("PAGANI_BC_BATCHES", "1")
+    say(f"bc ladder stages={stages} width={width} n={n}")
+    bc = ctx.bc(row, col)
+    obc = O.bc(row, col, np.arange(n, dtype=np.int32))
+    np.testing.assert_allclose(bc, obc, rtol=1e-9, atol=1e-9)
+    src = np.arange(0, n, 2, dtype=np.int32)
+    np.testing.assert_array_equal(ctx.bfs(row, col, src), np.stack([O.bfs(row, col, int(s)) for s in src]))
