@@ -517,6 +517,17 @@ __global__ void bfs_seed(int n, BatchBufs B)
     atomicOr(&B.visA[(long long)bb * n + v], 1ull << s);
 }
 
+// x of a lane given by a wave-uniform index, and a wave-uniform mask as this
+// lane's condition: both stay in scalar registers (three ds_bpermutes per
+// neighbour were what the heavy levels waited for).
+__device__ __forceinline__ u64 read_lane64(u64 x, int lane)
+{
+    const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)x, lane);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(unsigned)(x >> 32), lane);
+    return ((u64)hi << 32) | lo;
+}
+__device__ __forceinline__ bool lanes_of(u64 m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
 // Level d -> d+1 of every batch.  A vertex w not yet reached from source s
 // collects sigma[w][s] = sum of sigma[v][s] over neighbours v reached from s;
 // in an undirected graph those are exactly its level-d neighbours.  A batch
@@ -561,11 +572,10 @@ __global__ __launch_bounds__(256) void bfs_forward(const int *__restrict__ row, 
                 g[q] = 0;
                 gh[q] = false;
                 if (any) {
-                    const int sl = __ffsll((long long)any) - 1;
+                    const int sl = __builtin_ctzll(any);
                     any &= any - 1;
-                    const int vv = __shfl(v, sl);
-                    const u64 mm = __shfl(m, sl);
-                    if ((mm >> lane) & 1ull) {
+                    const int vv = __builtin_amdgcn_readlane(v, sl);
+                    if (lanes_of(read_lane64(m, sl))) {
                         g[q] = sigma[(long long)vv * S + lane];
                         gh[q] = true;
                     }
@@ -648,11 +658,10 @@ __global__ __launch_bounds__(256) void bc_backward(const int *__restrict__ row, 
             for (int q = 0; q < GATHER; q++) {
                 g[q] = 0.0;
                 if (any) {
-                    const int sl = __ffsll((long long)any) - 1;
+                    const int sl = __builtin_ctzll(any);
                     any &= any - 1;
-                    const int ww = __shfl(w, sl);
-                    const u64 mm = __shfl(m, sl);
-                    if ((mm >> lane) & 1ull) g[q] = coef[(long long)ww * S + lane];
+                    const int ww = __builtin_amdgcn_readlane(w, sl);
+                    if (lanes_of(read_lane64(m, sl))) g[q] = coef[(long long)ww * S + lane];
                 }
             }
 #pragma unroll
