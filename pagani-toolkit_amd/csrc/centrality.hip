@@ -31,6 +31,16 @@ constexpr double EC_EPS = 1e-6;     // CUEC_unweighted.cu:28
 constexpr int EC_TPB = pgdev::SP_TPB;
 constexpr int EC_BATCH = 32;        // launches per host check
 
+// rows of block b
+struct EcBlock {
+    int n, R;
+    __device__ __forceinline__ void operator()(int b, int &a0, int &nr) const
+    {
+        a0 = b * R;
+        nr = min(n - a0, R);
+    }
+};
+
 struct EcState {
     int stopped, iters;
     double lam, err1, err2;
@@ -55,8 +65,10 @@ __global__ __launch_bounds__(EC_TPB) void ec_init(int n, int R, double *__restri
 // Iteration k.  Every block takes the norm and the stop decision from the
 // previous launch's partials, then its rows of A u by the LDS-staged SpMV of
 // pg_spmv.hpp on the raw u, scaled once per row.  n = 40,009 with 16 M entries:
-// 21.9 us (27.1 us with one lane per row in blocks of 256 rows), three segments
-// of about 5 us each, staging and look-ups alike.
+// 20.0 us (27.1 us with one lane per row in blocks of 256 rows; 21.9 us with a
+// segment's first entries loaded behind its staging), three segments of about
+// 5 us each, bound by the entries' latency from beyond L2 (32 MB of them an
+// iteration), not by the look-ups: leaving out the fillers' changed nothing.
 template <bool W>
 __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, pgdev::SpLayout L, int n, int R, int G, int k,
                                                   const double *__restrict__ uin, double *__restrict__ uout,
@@ -70,7 +82,7 @@ __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, p
     if (st->stopped) return;
     const int tid = threadIdx.x;
     const int i0 = blockIdx.x * R, nr = min(n - i0, R);
-    const int im = min(i0 + tid, n - 1);
+    const int im = tid < nr ? i0 + (int)L.perm[i0 + tid] : n - 1;  // slot tid's row
     double ui, t;
     bool empty;
     const bool go = pgdev::sp_rows<W>(L, i0, nr, uin, n, xs, pt, rowv, [&]() {
@@ -98,7 +110,7 @@ __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, p
     if (!go) return;
     double s[3] = {0.0, 0.0, 0.0};
     if (tid < nr) {
-        const int i = i0 + tid;
+        const int i = im;
         const double y = empty ? 0.0 : rowv[tid] * t;  // t = inf once u = 0
         vhat[i] = ui * t;
         uout[i] = y;
@@ -197,9 +209,11 @@ extern "C" pg_status pg_eigenvector_centrality(pg_ctx *ctx, const int32_t *row, 
     PG_TRY(pg_bufT(ctx, "ec.idx", room, &L.idx));
     if (dval) PG_TRY(pg_bufT(ctx, "ec.val", room, &L.val));
     PG_TRY(pg_bufT(ctx, "ec.part", 2 * (size_t)n * L.nseg, &parts));
+    PG_TRY(pg_bufT(ctx, "ec.perm", (size_t)n, &L.perm));
     L.part = (int2 *)parts;
     pgdev::sp_build<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, dcol, dval, n, nullptr, nullptr, 0, nullptr, nullptr,
                                                             L, nullptr, 0);
+    pgdev::sp_order<<<(unsigned)G, pgdev::SP_TPB, 0, st>>>(drow, (const int *)nullptr, EcBlock{n, R}, L.perm);
     PG_KERNEL_CHECK(ctx);
     double *u[2], *part[2], *dvh, *dav;
     EcState *dst;

@@ -41,6 +41,18 @@ struct Block {
     int g, fb, nb, no, ng, pad[3];
 };
 
+// nodes of work block b
+struct ModBlock {
+    const Block *blk;
+    int npb;
+    __device__ __forceinline__ void operator()(int b, int &a0, int &nr) const
+    {
+        const Block B = blk[b];
+        a0 = B.no + (b - B.fb) * npb;
+        nr = min(B.no + B.ng - a0, npb);
+    }
+};
+
 // One wave of independent groups (the rounds created but not yet processed),
 // concatenated: group g owns nodes [no[g], no[g] + ng[g]) of the wave and
 // blocks [fb[g], fb[g] + nb[g]); a block never spans two groups, so every
@@ -104,7 +116,7 @@ __global__ __launch_bounds__(TPB) void mod_iter(Wave w, int it)
     double *yn = w.buf[(li + 1) % 3];
     const int i0 = B.no + (b - B.fb) * w.npb, nr = min(B.no + B.ng - i0, w.npb);
     const bool vec = w.stopmode == PG_MOD_STOP_VECTOR;
-    const int i = i0 + min(tid, max(nr - 1, 0));
+    const int i = tid < nr ? i0 + (int)w.lay.perm[i0 + tid] : i0;  // slot tid's node
     double yi, ki, si, ypi, beta, vnp, vn, sum[NPART];
     const bool go = pgdev::sp_rows<W>(w.lay, i0, nr, y + B.no, B.ng, xs, pt, rowv, [&]() {
         // every load that does not wait for the partials goes out before them
@@ -321,6 +333,7 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
         if (dval) PG_TRY(pg_bufT(ctx, "mod.lval", room, &lay.val));
         PG_TRY(pg_bufT(ctx, "mod.part", 2 * nn * nseg, &d_part));
         lay.part = (int2 *)d_part;
+        PG_TRY(pg_bufT(ctx, "mod.perm", nn, &lay.perm));
     }
 
     std::vector<double> k((size_t)n);
@@ -449,6 +462,7 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
         lay.cap = pgdev::sp_cap(gmax);
         pgdev::sp_build<<<(unsigned)pg_cdiv(std::max(nnodes, 1), 4), 256, 0, st>>>(
             drow, dcol, dval, nnodes, d_gid, d_res, lo, d_no, d_rloc, lay, d_sumbg, kmode == PG_MOD_BINARY_K ? 1 : 0);
+        pgdev::sp_order<<<(unsigned)nblk, pgdev::SP_TPB, 0, st>>>(drow, (const int *)d_gid, ModBlock{d_blk, npb}, lay.perm);
         mod_correction<<<(unsigned)pg_cdiv(std::max(nnodes, 1), 256), 256, 0, st>>>(d_gid, d_res, lo, d_kall, d_Kg, m2,
                                                                                    nnodes, d_k, d_sumbg);
         PG_KERNEL_CHECK(ctx);
