@@ -1205,7 +1205,7 @@ extern "C" pg_status pg_bc(pg_ctx *ctx, const int32_t *row, const int32_t *col, 
     PG_TRY(batch_bufs(ctx, n, nb, n + 2, B, true));
     fill_f64<<<(unsigned)pg_cdiv((long long)nb * n, 256), 256, 0, st>>>(B.bcpart, (long long)nb * n);
     std::vector<int32_t> pad((size_t)nb * S);
-    bool wide = std::getenv("PAGANI_BC_WIDE") != nullptr;  // 64-bit path counts from the start
+    bool wide = false;  // 64-bit path counts
     for (long long g0 = 0; g0 < nsrc; g0 += (long long)nb * S) {
         for (int s = 0; s < nb * S; s++) pad[s] = g0 + s < nsrc ? hsrc[g0 + s] : -1;
         PG_HIP(ctx, hipMemcpyAsync(B.srcs, pad.data(), pad.size() * 4, hipMemcpyHostToDevice, st));
