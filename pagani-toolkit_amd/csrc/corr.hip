@@ -2378,8 +2378,10 @@ __global__ __launch_bounds__(BITS_THREADS) void bucket_rows_bits(const long long
                     if ((unsigned)(tid + u * BITS_THREADS) < len)
                         colb[rs + bits_rank(bm4, gbase, (unsigned)ng, x[u])] = (int)(x[u] & COLMASK);
                 }
-                for (unsigned k0 = (unsigned)(tid + BITS_PF * BITS_THREADS); k0 < len;
-                     k0 += BITS_THREADS * BITS_UNROLL) {
+                // the row starts come from lanes 0 .. 15: no lane may leave
+                // this loop before the others of its wave
+                for (unsigned kb = BITS_PF * BITS_THREADS; kb < len; kb += BITS_THREADS * BITS_UNROLL) {
+                    const unsigned k0 = kb + (unsigned)tid;
                     unsigned y[BITS_UNROLL];
 #pragma unroll
                     for (int u = 0; u < BITS_UNROLL; u++)

@@ -27,6 +27,22 @@ def test_weighted_values_bitwise(ctx, n, t):
         np.testing.assert_array_equal(val.view(np.uint32), oval.view(np.uint32))
 
 
+# buckets of 16 rows beyond the 12,288 entries kept in registers, the last wave
+# of their entries with 1 to 63 lanes (bucket lengths vary with the rows)
+@pytest.mark.parametrize("n", [801, 1537, 2999, 4500])
+def test_dense_buckets(ctx, n):
+    from pagani_amd import synth
+    x = synth.bold(n, n, 40, 6)
+    z64, _ = O.zscore(x)
+    for thr in (-0.9, -0.05):
+        say(f"dense buckets n={n} thr={thr}")
+        info = ctx.corr_build(x, n, 40, thr)
+        row, col, _ = ctx.corr_csr(n, info.nnz)
+        orow, ocol, _ = O.corr_csr_r(z64, thr, False)
+        np.testing.assert_array_equal(row, orow)
+        np.testing.assert_array_equal(col, ocol)
+
+
 def _graph(n, m, seed, hub=0):
     """Random network of about m edges plus a vertex joined to `hub` others
     that are themselves a ring, as sorted symmetric CSR with weights."""
