@@ -1432,26 +1432,6 @@ __global__ void recheck_kernel(const int2 *__restrict__ pairs, const unsigned lo
         atomicMax(errmax, (unsigned long long)__double_as_longlong(err));
 }
 
-// r-mode: keep rechecked pairs with r64 > thr; count decisions that differed
-// from the fast test r~ > thr.
-__global__ void accept_kernel(const int2 *__restrict__ pairs, const float *__restrict__ rfast,
-                              const double *__restrict__ r64, const unsigned long long *__restrict__ cnt,
-                              long long cap, double thr, int2 *__restrict__ extra,
-                              unsigned long long *__restrict__ extra_cnt,
-                              unsigned long long *__restrict__ flips)
-{
-    long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    long long c = (long long)min((unsigned long long)cap, *cnt);
-    if (k >= c) return;
-    bool keep = r64[k] > thr;
-    bool fast = (double)rfast[k] > thr;
-    if (keep != fast) atomicAdd(flips, 1ull);
-    if (keep) {
-        unsigned long long p = atomicAdd(extra_cnt, 1ull);
-        extra[p] = pairs[k];
-    }
-}
-
 // The same FP64 r of a list of pairs.  A list that gives every wave of the
 // grid 64 pairs takes 64 per wave, a shorter one 16.
 template <int P>
@@ -1655,6 +1635,31 @@ __global__ __launch_bounds__(SEG_THREADS) void bucket_count(EdgeSrc s, int nbk, 
     });
     __syncthreads();
     for (int b = threadIdx.x; b < nbk; b += SEG_THREADS) cnt[(long long)g * nbk + b] = sc[b];
+}
+
+// r-mode: keep rechecked pairs with r64 > thr; count decisions that differed
+// from the fast test r~ > thr.
+__global__ void accept_kernel(const int2 *__restrict__ pairs, const float *__restrict__ rfast,
+                              const double *__restrict__ r64, const unsigned long long *__restrict__ cnt,
+                              long long cap, double thr, int2 *__restrict__ extra,
+                              unsigned long long *__restrict__ extra_cnt,
+                              unsigned long long *__restrict__ flips, unsigned *__restrict__ bcnt_row)
+{
+    long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    long long c = (long long)min((unsigned long long)cap, *cnt);
+    if (k >= c) return;
+    bool keep = r64[k] > thr;
+    bool fast = (double)rfast[k] > thr;
+    if (keep != fast) atomicAdd(flips, 1ull);
+    if (keep) {
+        unsigned long long p = atomicAdd(extra_cnt, 1ull);
+        const int2 e = pairs[k];
+        extra[p] = e;
+        if (bcnt_row) {  // the list's CSR bucket counts (window_count zeroed them)
+            atomicAdd(&bcnt_row[e.x >> BSH], 1u);
+            atomicAdd(&bcnt_row[e.y >> BSH], 1u);
+        }
+    }
 }
 
 // The window split and the segments' bucket counts in one pass over the
@@ -3936,6 +3941,101 @@ pg_status window_select(CorrRun &R, const SelCtl *ctl, long long ccap, long long
     return PG_OK;
 }
 
+// r threshold from the band-free emit: the segments keep r~ beside every pair
+// above thr - band, and the split into edges and candidates is one pass over
+// them that also takes the CSR's bucket counts.  Bound by the Gram, whose
+// epilogue is the cheaper one (n = 120,000, t = 300: 13.1 -> 11.7 ms).  From
+// R_FREE_MIN_N on, ms of a build at t = 240, 1 to 5% of the pairs kept, unweighted /
+// weighted, by the splitting epilogue and by this: n = 4,099 0.161 / 0.340,
+// 0.171 / 0.350; 8,192 0.235 / 0.559, 0.222 / 0.551; 16,384 0.425 / 0.909, 0.384 /
+// 0.881; 58,000 3.09 / 5.64, 2.77 / 5.39; 120,000 11.6 / 18.6, 10.6 / 17.8.
+// A density beyond the segments' guess (*built stays false, *seg0 is the size
+// that fits) is left to the splitting epilogue, which writes 8 bytes a pair
+// instead of 12 (10% kept, n = 16,384, weighted: 3.56 against 3.70 ms), and so is a
+// device without room for r~.
+constexpr int R_FREE_MIN_N = 8192;
+pg_status build_r_free(CorrRun &R, float thr_eff, long long *seg0, pg_corr_info &inf, bool *built)
+{
+    pg_ctx *ctx = R.ctx;
+    hipStream_t st = R.st;
+    const int n = R.n;
+    unsigned long long *c = R.counters;
+    SpReport *rep = (SpReport *)ctx->h_report;
+    SelCtl hc;
+    std::memset(&hc, 0, sizeof hc);
+    hc.lower = hc.L2 = round_down_f((double)thr_eff - R.band);
+    hc.U2 = round_up_f((double)thr_eff + R.band);
+    hc.ok = 1;
+    R.ga.lower = hc.lower;
+    R.ga.upper = -4.0f;  // every hit is a segment entry
+    const pg_status emitted = R.emit_launch(*seg0, 1 << 10, true);
+    if (emitted == PG_ENOMEM) {
+        PgBuf &b = ctx->bufs["corr.segr"];
+        if (b.p) (void)hipFree(b.p);  // nothing was launched on it
+        b = PgBuf();
+        return PG_OK;
+    }
+    PG_TRY(emitted);
+    sp_report<<<1, 256, 0, st>>>(R.seg_cnt, (int)R.nwg, c, nullptr, nullptr, nullptr, rep);
+    PG_KERNEL_CHECK(ctx);
+    PG_HIP(ctx, hipStreamSynchronize(st));
+    const long long mx = (long long)rep->seg_max, kept = (long long)rep->seg_sum;
+    if (mx > R.seg_cap) {
+        *seg0 = mx + mx / 8 + 4096;
+        return PG_OK;
+    }
+    R.seg_used = (mx + 31) / 32 * 32;
+    PG_HIP(ctx, stage_event(ctx, 3, st));
+    SelCtl *ctl;
+    PG_TRY(pg_bufT(ctx, "corr.selctl", 1, &ctl));
+    long long ccap = std::max<long long>(1 << 16, kept / 64);
+    for (;;) {  // at most twice: the second time every candidate has room
+        PG_HIP(ctx, hipMemcpyAsync(ctl, &hc, sizeof hc, hipMemcpyHostToDevice, st));
+        Window win;
+        PG_TRY(window_candidates(R, ctl, ccap, &win, true));
+        unsigned *bcnt;
+        PG_TRY(pg_bufT(ctx, "corr.bcnt", (size_t)R.nsrc * R.nbk, &bcnt));
+        accept_kernel<<<(unsigned)pg_cdiv(ccap, 256), 256, 0, st>>>(win.cand, win.cand_r, win.cand64, c + 0, ccap,
+                                                                    (double)thr_eff, win.extra, c + 1, c + 2,
+                                                                    bcnt + (size_t)R.nwg * R.nbk);
+        definite_sum<<<1, 1024, 0, st>>>(win.dpart, win.nd, c + 3);
+        PG_KERNEL_CHECK(ctx);
+        // sized and checked as in pg_corr_build's split form
+        long long room = 2 * kept;
+        if (room > INT32_MAX) {
+            sp_report<<<1, 256, 0, st>>>(R.seg_cnt, (int)R.nwg, c, nullptr, nullptr, nullptr, rep);
+            PG_KERNEL_CHECK(ctx);
+            PG_HIP(ctx, hipStreamSynchronize(st));
+            if ((long long)rep->counters[0] > ccap) {
+                ccap = (long long)rep->counters[0];
+                continue;
+            }
+            room = 2 * ((long long)rep->counters[3] + (long long)rep->counters[1]);
+        }
+        EdgeSrc src = R.edges(win.extra, c + 1, ccap);
+        src.seg_r = R.seg_r;
+        src.keep_above_dev = &ctl->U2;
+        PG_HIP(ctx, stage_event(ctx, 4, st));
+        PG_TRY(R.launch_csr(src, room, true));
+        PG_HIP(ctx, stage_event(ctx, 5, st));
+        sp_report<<<1, 256, 0, st>>>(R.seg_cnt, (int)R.nwg, c, nullptr, nullptr, R.row + n, rep);
+        PG_KERNEL_CHECK(ctx);
+        PG_HIP(ctx, hipStreamSynchronize(st));
+        if ((long long)rep->counters[0] <= ccap) break;
+        ccap = (long long)rep->counters[0];
+    }
+    std::memcpy(R.hcnt, rep->counters, sizeof R.hcnt);
+    inf.band_pairs = (long long)R.hcnt[0];
+    inf.band_flips = (long long)R.hcnt[2];
+    inf.band_max_err = host_err(R.hcnt[5]);
+    inf.nnz = 2 * ((long long)R.hcnt[3] + (long long)R.hcnt[1]);
+    inf.s_thresh = (float)(R.m1 > 0 ? 100.0 * (double)inf.nnz / (double)R.m1 / 2.0 : 0.0);
+    if ((long long)rep->rn != inf.nnz)
+        return pg_fail(ctx, PG_EFORMAT, "CSR build mismatch: row[n]=%d nnz=%lld", rep->rn, (long long)inf.nnz);
+    *built = true;
+    return PG_OK;
+}
+
 // The band is error_band()'s proven bound times 1.5; a rechecked pair whose
 // fast r~ is further from its FP64 r than the bound itself means the rounding
 // model behind the band does not hold on this device, and pairs outside the
@@ -3995,12 +4095,16 @@ extern "C" pg_status pg_corr_build(pg_ctx *ctx, const float *bold, int32_t n, in
     int2 *extra = nullptr;
     unsigned long long *extra_cnt = counters + 1, *flips = counters + 2;
 
-    if (!smode) {
+    long long seg0 = pg_cdiv(std::max<long long>((long long)(m1 * 0.03), 1 << 20), nwg) + 4096;
+    bool built = false;
+    if (!smode) PG_HIP(ctx, stage_event(ctx, 2, st));
+    if (!smode && R.g2path && n >= R_FREE_MIN_N) PG_TRY(build_r_free(R, thr_eff, &seg0, inf, &built));
+    if (built) {
+        // r threshold, done
+    } else if (!smode) {
         // ---------------------------------------------------- r threshold
         R.ga.upper = round_up_f((double)thr_eff + band);
         R.ga.lower = round_down_f((double)thr_eff - band);
-        PG_HIP(ctx, stage_event(ctx, 2, st));
-        const long long seg0 = pg_cdiv(std::max<long long>((long long)(m1 * 0.03), 1 << 20), nwg) + 4096;
         PG_TRY(R.emit_pass(seg0, 1 << 22, false));
         PG_HIP(ctx, stage_event(ctx, 3, st));
         const long long definite = R.seg_sum;
@@ -4013,7 +4117,8 @@ extern "C" pg_status pg_corr_build(pg_ctx *ctx, const float *bold, int32_t n, in
             launch_recheck(ctx, st, R.bandl, counters + 0, std::min(nband, R.band_cap), R.z64, n, t, band64, R.band_r,
                            counters + 5);
             accept_kernel<<<(unsigned)pg_cdiv(nband, 256), 256, 0, st>>>(
-                R.bandl, R.band_r, band64, counters + 0, R.band_cap, (double)thr_eff, extra, extra_cnt, flips);
+                R.bandl, R.band_r, band64, counters + 0, R.band_cap, (double)thr_eff, extra, extra_cnt, flips,
+                nullptr);
         }
         PG_KERNEL_CHECK(ctx);
         // the CSR is built for every rechecked pair's room and its size read
@@ -4400,7 +4505,8 @@ extern "C" pg_status pg_corr_select(pg_ctx *ctx, float thr, pg_corr_info *info)
             PG_HIP(ctx, hipMemcpyAsync(E.ctl, &hc, sizeof hc, hipMemcpyHostToDevice, st));
             PG_TRY(window_candidates(R, E.ctl, ccap, &win));
             accept_kernel<<<(unsigned)pg_cdiv(ccap, 256), 256, 0, st>>>(win.cand, win.cand_r, win.cand64, c + 0, ccap,
-                                                                        (double)thr_eff, win.extra, c + 1, c + 2);
+                                                                        (double)thr_eff, win.extra, c + 1, c + 2,
+                                                                        nullptr);
             definite_sum<<<1, 1024, 0, st>>>(win.dpart, win.nd, c + 3);
             PG_KERNEL_CHECK(ctx);
             PG_HIP(ctx, hipMemcpyAsync(R.hcnt, c, sizeof R.hcnt, hipMemcpyDeviceToHost, st));

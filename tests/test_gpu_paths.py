@@ -63,6 +63,30 @@ def _graph(n, m, seed, hub=0):
     return row, (both[order] % n).astype(np.int32), np.concatenate([w, w])[order]
 
 
+# 8,191 / 8,192: the splitting epilogue, the band-free one; copies of 200 series
+# put 560,000 pairs at one r, more than the candidate list's first size (thr
+# 1.0), and a tenth of all pairs past the segments' first size (thr 0.02)
+@pytest.mark.parametrize("n,copies,thr", [(8191, 0, 0.5), (8192, 0, 0.5), (8193, 0, 1.0), (8449, 0, 0.7),
+                                          (15000, 200, 1.0), (9001, 0, 0.02)])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_r_threshold_forms(ctx, n, copies, thr, weighted):
+    from pagani_amd import synth
+    x = synth.bold(n, copies or n, 24, 7)
+    if copies:
+        assert x.shape == (24, copies)
+        x = np.ascontiguousarray(x[:, np.arange(n) % copies])
+    z64, _ = O.zscore(x)
+    say(f"r threshold n={n} copies={copies} thr={thr} weighted={weighted}")
+    orow, ocol, oval = O.corr_csr_r(z64, thr, weighted)
+    for _ in range(2):
+        info = ctx.corr_build(x, n, 24, thr, weighted=weighted)
+        row, col, val = ctx.corr_csr(n, info.nnz, weighted)
+        np.testing.assert_array_equal(row, orow)
+        np.testing.assert_array_equal(col, ocol)
+        if weighted:
+            np.testing.assert_array_equal(val.view(np.uint32), oval.view(np.uint32))
+
+
 # 65,534 / 65,535 / 65,536: the last 16-bit lists, the first 32-bit ones
 @pytest.mark.parametrize("n,m,hub", [(2, 3, 0), (3, 9, 0), (63, 700, 0), (64, 1500, 20), (257, 12000, 256),
                                      (5000, 60000, 1500), (65534, 150000, 1023), (65535, 150000, 1024),
