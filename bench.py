@@ -160,7 +160,7 @@ def run_metrics(a):
     _, dt = _timed(ctx, lambda: ctx.bc(row, col, None, out=bc))
     te = float(n) * nnz
     out["bc_all_sources"] = {"sources": n, "seconds": dt, "gteps": te / dt / 1e9,
-                             "hbm_model_frac": n * (16.0 * nnz + 40.0 * n) / dt / HBM_PEAK}
+                             "hbm_model_frac": n * (12.0 * nnz + 36.0 * n) / dt / HBM_PEAK}
     log(f"bc all {n} sources: {dt:.2f} s = {te / dt / 1e9:.1f} GTEPS")
     eff = torch.empty(n, dtype=torch.float32, device="cuda")
     ctx.bfs_efficiency(row, col, eff)  # first call sizes the context's buffers
@@ -519,7 +519,7 @@ def main(argv=None) -> int:
         ctx.synchronize()
         bdt = time.perf_counter() - t0
         te = float(a.bc_sources) * nnz
-        bytes_model = a.bc_sources * (16.0 * nnz + 40.0 * n)
+        bytes_model = a.bc_sources * (12.0 * nnz + 36.0 * n)
         out["bc"] = {"sources": a.bc_sources, "seconds": bdt, "gteps": te / bdt / 1e9,
                      "hbm_model_frac": bytes_model / bdt / HBM_PEAK,
                      "all_sources_est_s": bdt * n / a.bc_sources}
