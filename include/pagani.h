@@ -135,13 +135,13 @@ pg_status pg_corr_z64_view(pg_ctx *ctx, const double **z64);
 /* Dense correlation matrix of one or more subjects: subject averaging and the
  * .cormat output (U CorMat.cpp:236-262, 380-620, 775-838; W CorMat.cpp:386-600).
  * The matrix is the packed upper triangle, row-major over i < j, M1 = n(n-1)/2
- * floats, held by the context.  pg_cormat_begin starts it anew (all zero until a subject is added);
- * pg_cormat_add adds
- * one subject's (float) r per pair (r = the FP64 Pearson r, clamped to [-1,1]),
- * or its Fisher z when fisher != 0 (U CorMat.cpp:35-42); every subject has the
- * same n, t may differ.  pg_cormat_finish divides by the subject count and,
- * for Fisher, maps back (U CorMat.cpp:507-517); a single subject without
- * Fisher is its own r matrix.  pg_cormat_read copies values [offset,
+ * floats, held by the context.  pg_cormat_begin starts it anew (all zero until
+ * a subject is added); pg_cormat_add adds one subject's (float) r per pair
+ * (r = the FP64 Pearson r, clamped to [-1,1]), or its Fisher z when
+ * fisher != 0 (U CorMat.cpp:35-42); every subject has the same n, t may
+ * differ.  pg_cormat_finish divides by the subject count and, for Fisher, maps
+ * back (U CorMat.cpp:507-517); a single subject without Fisher is its own r
+ * matrix.  pg_cormat_read copies values [offset,
  * offset+count) out (host or device).  pg_cormat_threshold applies a threshold
  * to the finished matrix as the reference does for averaged networks
  * (FormFullGraph: a > thr, no 1e-6 offset; FormFullGraph_s: the k largest, ties

@@ -278,7 +278,7 @@ __global__ void cm_finish(long long m, float *__restrict__ a, int nsub, int fish
     const long long m4 = m >> 2, stride = (long long)gridDim.x * blockDim.x;
     const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     float4 *a4 = (float4 *)a;
-    for (long long q = t0; q < m4; q += stride) {  // 16-byte accesses, as cm_accumulate
+    for (long long q = t0; q < m4; q += stride) {  // 16-byte accesses
         float4 v = a4[q];
         v.x = v.x / s;
         v.y = v.y / s;
