@@ -148,6 +148,43 @@ def test_segmented_spmv(ctx, n, m, hub, weighted):
     assert abs(lam - olam) <= 1e-9 * abs(olam)
 
 
+def _core_network(n, core, deg, seed):
+    """A clique of `core` vertices in a sparse random network: a leading
+    eigenvalue far from the rest, so that a power iteration ends soon."""
+    rng = np.random.default_rng(seed)
+    m = n * deg // 2
+    k = rng.choice(n, core, replace=False).astype(np.int64)
+    i, j = np.triu_indices(core, 1)
+    a, b = np.concatenate([rng.integers(0, n, m), k[i]]), np.concatenate([rng.integers(0, n, m), k[j]])
+    lo, hi = np.minimum(a, b), np.maximum(a, b)
+    key = np.unique(lo[lo != hi] * np.int64(n) + hi[lo != hi])
+    lo, hi = key // n, key % n
+    w = rng.uniform(0.5, 1.0, key.size).astype(np.float32)
+    both = np.concatenate([key, hi * n + lo])
+    order = np.argsort(both, kind="stable")
+    row = np.zeros(n + 1, np.int32)
+    row[1:] = np.cumsum(np.bincount(both[order] // n, minlength=n))
+    return row, (both[order] % n).astype(np.int32), np.concatenate([w, w])[order]
+
+
+# 1,024 rows per work-group: more of them than 256 CUs hold at once, so that
+# some start while the launch's first one has already found the stop
+@pytest.mark.parametrize("n", [262144, 300003, 600001])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_centrality_in_many_rounds_of_blocks(ctx, n, weighted):
+    row, col, val = _core_network(n, 150, 4, n)
+    v = val if weighted else None
+    say(f"centrality rounds n={n} nnz={col.size} weighted={weighted}")
+    ovh, oav, olam, oit = O.ec(row, col, v)
+    assert oit < 100
+    for _ in range(3):
+        vh, av, lam, it = ctx.eigenvector_centrality(row, col, v)
+        assert it == oit
+        np.testing.assert_allclose(vh, ovh, rtol=1e-9, atol=1e-12)
+        np.testing.assert_allclose(av, oav, rtol=1e-9, atol=1e-12 * max(1.0, abs(olam)))
+        assert abs(lam - olam) <= 1e-9 * abs(olam)
+
+
 @pytest.mark.parametrize("n,m,hub", [(300, 9000, 299), (16385, 60000, 700), (33000, 90000, 2000)])
 @pytest.mark.parametrize("stop", [0, 1])
 @pytest.mark.parametrize("weighted", [False, True])
