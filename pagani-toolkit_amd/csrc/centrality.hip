@@ -69,7 +69,7 @@ __global__ __launch_bounds__(EC_TPB) void ec_init(int n, int R, double *__restri
 // segment's first entries loaded behind its staging), three segments of about
 // 5 us each, bound by the entries' latency from beyond L2 (32 MB of them an
 // iteration), not by the look-ups: leaving out the fillers' changed nothing.
-template <bool W>
+template <bool W, bool GATHER>
 __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, pgdev::SpLayout L, int n, int R, int G, int k,
                                                   const double *__restrict__ uin, double *__restrict__ uout,
                                                   double *__restrict__ vhat, const double *__restrict__ pin,
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, p
     const int im = tid < nr ? i0 + (int)L.perm[i0 + tid] : n - 1;  // slot tid's row
     double ui, t;
     bool empty;
-    const bool go = pgdev::sp_rows<W>(L, i0, nr, uin, n, xs, pt, rowv, [&]() {
+    const bool go = pgdev::sp_product<W, GATHER>(L, i0, nr, uin, n, xs, pt, rowv, [&]() {
         ui = uin[im];
         empty = row[im] == row[im + 1];
         double a[3];
@@ -203,17 +203,26 @@ extern "C" pg_status pg_eigenvector_centrality(pg_ctx *ctx, const int32_t *row, 
     // about one block per CU (its LDS holds a vector segment)
     const int R = (int)std::min<long long>(pgdev::SP_ROWS, std::max<long long>(16, pg_cdiv(n, std::max(ctx->num_cu, 1))));
     const int G = (int)pg_cdiv(n, R);
-    pgdev::SpLayout L;
-    L.nseg = pgdev::sp_nseg(n);
-    L.cap = pgdev::sp_cap(n);
-    L.val = nullptr;
-    const size_t lds = pgdev::sp_lds(L.cap), room = pgdev::sp_room(n, nnz, L.nseg);
-    const void *iter_fn = dval ? (const void *)ec_iter<true> : (const void *)ec_iter<false>;
-    PG_HIP(ctx, hipFuncSetAttribute(iter_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    pgdev::SpLayout L{};
+    const bool gather = pgdev::sp_gathers(n, nnz, G);
     int *parts;
-    PG_TRY(pg_bufT(ctx, "ec.idx", room, &L.idx));
-    if (dval) PG_TRY(pg_bufT(ctx, "ec.val", room, &L.val));
-    PG_TRY(pg_bufT(ctx, "ec.part", 2 * (size_t)n * L.nseg, &parts));
+    if (gather) {
+        PG_TRY(pg_bufT(ctx, "ec.gcol", (size_t)nnz, &L.gcol));
+        if (dval) PG_TRY(pg_bufT(ctx, "ec.val", (size_t)nnz, &L.val));
+        PG_TRY(pg_bufT(ctx, "ec.part", 2 * (size_t)n, &parts));
+    } else {
+        L.nseg = pgdev::sp_nseg(n);
+        L.cap = pgdev::sp_cap(n);
+        const size_t room = pgdev::sp_room(n, nnz, L.nseg);
+        PG_TRY(pg_bufT(ctx, "ec.idx", room, &L.idx));
+        if (dval) PG_TRY(pg_bufT(ctx, "ec.val", room, &L.val));
+        PG_TRY(pg_bufT(ctx, "ec.part", 2 * (size_t)n * L.nseg, &parts));
+    }
+    const size_t lds = gather ? 0 : pgdev::sp_lds(L.cap);
+    const auto iter_fn = gather ? (dval ? ec_iter<true, true> : ec_iter<false, true>)
+                                : (dval ? ec_iter<true, false> : ec_iter<false, false>);
+    if (!gather)
+        PG_HIP(ctx, hipFuncSetAttribute((const void *)iter_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     PG_TRY(pg_bufT(ctx, "ec.perm", (size_t)n, &L.perm));
     L.part = (int2 *)parts;
     pgdev::sp_build<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(drow, dcol, dval, n, nullptr, nullptr, 0, nullptr, nullptr,
@@ -236,12 +245,8 @@ extern "C" pg_status pg_eigenvector_centrality(pg_ctx *ctx, const int32_t *row, 
     EcState h{};
     for (int k0 = 0; k0 <= EC_MAX_ITER; k0 += EC_BATCH) {
         for (int k = k0; k < k0 + EC_BATCH && k <= EC_MAX_ITER; k++)
-            if (dval)
-                ec_iter<true><<<(unsigned)G, EC_TPB, lds, st>>>(drow, L, n, R, G, k, u[k & 1], u[(k + 1) & 1], dvh,
-                                                                part[(k + 1) & 1], part[k & 1], dst);
-            else
-                ec_iter<false><<<(unsigned)G, EC_TPB, lds, st>>>(drow, L, n, R, G, k, u[k & 1], u[(k + 1) & 1], dvh,
-                                                                 part[(k + 1) & 1], part[k & 1], dst);
+            iter_fn<<<(unsigned)G, EC_TPB, lds, st>>>(drow, L, n, R, G, k, u[k & 1], u[(k + 1) & 1], dvh,
+                                                      part[(k + 1) & 1], part[k & 1], dst);
         PG_KERNEL_CHECK(ctx);
         PG_HIP(ctx, hipMemcpyAsync(&h, dst, sizeof h, hipMemcpyDeviceToHost, st));
         PG_HIP(ctx, hipStreamSynchronize(st));

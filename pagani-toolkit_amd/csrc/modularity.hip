@@ -100,7 +100,7 @@ enum { P_YY, P_YK, P_A, P_B, NPART };
 // it the launch and the chain of loads up to the first row (55 us as two
 // launches that gathered the vector from L2 with a wave per row, four per
 // CU).  Every skip below is uniform in a block.
-template <bool W>
+template <bool W, bool GATHER>
 __global__ __launch_bounds__(TPB) void mod_iter(Wave w, int it)
 {
     extern __shared__ double xs[];
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(TPB) void mod_iter(Wave w, int it)
     const bool vec = w.stopmode == PG_MOD_STOP_VECTOR;
     const int i = tid < nr ? i0 + (int)w.lay.perm[i0 + tid] : i0;  // slot tid's node
     double yi, ki, si, ypi, beta, vnp, vn, sum[NPART];
-    const bool go = pgdev::sp_rows<W>(w.lay, i0, nr, y + B.no, B.ng, xs, pt, rowv, [&]() {
+    const bool go = pgdev::sp_product<W, GATHER>(w.lay, i0, nr, y + B.no, B.ng, xs, pt, rowv, [&]() {
         // every load that does not wait for the partials goes out before them
         yi = y[i];
         ki = w.k[i];
@@ -323,13 +323,16 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
     PG_TRY(pg_bufT(ctx, "mod.inside", nn, &d_in));
     PG_TRY(pg_bufT(ctx, "mod.res", nn, &d_res));
     PG_TRY(pg_bufT(ctx, "mod.rloc", nn, &d_rloc));
-    // edges inside the groups of a wave: sized once for the whole network
-    pgdev::SpLayout lay;
+    // edges inside the groups of a wave: sized, and their form chosen, once for
+    // the whole network
+    const int npb0 = (int)std::min<long long>(NPB_MAX, std::max<long long>(16, pg_cdiv(n, std::max(ctx->num_cu, 1))));
+    const bool gather = pgdev::sp_gathers(n, nnz, pg_cdiv(n, npb0));
+    pgdev::SpLayout lay{};
     {
-        const int nseg = pgdev::sp_nseg(n);
-        const size_t room = pgdev::sp_room(n, nnz, nseg);
-        PG_TRY(pg_bufT(ctx, "mod.idx", room, &lay.idx));
-        lay.val = nullptr;
+        const int nseg = gather ? 1 : pgdev::sp_nseg(n);
+        const size_t room = gather ? (size_t)nnz : pgdev::sp_room(n, nnz, nseg);
+        if (gather) PG_TRY(pg_bufT(ctx, "mod.gcol", room, &lay.gcol));
+        else PG_TRY(pg_bufT(ctx, "mod.idx", room, &lay.idx));
         if (dval) PG_TRY(pg_bufT(ctx, "mod.lval", room, &lay.val));
         PG_TRY(pg_bufT(ctx, "mod.part", 2 * nn * nseg, &d_part));
         lay.part = (int2 *)d_part;
@@ -458,8 +461,8 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
         PG_TRY(h2d(d_res, res.data(), (size_t)n * 4));
         PG_TRY(h2d(d_rloc, rloc.data(), (size_t)n * 4));
         // the groups' edges, laid out on the device
-        lay.nseg = pgdev::sp_nseg(gmax);
-        lay.cap = pgdev::sp_cap(gmax);
+        lay.nseg = gather ? 0 : pgdev::sp_nseg(gmax);
+        lay.cap = gather ? 0 : pgdev::sp_cap(gmax);
         pgdev::sp_build<<<(unsigned)pg_cdiv(std::max(nnodes, 1), 4), 256, 0, st>>>(
             drow, dcol, dval, nnodes, d_gid, d_res, lo, d_no, d_rloc, lay, d_sumbg, kmode == PG_MOD_BINARY_K ? 1 : 0);
         pgdev::sp_order<<<(unsigned)nblk, pgdev::SP_TPB, 0, st>>>(drow, (const int *)d_gid, ModBlock{d_blk, npb}, lay.perm);
@@ -501,16 +504,15 @@ extern "C" pg_status pg_modularity_ex(pg_ctx *ctx, const int32_t *row, const int
         std::vector<double> lam_total((size_t)G, 0.0), hbeta((size_t)G, 0.0);
         mod_start<<<(unsigned)nblk, TPB, 0, st>>>(w, 0);
         PG_KERNEL_CHECK(ctx);
-        const size_t lds = pgdev::sp_lds(lay.cap);
-        const void *iter_fn = lay.val ? (const void *)mod_iter<true> : (const void *)mod_iter<false>;
-        PG_HIP(ctx, hipFuncSetAttribute(iter_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        const size_t lds = gather ? 0 : pgdev::sp_lds(lay.cap);
+        const auto iter_fn = gather ? (lay.val ? mod_iter<true, true> : mod_iter<false, true>)
+                                    : (lay.val ? mod_iter<true, false> : mod_iter<false, false>);
+        if (!gather)
+            PG_HIP(ctx, hipFuncSetAttribute((const void *)iter_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         int it = 0, running = G;
         std::vector<double> hlam((size_t)G);
         while (running > 0) {
-            for (int q = 0; q < BATCH; q++) {
-                if (lay.val) mod_iter<true><<<(unsigned)nblk, TPB, lds, st>>>(w, it + q);
-                else mod_iter<false><<<(unsigned)nblk, TPB, lds, st>>>(w, it + q);
-            }
+            for (int q = 0; q < BATCH; q++) iter_fn<<<(unsigned)nblk, TPB, lds, st>>>(w, it + q);
             it += BATCH;
             PG_KERNEL_CHECK(ctx);
             PG_HIP(ctx, hipMemcpyAsync(hstate.data(), d_state, (size_t)G * sizeof(int2), hipMemcpyDeviceToHost, st));

@@ -12,6 +12,11 @@
 // and a row of up to 256 entries has all its loads in flight.  Row i's parts
 // start at group ceil(row[i] / 4) + i * nseg and follow each other: the
 // fillers always fit before row i + 1's, so the layout needs no scan.
+//
+// Staging costs a work-group the whole vector, however few entries its rows
+// have, and the layout a part per row and segment.  A sparse network (sp_gathers)
+// keeps its entries in row order with 32-bit columns and gathers the vector
+// from L2: memory in the entries and rows only, at any length of the vector.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -29,10 +34,11 @@ typedef double sp_d2u __attribute__((ext_vector_type(2), aligned(8)));
 
 struct SpLayout {
     uint16_t *idx;  // groups of 4
+    int *gcol;      // the gathered form's columns: row i's from place row[i] on
     float *val;     // the same places (NULL: every weight is 1)
-    int2 *part;     // [rows][nseg]: first group, groups
+    int2 *part;     // [rows][nseg]: first group, groups; gathered: [rows]: first entry, entries
     uint16_t *perm; // [rows]: a work-group's row of each of its slots, longest rows first
-    int nseg, cap;  // segments of a row's vector; its entries per segment (the zero slot's index)
+    int nseg, cap;  // segments of a row's vector (0: gathered); its entries per segment (the zero slot's index)
 };
 
 inline int sp_nseg(long long n) { return (int)std::max<long long>(1, (n + SP_SEG - 1) / SP_SEG); }
@@ -44,6 +50,19 @@ inline size_t sp_room(long long n, long long nnz, int nseg)
 }
 // dynamic LDS: the segment, the zero slot
 inline size_t sp_lds(int cap) { return ((size_t)cap + 1) * sizeof(double); }
+
+// Gathered form for nnz entries of n rows in `blocks` work-groups: fewer than
+// 3,000 entries per work-group and segment.  Microseconds of a modularity
+// iteration, staged / gathered (random networks, unweighted or weighted), at
+// this many of them: n = 2,000 7.9 / 6.8 at 320, 15.5 / 16.1 at 3,000 (two
+// passes); 16,000 18.2 / 16.6 at 1,260, 9.4 / 9.3 at 3,150, 18.9 / 21.5 at
+// 6,280; 58,000 28.7 / 12.2 at 1,130, 28.6 / 18.7 at 2,830, 57.6 / 58.9 at
+// 5,660, 29.7 / 87.0 at 22,600; 200,000 176 / 32 at 1,200, 192 / 176 at 12,000;
+// 1,000,000 2,800 / 81 at 165.  The staged form's group numbers are 32-bit: it is
+// taken with nnz >= 3,000 n nseg / SP_ROWS at least, hence n * nseg + nnz / 4 <
+// 0.6 nnz < 2^31.
+constexpr long long SP_GATHER = 3000;
+inline bool sp_gathers(long long n, long long nnz, long long blocks) { return nnz < SP_GATHER * blocks * sp_nseg(n); }
 
 // Layout of rows a = 0 .. nrows - 1 by one wave each: row i = gid[a] (a itself
 // when gid is NULL), its entries (i, j) with grp[j] == grp[i] (all when grp is
@@ -61,12 +80,33 @@ static __global__ __launch_bounds__(256) void sp_build(const int *__restrict__ r
     const int i = gid ? gid[a] : a;
     const int r0 = row[i], r1 = row[i + 1];
     const int g = grp ? grp[i] : 0, b0 = grp ? base[g - grp0] : 0;
-    int g0 = (r0 + 3) / 4 + i * L.nseg;
+    int g0 = (int)(((long long)r0 + 3) / 4 + (long long)i * L.nseg);
     double k = 0.0;
+    if (L.nseg == 0) {
+        int have = 0;
+        for (long long e0 = r0; e0 < r1; e0 += 64) {
+            const long long e = e0 + lane;
+            int p = -1;
+            if (e < r1) {
+                const int j = col[e];
+                if (!grp || grp[j] == g) p = grp ? loc[j] - b0 : j;
+            }
+            const unsigned long long m = __ballot(p >= 0);
+            if (p >= 0) {
+                const int at = r0 + have + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+                const float w = val ? val[e] : 1.0f;
+                L.gcol[at] = p;
+                if (L.val) L.val[at] = w;
+                k += count ? 1.0 : (double)w;
+            }
+            have += __popcll(m);
+        }
+        if (lane == 0) L.part[a] = make_int2(r0, have);
+    }
     for (int s = 0; s < L.nseg; s++) {
         int have = 0;
-        for (int e0 = r0; e0 < r1; e0 += 64) {
-            const int e = e0 + lane;
+        for (long long e0 = r0; e0 < r1; e0 += 64) {
+            const long long e = e0 + lane;
             int p = -1;
             if (e < r1) {
                 const int j = col[e];
@@ -256,6 +296,79 @@ __device__ __forceinline__ bool sp_rows(const SpLayout &L, int a0, int nr, const
     }
     __syncthreads();
     return true;
+}
+
+// Four entries of row part p (first entry, entries) per lane, from its entry k on.
+template <bool W>
+struct SpGather {
+    int c[4];
+    float w[4];
+    __device__ __forceinline__ void load(const SpLayout &L, int2 p, int k)
+    {
+        const long long e = (long long)p.x + k;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const bool in = k + 16 * u < p.y;
+            c[u] = in ? L.gcol[e + 16 * u] : -1;
+            if (W) w[u] = in ? L.val[e + 16 * u] : 0.0f;
+        }
+    }
+    __device__ __forceinline__ double dot(const double *__restrict__ x, double acc) const
+    {
+        double v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = c[u] >= 0 ? x[c[u]] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) acc = W ? fma(v[u], (double)w[u], acc) : acc + v[u];
+        return acc;
+    }
+};
+
+// sp_rows of the gathered form: x is read where it lies.  The entries of the
+// next 64 slots are loaded under the look-ups of these.
+template <bool W, class F>
+__device__ __forceinline__ bool sp_rows_gather(const SpLayout &L, int a0, int nr, const double *__restrict__ x,
+                                               int2 *__restrict__ pt, double *__restrict__ rowv, F &&between)
+{
+    const int tid = threadIdx.x, l = tid & 15, q = tid >> 4;
+    int2 pn = make_int2(0, 0), p = make_int2(0, 0);
+    if (tid < nr) pn = L.part[a0 + (int)L.perm[a0 + tid]];
+    if (q < nr) p = L.part[a0 + (int)L.perm[a0 + q]];
+    if (!between()) return false;
+    SpGather<W> b, c;
+    b.load(L, p, l);
+    if (tid < nr) pt[tid] = pn;
+    __syncthreads();
+    constexpr int Q = SP_TPB / 16;
+    int r = q;  // this pass's slot, and the next's
+    for (int k0 = 0; k0 < nr; k0 += Q) {
+        const int rn = k0 + Q + ((k0 / Q) & 1 ? q : Q - 1 - q);
+        double acc = 0.0;
+        for (int k = 64; k < p.y; k += 64) {  // more of this row to come
+            c.load(L, p, k + l);
+            acc = b.dot(x, acc);
+            b = c;
+        }
+        p = rn < nr ? pt[rn] : make_int2(0, 0);
+        c.load(L, p, l);
+        acc = b.dot(x, acc);
+        b = c;
+        acc = sp_sum16(acc);
+        if (l == 0 && r < nr) rowv[r] = acc;
+        r = rn;
+    }
+    __syncthreads();
+    return true;
+}
+
+// Either form.
+template <bool W, bool GATHER, class F>
+__device__ __forceinline__ bool sp_product(const SpLayout &L, int a0, int nr, const double *__restrict__ x, int len,
+                                           double *__restrict__ xs, int2 *__restrict__ pt, double *__restrict__ rowv,
+                                           F &&between)
+{
+    if constexpr (GATHER) return sp_rows_gather<W>(L, a0, nr, x, pt, rowv, between);
+    else return sp_rows<W>(L, a0, nr, x, len, xs, pt, rowv, between);
 }
 
 // Q sums over the first nr threads of the work-group in a fixed order, written

@@ -129,8 +129,8 @@ def test_clustering_zero_and_negative_weights(ctx):
         np.testing.assert_allclose(c[ok], oc[ok], rtol=1e-12, atol=0)
 
 
-# one, two and three 16,384-entry vector segments with rows that end inside a
-# group; a hub row longer than a batch of 256 entries
+# sparse networks, whose vector is gathered: rows that end inside a batch of 64
+# entries, a hub row of several
 @pytest.mark.parametrize("n,m,hub", [(5, 7, 0), (300, 9000, 299), (16384, 60000, 700), (16385, 60000, 700),
                                      (33000, 90000, 2000)])
 @pytest.mark.parametrize("weighted", [False, True])
@@ -183,6 +183,54 @@ def test_centrality_in_many_rounds_of_blocks(ctx, n, weighted):
         np.testing.assert_allclose(vh, ovh, rtol=1e-9, atol=1e-12)
         np.testing.assert_allclose(av, oav, rtol=1e-9, atol=1e-12 * max(1.0, abs(olam)))
         assert abs(lam - olam) <= 1e-9 * abs(olam)
+
+
+# one (short and full), two and three staged 16,384-entry vector segments with
+# rows that end inside a group; a hub row longer than a batch of 256 entries
+STAGED = [(700, 120000, 600), (16384, 900000, 700), (16385, 1700000, 700), (33000, 2600000, 2000)]
+
+
+@pytest.mark.parametrize("n,m,hub", STAGED)
+@pytest.mark.parametrize("weighted", [False, True])
+def test_staged_spmv(ctx, n, m, hub, weighted):
+    row, col, val = _graph(n, m, 3 * n + m, hub)
+    v = val if weighted else None
+    say(f"staged spmv n={n} nnz={col.size} weighted={weighted}")
+    # 3,000 entries per work-group and segment: the gathered form's limit
+    assert col.size >= 3000 * -(-n // max(16, -(-n // 256))) * -(-n // 16384)
+    vh, av, lam, it = ctx.eigenvector_centrality(row, col, v)
+    ovh, oav, olam, oit = O.ec(row, col, v)
+    assert it == oit
+    np.testing.assert_allclose(vh, ovh, rtol=1e-9, atol=1e-12)
+    np.testing.assert_allclose(av, oav, rtol=1e-9, atol=1e-12 * max(1.0, abs(olam)))
+    assert abs(lam - olam) <= 1e-9 * abs(olam)
+    for cap in (2, 40):  # vector stop at the cap: no division of noise by a gap
+        got = ctx.modularity(row, col, v, 0, stop=0, max_iter=cap, max_depth=1)
+        want = O.modularity(row, col, v, 0, stop=0, max_iter=cap, max_depth=1)
+        assert abs(got[2] - want[2]) <= 1e-9 * max(1.0, abs(want[2]))
+        np.testing.assert_allclose(got[3], want[3], rtol=1e-7, atol=1e-9)
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_power_iterations_on_millions_of_vertices(ctx, weighted):
+    """Rows times vector segments beyond 2^31: the layout of a sparse network
+    grows with its entries and rows only."""
+    n = 6_000_000
+    row, col, val = _core_network(n, 300, 2, 17)
+    v = val if weighted else None
+    say(f"power iterations n={n} nnz={col.size} weighted={weighted}")
+    vh, av, lam, it = ctx.eigenvector_centrality(row, col, v)
+    ovh, oav, olam, oit = O.ec(row, col, v)
+    assert it == oit
+    np.testing.assert_allclose(vh, ovh, rtol=1e-9, atol=1e-12)
+    np.testing.assert_allclose(av, oav, rtol=1e-9, atol=1e-12 * max(1.0, abs(olam)))
+    assert abs(lam - olam) <= 1e-9 * abs(olam)
+    got = ctx.modularity(row, col, v, 0, stop=1, max_iter=64, max_depth=1)
+    want = O.modularity(row, col, v, 0, stop=1, max_iter=64, max_depth=1)
+    assert abs(got[2] - want[2]) <= 1e-9 * max(1.0, abs(want[2]))
+    np.testing.assert_allclose(got[3], want[3], rtol=1e-7, atol=1e-9)
+    clear = np.abs(want[3]) > 2e-9  # a vertex's side is its entry's sign
+    np.testing.assert_array_equal(got[0][clear], want[0][clear])
 
 
 @pytest.mark.parametrize("n,m,hub", [(300, 9000, 299), (16385, 60000, 700), (33000, 90000, 2000)])
