@@ -42,7 +42,7 @@ struct EcBlock {
 };
 
 struct EcState {
-    int stopped, iters;
+    int stopped, iters;  // stopped: 1 + the launch that found the stop, 0 before
     double lam, err1, err2;
 };
 
@@ -79,7 +79,11 @@ __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, p
     __shared__ double rowv[pgdev::SP_ROWS];
     __shared__ int2 pt[pgdev::SP_ROWS];
     __shared__ double red[EC_TPB / 64 * 3], tot[3];
-    __shared__ int skip;
+    // only a stop of an earlier launch counts: block 0 of this one may set it
+    // while other blocks start, and the waves of a block have to agree (all
+    // reach that same decision from the partials)
+    const int stop = st->stopped;
+    if (stop > 0 && stop <= k) return;
     const int tid = threadIdx.x;
     const int i0 = blockIdx.x * R, nr = min(n - i0, R);
     const int im = tid < nr ? i0 + (int)L.perm[i0 + tid] : n - 1;  // slot tid's row
@@ -89,12 +93,7 @@ __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, p
         ui = uin[im];
         empty = row[im] == row[im + 1];
         double a[3];
-        // the stop flag may be set by this launch's first block while this one
-        // starts, so one thread reads it for the whole block; a block that
-        // reads 0 reaches the same decision from the partials
-        if (tid == 0) skip = st->stopped;
-        pgdev::sp_partials<3>(pin, 0, G, a, tot);  // its barrier publishes skip
-        if (skip) return false;
+        pgdev::sp_partials<3>(pin, 0, G, a, tot);
         if (k > 0) {
             const double e1 = sqrt(a[0]), e2 = sqrt(a[1]);
             if (!(e1 > EC_EPS && e2 > EC_EPS) || k >= EC_MAX_ITER) {
@@ -102,7 +101,7 @@ __global__ __launch_bounds__(EC_TPB) void ec_iter(const int *__restrict__ row, p
                     st->err1 = e1;
                     st->err2 = e2;
                     st->iters = k;
-                    st->stopped = 1;
+                    st->stopped = k + 1;
                 }
                 return false;
             }
