@@ -4987,10 +4987,12 @@ extern "C" pg_status pg_corr_csr(pg_ctx *ctx, int32_t *row, int32_t *col, float 
 {
     if (!ctx) return PG_EINVAL;
     if (ctx->cnnz < 0) return pg_fail(ctx, PG_ESTATE, "no CSR built yet");
+    PG_HIP(ctx, hipSetDevice(ctx->device));
     const long long nrow = (long long)ctx->cn + 1, nnz = ctx->cnnz;
     const bool want_val = val && ctx->cweighted;
-    if (row && col && (!want_val || pg_is_device_ptr(val)) && pg_is_device_ptr(row) && pg_is_device_ptr(col)) {
-        // to device memory: the arrays in one launch
+    if (pg_is_local_ptr(ctx, row) && pg_is_local_ptr(ctx, col) && (!want_val || pg_is_local_ptr(ctx, val))) {
+        // to this device's memory: the arrays in one launch (other GPUs' and
+        // managed memory by the runtime's copies)
         const long long most = std::max(nrow, nnz);
         csr_copy<<<(unsigned)std::min<long long>(pg_cdiv(most, 1024), 8LL * std::max(ctx->num_cu, 1)), 256, 0, ctx->stream>>>(
             ctx->c_row, nrow, ctx->c_col, want_val ? (const int *)ctx->c_val : nullptr, nnz, row, col, (int *)val);

@@ -99,6 +99,8 @@ inline pg_status pg_bufT(pg_ctx *ctx, const char *name, size_t count, T **out)
 }
 
 bool pg_is_device_ptr(const void *p);
+// Memory of the context's own device (not managed, not another GPU's).
+bool pg_is_local_ptr(const pg_ctx *ctx, const void *p);
 
 // Device view of an input: device pointers pass through, host pointers are
 // copied into the named buffer.

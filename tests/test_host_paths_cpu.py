@@ -1,0 +1,69 @@
+"""Host code of libpagani on a stub HIP runtime (hip_stub.cpp): which device is
+current at a launch, what happens when an allocation fails.  Kernels do not
+run, so a network has no edges here; no GPU is needed."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+PRELUDE = """
+import ctypes as C, os, sys
+stub = C.CDLL({stub!r}, mode=os.RTLD_GLOBAL)
+sys.modules["torch"] = None  # its HIP runtime is not wanted
+sys.path.insert(0, {pkg!r})
+import numpy as np
+import pagani_amd
+from pagani_amd import lib as L
+stub.stub_alloc.restype = C.c_void_p
+stub.stub_alloc.argtypes = [C.c_size_t, C.c_int, C.c_int]
+HOOK = C.CFUNCTYPE(None, C.c_char_p, C.c_int, C.c_int, C.POINTER(C.c_void_p))
+launches, check = [], lambda name, args: None
+@HOOK
+def hook(name, current, device, args):
+    launches.append((name.decode(), current, device))
+    check(name.decode(), args)
+stub.stub_hook(hook)
+def misplaced():
+    return [x for x in launches if x[1] != x[2]]
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("hip") / "libhipstub.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_stub.cpp"), "-o", out], check=True)
+    return out
+
+
+def run(stub, code):
+    src = PRELUDE.format(stub=stub, pkg=os.path.join(ROOT, "pagani-toolkit_amd")) + textwrap.dedent(code)
+    r = subprocess.run([sys.executable, "-c", src], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr + r.stdout
+
+
+def test_corr_csr_on_its_own_device(stub):
+    """pg_corr_csr of a context on device 1 while device 0 is current: its
+    kernel runs on device 1, and only for arrays that lie there; other devices'
+    and managed memory are copied to by the runtime."""
+    run(stub, """
+    ctx = pagani_amd.Context(1)
+    n = 40
+    ctx.corr_build(np.zeros((20, n), np.float32), n, 20, 0.3, weighted=True)
+    assert launches and not misplaced()
+    def take(device, managed):
+        stub.hipSetDevice(0)
+        launches.clear()
+        before = stub.stub_copies()
+        row, col, val = (C.c_void_p(stub.stub_alloc(4 * (n + 1), device, managed)) for _ in range(3))
+        ctx._check(ctx._lib.pg_corr_csr(ctx._h, row, col, val))
+        return len(launches), stub.stub_copies() - before
+    assert take(1, 0) == (1, 0) and not misplaced()
+    assert take(0, 0)[0] == 0 and take(0, 0)[1] >= 1
+    assert take(1, 1)[0] == 0 and take(1, 1)[1] >= 1
+    """)
