@@ -1087,23 +1087,36 @@ extern "C" pg_status pg_cp_binary_static(pg_ctx *ctx, const int32_t *row, const 
 }
 
 namespace {
-// LDS: the factors of up to 1,024 neighbours (8 KB: seven work-groups share a
-// CU at n = 30,000; longer rows read theirs from memory), bitmap, prefixes.
+// LDS of cpw_lists: bitmap, prefixes, and the factors of up to CPW_CAP neighbours
+// (longer rows read theirs from memory) as far as they leave a CU as many
+// work-groups as the bitmap and prefixes alone would: its eight up to n = 38,000,
+// two at n = 300,000 (with 480 factors; degree 10: 5.5 ms, 10.5 with one), one
+// at the largest n, whose bitmap leaves room for 127.
 constexpr int CPW_CAP = 1024;
+constexpr size_t CPW_STATIC = 256 * 8 + 256 * 4;  // the kernel's own arrays
+constexpr size_t LDS_GRAIN = 1280;                // LDS is given out in 320 words
+inline int cpw_cap(size_t lds, size_t bitmap)
+{
+    const size_t base = bitmap + CPW_STATIC;
+    const size_t share = lds / std::min<size_t>(8, lds / base) / LDS_GRAIN * LDS_GRAIN;
+    return share > base ? (int)std::min<size_t>(CPW_CAP, (share - base) / 8) : 0;
+}
 template <class CT>
 pg_status launch_cpw(pg_ctx *ctx, const int *row, const int *col, const float *val, const double *fac, int n, int kind,
                      void *up, int4 *meta, double *cp)
 {
     hipStream_t st = ctx->stream;
-    const size_t lds = CPW_CAP * 8 + ((size_t)n / 32 + 1) * (4 + sizeof(CT));
+    const size_t bitmap = ((size_t)n / 32 + 1) * (4 + sizeof(CT));
+    const int cap = cpw_cap(ctx->lds_per_block, bitmap);
+    const size_t lds = (size_t)cap * 8 + bitmap;
     const void *fn = kind == PG_CP_BARRAT ? (const void *)cpw_lists<CT, PG_CP_BARRAT>
                                           : (const void *)cpw_lists<CT, PG_CP_ONNELA>;
     PG_HIP(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     upper_lists<CT><<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(row, col, val, n, (CT *)up, meta, nullptr);
     if (kind == PG_CP_BARRAT)
-        cpw_lists<CT, PG_CP_BARRAT><<<(unsigned)n, 256, lds, st>>>(row, col, val, fac, (const CT *)up, meta, n, CPW_CAP, cp);
+        cpw_lists<CT, PG_CP_BARRAT><<<(unsigned)n, 256, lds, st>>>(row, col, val, fac, (const CT *)up, meta, n, cap, cp);
     else
-        cpw_lists<CT, PG_CP_ONNELA><<<(unsigned)n, 256, lds, st>>>(row, col, val, fac, (const CT *)up, meta, n, CPW_CAP, cp);
+        cpw_lists<CT, PG_CP_ONNELA><<<(unsigned)n, 256, lds, st>>>(row, col, val, fac, (const CT *)up, meta, n, cap, cp);
     PG_KERNEL_CHECK(ctx);
     return PG_OK;
 }

@@ -110,6 +110,20 @@ def test_clustering_lists(ctx, n, m, hub):
             assert abs(mw - omw) <= 1e-12 * max(abs(omw), 1e-300)
 
 
+# two work-groups a CU, one, and the largest n whose bitmap and prefixes fit
+# (127 factors beside them): hubs below and above the factors held in LDS
+@pytest.mark.parametrize("n", [300000, 610304, 638976])
+@pytest.mark.parametrize("hub", [100, 3000])
+def test_weighted_clustering_of_large_networks(ctx, n, hub):
+    row, col, val = _graph(n, 2 * n, n + hub, hub)
+    for kind in (1, 2):
+        say(f"weighted clustering n={n} hub={hub} kind={kind}")
+        c, mean = ctx.cp_weighted(row, col, val, kind, 0)
+        oc, omean = O.cp_weighted(row, col, val, kind, 0)
+        np.testing.assert_allclose(c, oc, rtol=1e-12, atol=0)
+        assert abs(mean - omean) <= 1e-12 * max(abs(omean), 1e-300)
+
+
 def test_clustering_zero_and_negative_weights(ctx):
     """Zero weights close no triangle; a negative product has no real root."""
     row, col, val = _graph(300, 9000, 5)
