@@ -179,12 +179,16 @@ inline bool upper16(int n) { return n < 65535; }
 
 // One wave per row v: meta[v] = (first group, groups, first entry above the
 // diagonal).  With val, an entry of weight 0 becomes the filler column (it
-// closes no triangle but keeps its place).  skip: nothing is read or written
-// when *skip is set (a captured subject whose CSR was not built).
+// closes no triangle but keeps its place), and f gets the FP64 factor of every
+// entry of the row: Onnela's cube root of w / wmax (a triangle's (w1 w2 w3 /
+// wmax^3)^(1/3) is the product of three of them: one root per entry in place
+// of a power per triangle), Barrat's w itself (wmaxp NULL).  skip: nothing is
+// read or written when *skip is set (a captured subject whose CSR was not built).
 template <class CT>
 __global__ __launch_bounds__(256) void upper_lists(const int *__restrict__ row, const int *__restrict__ col,
                                                    const float *__restrict__ val, int n, CT *__restrict__ up,
-                                                   int4 *__restrict__ meta, const unsigned *__restrict__ skip)
+                                                   int4 *__restrict__ meta, const unsigned *__restrict__ skip,
+                                                   const float *__restrict__ wmaxp, double *__restrict__ f)
 {
     if (skip && *skip) return;
     const int v = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -206,6 +210,12 @@ __global__ __launch_bounds__(256) void upper_lists(const int *__restrict__ row, 
         up[4ll * g0 + k] = (CT)(in ? col[e] : n);
     }
     if (lane == 0) meta[v] = make_int4(g0, ng, s, 0);
+    if (!f) return;
+    const double wmax = wmaxp ? (double)*wmaxp : 1.0;
+    for (int e = a + lane; e < b; e += 64) {
+        const double w = (double)val[e];
+        f[e] = wmaxp ? cbrt(w / wmax) : w;
+    }
 }
 
 // One block per vertex u: T_u = #{(v, w) : v < w, v, w in N(u), (v, w) in E},
@@ -346,18 +356,6 @@ __global__ __launch_bounds__(256) void max_kernel(const float *__restrict__ x, l
         __syncthreads();
     }
     if (threadIdx.x == 0) out[blockIdx.x] = red[0];
-}
-
-// The FP64 factor of every entry: Onnela's cube root of w / wmax (a triangle's
-// (w1 w2 w3 / wmax^3)^(1/3) is the product of three of them: one root per
-// entry in place of a power per triangle), Barrat's w itself.
-__global__ __launch_bounds__(256) void cpw_factors(const float *__restrict__ val, long long nnz, int kind,
-                                                   const float *__restrict__ wmaxp, double *__restrict__ f)
-{
-    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= nnz) return;
-    const double w = (double)val[e];
-    f[e] = kind == PG_CP_BARRAT ? w : cbrt(w / (double)*wmaxp);
 }
 
 // Weighted clustering of vertex u (one block) over the packed upper lists:
@@ -854,7 +852,8 @@ template <class CT>
 void launch_triangles(hipStream_t st, const int *row, const int *col, int n, void *up, int4 *meta, long long *tri,
                       float *cp, const unsigned *skip = nullptr)
 {
-    upper_lists<CT><<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(row, col, nullptr, n, (CT *)up, meta, skip);
+    upper_lists<CT><<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(row, col, nullptr, n, (CT *)up, meta, skip, nullptr,
+                                                        nullptr);
     triangles_lists<CT><<<(unsigned)n, 256, ((size_t)n / 32 + 1) * 4, st>>>(row, col, (const CT *)up, meta, n, tri, cp,
                                                                             skip);
 }
@@ -1089,9 +1088,9 @@ extern "C" pg_status pg_cp_binary_static(pg_ctx *ctx, const int32_t *row, const 
 namespace {
 // LDS of cpw_lists: bitmap, prefixes, and the factors of up to CPW_CAP neighbours
 // (longer rows read theirs from memory) as far as they leave a CU as many
-// work-groups as the bitmap and prefixes alone would: its eight up to n = 38,000,
-// two at n = 300,000 (with 480 factors; degree 10: 5.5 ms, 10.5 with one), one
-// at the largest n, whose bitmap leaves room for 127.
+// work-groups as the bitmap and prefixes alone would: eight up to n = 69,632 (all
+// factors up to 49,000), two at n = 300,000 (with 480 factors; degree 10: 5.5 ms,
+// 10.5 with one), one at the largest n, whose bitmap leaves room for 127.
 constexpr int CPW_CAP = 1024;
 constexpr size_t CPW_STATIC = 256 * 8 + 256 * 4;  // the kernel's own arrays
 constexpr size_t LDS_GRAIN = 1280;                // LDS is given out in 320 words
@@ -1102,8 +1101,8 @@ inline int cpw_cap(size_t lds, size_t bitmap)
     return share > base ? (int)std::min<size_t>(CPW_CAP, (share - base) / 8) : 0;
 }
 template <class CT>
-pg_status launch_cpw(pg_ctx *ctx, const int *row, const int *col, const float *val, const double *fac, int n, int kind,
-                     void *up, int4 *meta, double *cp)
+pg_status launch_cpw(pg_ctx *ctx, const int *row, const int *col, const float *val, const float *wmax, double *fac,
+                     int n, int kind, void *up, int4 *meta, double *cp)
 {
     hipStream_t st = ctx->stream;
     const size_t bitmap = ((size_t)n / 32 + 1) * (4 + sizeof(CT));
@@ -1111,8 +1110,8 @@ pg_status launch_cpw(pg_ctx *ctx, const int *row, const int *col, const float *v
     const size_t lds = (size_t)cap * 8 + bitmap;
     const void *fn = kind == PG_CP_BARRAT ? (const void *)cpw_lists<CT, PG_CP_BARRAT>
                                           : (const void *)cpw_lists<CT, PG_CP_ONNELA>;
-    PG_HIP(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    upper_lists<CT><<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(row, col, val, n, (CT *)up, meta, nullptr);
+    if (lds > 48 * 1024) PG_HIP(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    upper_lists<CT><<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(row, col, val, n, (CT *)up, meta, nullptr, wmax, fac);
     if (kind == PG_CP_BARRAT)
         cpw_lists<CT, PG_CP_BARRAT><<<(unsigned)n, 256, lds, st>>>(row, col, val, fac, (const CT *)up, meta, n, cap, cp);
     else
@@ -1146,14 +1145,17 @@ extern "C" pg_status pg_cp_weighted(pg_ctx *ctx, const int32_t *row, const int32
     PG_TRY(pg_bufT(ctx, "cp.meta", (size_t)n, &meta));
     PG_TRY(pg_out(ctx, cp, (size_t)n, "out.cpw", &dcp));
     hipStream_t st = ctx->stream;
-    long long lim = wmax_mode == 1 ? std::min<long long>(n, nnz) : nnz;
-    const int gm = (int)std::max<long long>(1, std::min<long long>(MAX_WG, pg_cdiv(lim, 1024)));
-    max_kernel<<<gm, 256, 0, st>>>(dval, lim, dwmax + 1);
-    max_kernel<<<1, 256, 0, st>>>(dwmax + 1, gm, dwmax);
-    if (nnz > 0) cpw_factors<<<(unsigned)pg_cdiv(nnz, 256), 256, 0, st>>>(dval, nnz, kind, dwmax, fac);
+    if (kind == PG_CP_BARRAT) {
+        dwmax = nullptr;
+    } else {
+        long long lim = wmax_mode == 1 ? std::min<long long>(n, nnz) : nnz;
+        const int gm = (int)std::max<long long>(1, std::min<long long>(MAX_WG, pg_cdiv(lim, 8192)));
+        max_kernel<<<gm, 256, 0, st>>>(dval, lim, gm > 1 ? dwmax + 1 : dwmax);
+        if (gm > 1) max_kernel<<<1, 256, 0, st>>>(dwmax + 1, gm, dwmax);
+    }
     if (n > 0) {
-        if (upper16(n)) PG_TRY(launch_cpw<uint16_t>(ctx, drow, dcol, dval, fac, n, kind, up, meta, dcp));
-        else PG_TRY(launch_cpw<uint32_t>(ctx, drow, dcol, dval, fac, n, kind, up, meta, dcp));
+        if (upper16(n)) PG_TRY(launch_cpw<uint16_t>(ctx, drow, dcol, dval, dwmax, fac, n, kind, up, meta, dcp));
+        else PG_TRY(launch_cpw<uint32_t>(ctx, drow, dcol, dval, dwmax, fac, n, kind, up, meta, dcp));
     }
     mean_kernel<double><<<1, MEAN_TPB, 0, st>>>(dcp, n, dmean);
     PG_KERNEL_CHECK(ctx);

@@ -67,3 +67,18 @@ def test_corr_csr_on_its_own_device(stub):
     assert take(0, 0)[0] == 0 and take(0, 0)[1] >= 1
     assert take(1, 1)[0] == 0 and take(1, 1)[1] >= 1
     """)
+
+
+def test_weighted_clustering_launches(stub):
+    """A region-level call is its launches: the check, (Onnela) the maximum, the
+    lists with the factors, the clustering, the mean."""
+    run(stub, """
+    n = 116
+    row, col, val = np.zeros(n + 1, np.int32), np.zeros(200, np.int32), np.ones(200, np.float32)
+    row[1:] = 200
+    ctx = pagani_amd.Context(0)
+    for kind, count in ((1, 4), (2, 5)):
+        launches.clear()
+        ctx.cp_weighted(row, col, val, kind)
+        assert len(launches) == count, launches
+    """)
