@@ -203,7 +203,7 @@ __global__ __launch_bounds__(256) void upper_lists(const int *__restrict__ row, 
         }
     }
     s = min(s, b);
-    const int g0 = (a + 3) / 4 + v, ng = (b - s + 3) / 4;
+    const int g0 = (int)(((unsigned)a + 3u) / 4) + v, ng = (b - s + 3) / 4;
     for (int k = lane; k < 4 * ng; k += 64) {
         const int e = s + k;
         const bool in = e < b && !(val && val[e] == 0.0f);
