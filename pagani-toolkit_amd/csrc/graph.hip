@@ -910,23 +910,18 @@ extern "C" pg_status pg_cp_binary(pg_ctx *ctx, const int32_t *row, const int32_t
     // at before they index with the CSR, and the mean's launch reports both
     float *dcp;
     int *bad;
-    const bool fresh = ctx->bufs.find("cp.bad") == ctx->bufs.end();
     PG_TRY(pg_bufT(ctx, "cp.bad", 1, &bad));
     PG_TRY(pg_out(ctx, cp, (size_t)n, "out.cp", &dcp));
     hipStream_t st = ctx->stream;
-    if (fresh) PG_HIP(ctx, hipMemsetAsync(bad, 0, 4, st));
+    if (!ctx->cp_bad_clear) PG_HIP(ctx, hipMemsetAsync(bad, 0, 4, st));
+    ctx->cp_bad_clear = false;  // until the mean's launch has left it so
     pg_validate_launch(ctx, drow, dcol, n, nnz, true, bad);
-    if (n > 0) {
-        const pg_status rs = run_triangles(ctx, drow, dcol, n, nnz, nullptr, dcp, (const unsigned *)bad);
-        if (rs != PG_OK) {
-            (void)hipMemsetAsync(bad, 0, 4, st);  // as the mean's launch would have left it
-            return rs;
-        }
-    }
+    if (n > 0) PG_TRY(run_triangles(ctx, drow, dcol, n, nnz, nullptr, dcp, (const unsigned *)bad));
     PgCheck *chk = pg_check(ctx);
     mean_kernel<float><<<1, MEAN_TPB, 0, st>>>(dcp, n, nullptr, chk, bad);
     PG_KERNEL_CHECK(ctx);
     PG_HIP(ctx, hipStreamSynchronize(st));
+    ctx->cp_bad_clear = true;
     if (*(volatile int *)&chk->bad) return pg_malformed(ctx, true);
     const double m = *(volatile double *)&chk->mean;
     PG_TRY(pg_out_finish(ctx, cp, dcp, (size_t)n));

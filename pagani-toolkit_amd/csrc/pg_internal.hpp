@@ -37,6 +37,7 @@ struct pg_ctx {
     bool tuning = false;             // inside a search: no nested search
     std::string arch;                // gcnArchName without features, read once
     void *h_report = nullptr;        // pinned host buffer for small result read-backs
+    bool cp_bad_clear = false;       // the "cp.bad" word is 0 (a pg_cp_binary call ran to its end)
     // the Gram supertile list last copied to the "corr.stl" buffer and its key
     // (row tiles, column tiles, tile aspect, supertile edge, length)
     void *stl_dev = nullptr;

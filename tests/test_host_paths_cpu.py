@@ -82,3 +82,30 @@ def test_weighted_clustering_launches(stub):
         ctx.cp_weighted(row, col, val, kind)
         assert len(launches) == count, launches
     """)
+
+
+def test_clustering_flag_after_a_failed_allocation(stub):
+    """Each allocation of a context's first pg_cp_binary fails once: the next
+    call finds its malformed-CSR flag clear."""
+    run(stub, """
+    n = 40
+    row, col = np.zeros(n + 1, np.int32), np.zeros(0, np.int32)
+    flags = []
+    def check(name, args):
+        if "csr_validate" in name:
+            flags.append(C.cast(args[5], C.POINTER(C.POINTER(C.c_int)))[0][0])
+    failed = 0
+    for nth in range(1, 12):
+        ctx = pagani_amd.Context(0)
+        stub.stub_fail_malloc(nth)
+        try:
+            ctx.cp_binary(row, col)
+        except pagani_amd.PgError as e:
+            assert e.status == 2, e
+            failed += 1
+        stub.stub_fail_malloc(0)
+        flags.clear()
+        ctx.cp_binary(row, col)
+        assert flags == [0], (nth, flags)
+    assert failed >= 4
+    """)
