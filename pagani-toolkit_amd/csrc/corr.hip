@@ -1909,28 +1909,16 @@ __global__ __launch_bounds__(256) void edge_values(EdgeSrc s, const double *__re
     }
 }
 
-// The same with a thread per entry, for series beyond PairSum's 32-bit offsets.
-__global__ __launch_bounds__(256) void edge_values_wide(EdgeSrc s, const double *__restrict__ z, int t)
-{
-    const int g = blockIdx.y;
-    const long long c = src_count(s, g);
-    const float ka = src_bound(s);
-    for (long long k = (long long)blockIdx.x * 256 + threadIdx.x; k < c; k += (long long)gridDim.x * 256) {
-        if (s.seg_r && g < s.nseg && s.seg_r[(long long)g * s.seg_cap + k] <= ka) continue;
-        const int2 e = src_edge(s, g, k);
-        float *out = g < s.nseg ? s.seg_w + (long long)g * s.w_cap : s.extra_w;
-        out[k] = (float)r64_pair(z, t, e.x, e.y);
-    }
-}
-
 // Entries beyond `cap` (a selection that did not hold; the caller checks
 // row[n] and rebuilds) are dropped rather than written.
-// W: the weight of every entry goes along (weighted CSR).
-template <bool W>
+// W: the weight of every entry goes along (weighted CSR), from beside the lists
+// or, with no memory for those (launch_csr), summed here by the entry's thread.
+enum { W_NONE, W_LISTED, W_SUMMED };
+template <int W>
 __global__ __launch_bounds__(SEG_THREADS) void bucket_scatter(EdgeSrc s, int nbk, const long long *__restrict__ off,
                                                               const long long *__restrict__ bstart,
                                                               unsigned *__restrict__ ent, float *__restrict__ entv,
-                                                              long long cap)
+                                                              const double *__restrict__ z, int t, long long cap)
 {
     // per-bucket: this segment's output base (bstart + off; below cap, which
     // is at most INT32_MAX, whenever anything is written) and a cursor
@@ -1945,7 +1933,7 @@ __global__ __launch_bounds__(SEG_THREADS) void bucket_scatter(EdgeSrc s, int nbk
     const long long c = src_count(s, g);
     const float ka = src_bound(s);
     if (bstart[nbk] > cap) return;
-    seg_batches<W>(s, g, c, [&](const SegBatch<W> &a) {
+    seg_batches<W == W_LISTED>(s, g, c, [&](const SegBatch<W == W_LISTED> &a) {
 #pragma unroll
         for (int u = 0; u < SEG_UNROLL; u++) {
             if (!a.keep(u, ka)) continue;
@@ -1955,9 +1943,10 @@ __global__ __launch_bounds__(SEG_THREADS) void bucket_scatter(EdgeSrc s, int nbk
             const unsigned pr = sbase[br] + atomicAdd(&sc[br], 1u);
             ent[pf] = ((unsigned)(e.x & (BROWS - 1)) << 25) | (unsigned)e.y;
             ent[pr] = ((unsigned)(e.y & (BROWS - 1)) << 25) | (unsigned)e.x;
-            if (W) {
-                entv[pf] = a.w[u];
-                entv[pr] = a.w[u];
+            if (W != W_NONE) {
+                const float w = W == W_LISTED ? a.w[u] : (float)r64_pair(z, t, e.x, e.y);
+                entv[pf] = w;
+                entv[pr] = w;
             }
         }
     });
@@ -3405,32 +3394,40 @@ __global__ __launch_bounds__(256) void sp_report(const unsigned long long *__res
     }
 }
 
-// The CSR of n vertices from the nsrc sources of src (nnz entries; weights
-// beside the lists when weighted), launched without a host check; row[n]
-// reports the entries found.  Work buffers are named pfx + ...
+// One array of a work buffer that several share (256-byte steps).
+constexpr size_t slot_bytes(size_t bytes) { return (bytes + 255) / 256 * 256; }
+
+// The entries' work arrays, one after the other in the buffer pfx + "sort".
+inline size_t sort_bytes(bool weighted, long long nnz)
+{
+    return (weighted ? 4 : 2) * slot_bytes((size_t)std::max<long long>(nnz, 1) * 4);
+}
+
+// The CSR of n vertices from the nsrc sources of src (nnz entries; when weighted,
+// weights beside the lists, or, src.seg_w being NULL, summed from the rows z64
+// of t), launched without a host check; row[n] reports the entries found.  Work
+// buffers are named pfx + ...
 pg_status csr_launch(pg_ctx *ctx, const char *pfx, const EdgeSrc &src, int n, int nsrc, bool weighted, long long nnz,
-                     bool seg_counted, int *row, int *col, float *val)
+                     bool seg_counted, int *row, int *col, float *val, const double *z64 = nullptr, int t = 0)
 {
     hipStream_t st = ctx->stream;
     const std::string p = pfx;
     const size_t nnzs = (size_t)std::max<long long>(nnz, 1);
     const int nbk = (int)pg_cdiv(n, BROWS);
-    unsigned *bcnt, *ent;
+    unsigned *bcnt;
     long long *boff, *bstart, *btot;
-    int *ctmp = nullptr;
-    float *entv = nullptr, *vtmp = nullptr;
     PG_TRY(pg_bufT(ctx, (p + "bcnt").c_str(), (size_t)nsrc * nbk, &bcnt));
     PG_TRY(pg_bufT(ctx, (p + "boff").c_str(), (size_t)nsrc * nbk, &boff));
     PG_TRY(pg_bufT(ctx, (p + "bstart").c_str(), (size_t)nbk + 1, &bstart));
     PG_TRY(pg_bufT(ctx, (p + "btot").c_str(), (size_t)nbk + 1, &btot));
-    PG_TRY(pg_bufT(ctx, (p + "ent").c_str(), nnzs, &ent));
     const BitsPlan bp = weighted ? BitsPlan() : rows_bits_plan(n, ctx->lds_per_block);
     const size_t lbits = bp.lds;
-    if (!lbits) PG_TRY(pg_bufT(ctx, (p + "ctmp").c_str(), nnzs, &ctmp));
-    if (weighted) {
-        PG_TRY(pg_bufT(ctx, (p + "entv").c_str(), nnzs, &entv));
-        PG_TRY(pg_bufT(ctx, (p + "vtmp").c_str(), nnzs, &vtmp));
-    }
+    char *sort;
+    PG_TRY(pg_bufT(ctx, (p + "sort").c_str(), lbits ? nnzs * 4 : sort_bytes(weighted, nnz), &sort));
+    const size_t step = slot_bytes(nnzs * 4);
+    unsigned *ent = (unsigned *)sort;
+    int *ctmp = (int *)(sort + step);
+    float *entv = (float *)(sort + 2 * step), *vtmp = (float *)(sort + 3 * step);  // weighted only
     const size_t shb = (size_t)nbk * 4;
     if (!seg_counted) {
         if (shb > 64 * 1024) PG_HIP(ctx, set_shared_limit(ctx, (const void *)bucket_count, shb));
@@ -3439,14 +3436,9 @@ pg_status csr_launch(pg_ctx *ctx, const char *pfx, const EdgeSrc &src, int n, in
     bucket_scan_local<<<(unsigned)pg_cdiv(nbk, SCAN_BK), SCAN_BK * SCAN_SG, 0, st>>>(bcnt, nsrc, nbk, boff, btot);
     bucket_scan_global<<<1, 1024, 0, st>>>(btot, nbk, bstart);
     const size_t shs = (size_t)nbk * (4 + 4);  // bases + cursors
-    const void *scatter_fn = weighted ? (const void *)bucket_scatter<true> : (const void *)bucket_scatter<false>;
-    if (shs > 64 * 1024) PG_HIP(ctx, set_shared_limit(ctx, scatter_fn, shs));
-    if (weighted)
-        bucket_scatter<true><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, entv,
-                                                                       (long long)nnzs);
-    else
-        bucket_scatter<false><<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, nullptr,
-                                                                        (long long)nnzs);
+    const auto scatter = !weighted ? bucket_scatter<W_NONE> : src.seg_w ? bucket_scatter<W_LISTED> : bucket_scatter<W_SUMMED>;
+    if (shs > 64 * 1024) PG_HIP(ctx, set_shared_limit(ctx, (const void *)scatter, shs));
+    scatter<<<(unsigned)nsrc, SEG_THREADS, shs, st>>>(src, nbk, boff, bstart, ent, entv, z64, t, (long long)nnzs);
     if (lbits) {
         PG_HIP(ctx, set_shared_limit(ctx, rows_bits_fn(bp.rank), (int)lbits));
         launch_rows_bits(ctx, bp, st, bstart, ent, n, nbk, row, col, (long long)nnzs);
@@ -3732,33 +3724,31 @@ struct CorrRun {
         return PG_OK;
     }
 
-    // The weights of src's kept entries, into buffers beside its lists.
-    pg_status launch_edge_values(EdgeSrc &src)
+    // The weights of src's kept entries, beside its lists in "corr.segw"; the
+    // chunked series and the partial sums lie where the sort's arrays follow.
+    // Without room for either, src.seg_w stays NULL and the scatter sums.
+    pg_status launch_edge_values(EdgeSrc &src, long long nnz)
     {
+        const long long nw = src.nseg * seg_used, ne = std::max<long long>(src.extra_cap, 1);
+        const int tc = (int)pg_cdiv(t, 16);
+        const size_t zb = slot_bytes((size_t)tc * n * 16 * 8), pb = tc > VAL_SLICE ? (size_t)(nw + ne) * 8 : 0;
+        float *w;
+        char *sort;
+        pg_status s = pg_bufT(ctx, "corr.segw", (size_t)(nw + ne), &w);
+        if (s == PG_OK) s = pg_bufT(ctx, "corr.sort", std::max(zb + pb, sort_bytes(true, nnz)), &sort);
+        if (s == PG_ENOMEM) return PG_OK;
+        PG_TRY(s);
+        src.seg_w = w;
+        src.extra_w = w + nw;
         src.w_cap = seg_used;
-        const size_t nw = (size_t)std::max<long long>(src.nseg * src.w_cap, 1), ne = (size_t)std::max<long long>(src.extra_cap, 1);
-        PG_TRY(pg_bufT(ctx, "corr.segw", nw, &src.seg_w));
-        PG_TRY(pg_bufT(ctx, "corr.extraw", ne, &src.extra_w));
-        // a chunk's row offsets are 32-bit
-        if (n < (1 << 28)) {
-            // three work-groups of 43 KB fit a CU: about that many in all
-            const int nsub = (int)std::max<long long>(1, pg_cdiv(3LL * std::max(ctx->num_cu, 1), std::max(src.nseg, 1)));
-            const long long ex = std::max<long long>(1, std::min<long long>(pg_cdiv(src.extra_cap, 256), 2LL * std::max(ctx->num_cu, 1)));
-            const int slice = VAL_SLICE;
-            const int tc = (int)pg_cdiv(t, 16);
-            double *zc, *part = nullptr, *epart = nullptr;
-            PG_TRY(pg_bufT(ctx, "corr.zc", (size_t)tc * n * 16, &zc));
-            if (tc > slice) {
-                PG_TRY(pg_bufT(ctx, "corr.segp", nw, &part));
-                PG_TRY(pg_bufT(ctx, "corr.extrap", ne, &epart));
-            }
-            zchunk_copy<<<dim3((unsigned)pg_cdiv(n, 32), (unsigned)tc), 256, 0, st>>>(z64, n, t, zc);
-            for (int c0 = 0; c0 < tc; c0 += slice)
-                edge_values<<<(unsigned)(src.nseg * nsub + ex), 256, 0, st>>>(src, zc, n, tc, nsub, c0,
-                                                                              std::min(tc, c0 + slice), part, epart);
-        } else {
-            edge_values_wide<<<dim3(8, (unsigned)src.nseg + 1), 256, 0, st>>>(src, z64, t);
-        }
+        double *zc = (double *)sort, *part = (double *)(sort + zb);
+        // three work-groups of 43 KB fit a CU: about that many in all
+        const int nsub = (int)std::max<long long>(1, pg_cdiv(3LL * std::max(ctx->num_cu, 1), std::max(src.nseg, 1)));
+        const long long ex = std::max<long long>(1, std::min<long long>(pg_cdiv(src.extra_cap, 256), 2LL * std::max(ctx->num_cu, 1)));
+        zchunk_copy<<<dim3((unsigned)pg_cdiv(n, 32), (unsigned)tc), 256, 0, st>>>(z64, n, t, zc);
+        for (int c0 = 0; c0 < tc; c0 += VAL_SLICE)
+            edge_values<<<(unsigned)(src.nseg * nsub + ex), 256, 0, st>>>(src, zc, n, tc, nsub, c0,
+                                                                          std::min(tc, c0 + VAL_SLICE), part, part + nw);
         PG_KERNEL_CHECK(ctx);
         return PG_OK;
     }
@@ -3778,8 +3768,8 @@ struct CorrRun {
             PG_HIP(ctx, hipMemsetAsync(row, 0, 4, st));
             return PG_OK;
         }
-        if (weighted) PG_TRY(launch_edge_values(src));
-        return csr_launch(ctx, "corr.", src, n, nsrc, weighted, nnz, seg_counted, row, col, val);
+        if (weighted) PG_TRY(launch_edge_values(src, nnz));
+        return csr_launch(ctx, "corr.", src, n, nsrc, weighted, nnz, seg_counted, row, col, val, z64, t);
     }
 
     // launch, wait, and check row[n]
@@ -4814,7 +4804,7 @@ pg_status pg_cohort_corr_plan(pg_ctx *ctx, int nsub, const int32_t *n, const int
     PG_HIP(ctx, set_shared_limit(ctx, (const void *)window_count, (int)((size_t)max_nbk * 4)));
     const size_t shs = (size_t)max_nbk * 8;
     if (shs > 64 * 1024)
-        PG_HIP(ctx, set_shared_limit(ctx, (const void *)bucket_scatter<false>, (int)shs));
+        PG_HIP(ctx, set_shared_limit(ctx, (const void *)bucket_scatter<W_NONE>, (int)shs));
     PG_HIP(ctx, set_shared_limit(ctx, (const void *)bucket_rows<false>, (int)max_rows_lds));
     PG_HIP(ctx, set_shared_limit(ctx, rows_bits_fn(false), (int)max_bits_lds));
     PG_HIP(ctx, set_shared_limit(ctx, rows_bits_fn(true), (int)max_bits_lds));
@@ -4907,8 +4897,8 @@ pg_status pg_cohort_corr_enqueue(PgCohortCorr *P, int s, const float *dbold, int
     bucket_scan_local<<<(unsigned)pg_cdiv(S.nbk, SCAN_BK), SCAN_BK * SCAN_SG, 0, st>>>(P->bcnt, nsrcb, S.nbk,
                                                                                      P->boff, P->btot);
     bucket_scan_global<<<1, 1024, 0, st>>>(P->btot, S.nbk, P->bstart);
-    bucket_scatter<false><<<(unsigned)nsrcb, SEG_THREADS, (size_t)S.nbk * 8, st>>>(es, S.nbk, P->boff, P->bstart,
-                                                                                   P->ent, nullptr, nnz);
+    bucket_scatter<W_NONE><<<(unsigned)nsrcb, SEG_THREADS, (size_t)S.nbk * 8, st>>>(
+        es, S.nbk, P->boff, P->bstart, P->ent, nullptr, nullptr, 0, nnz);
     if (S.bits_lds) {
         BitsPlan bp;
         bp.rank = S.bits_rank;

@@ -344,3 +344,62 @@ def test_bc_path_counts_beyond_32_bits(ctx, stages, width, monkeypatch):
     np.testing.assert_allclose(bc, obc, rtol=1e-9, atol=1e-9)
     src = np.arange(0, n, 2, dtype=np.int32)
     np.testing.assert_array_equal(ctx.bfs(row, col, src), np.stack([O.bfs(row, col, int(s)) for s in src]))
+
+
+FAILING = """
+import ctypes as C, os, sys
+mem = C.CDLL({mem!r}, mode=os.RTLD_GLOBAL)
+sys.modules["torch"] = None  # ROCm's own runtime, so that hipMalloc is the test's
+for p in ({root!r}, {pkg!r}):
+    sys.path.insert(0, p)
+import numpy as np
+import pagani_amd
+from pagani_amd import synth
+
+def build(ctx, x, prec, sparsity):
+    info = ctx.corr_build(x, x.shape[1], x.shape[0], 5.0 if sparsity else 0.2, sparsity=sparsity, weighted=True, prec=prec)
+    return ctx.corr_csr(x.shape[1], info.nnz, True)
+
+x = synth.bold(7, 1500, 101, 6)
+for prec in (0, 1):
+    for sparsity in (False, True):
+        with pagani_amd.Context(0) as ctx:
+            want = build(ctx, x, prec, sparsity)
+        spared, made, nth = 0, 0, 0
+        while made >= nth:
+            nth += 1
+            print("prec", prec, "sparsity", sparsity, "request", nth, flush=True)
+            with pagani_amd.Context(0) as ctx:
+                mem.malloc_fails(nth)
+                try:
+                    got = build(ctx, x, prec, sparsity)
+                except pagani_amd.PgError as e:
+                    assert e.status == 2, e
+                    got = None
+                made = mem.malloc_requests()
+                mem.malloc_fails(0)
+                if got is None:  # and the context still works
+                    got = build(ctx, x, prec, sparsity)
+                elif made >= nth:
+                    spared += 1
+                for a, b in zip(got, want):
+                    assert np.array_equal(a.view(np.uint32), b.view(np.uint32)), nth
+        assert spared >= 2, spared
+"""
+
+
+def test_weighted_builds_without_room_for_the_lists(tmp_path):
+    """Each allocation of a weighted build's first call refused in turn: the
+    weights summed in the scatter are those of the lists, bit for bit."""
+    import os
+    import subprocess
+    import sys
+    here = os.path.dirname(os.path.abspath(__file__))
+    root = os.path.dirname(here)
+    mem = str(tmp_path / "libmallocfails.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", os.path.join(here, "hip_malloc_fails.cpp"), "-ldl", "-o", mem],
+                   check=True)
+    src = FAILING.format(mem=mem, root=root, pkg=os.path.join(root, "pagani-toolkit_amd"))
+    say("weighted builds with one refused allocation each")
+    r = subprocess.run([sys.executable, "-c", src], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:] + r.stdout[-500:]

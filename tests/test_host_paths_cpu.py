@@ -109,3 +109,36 @@ def test_clustering_flag_after_a_failed_allocation(stub):
         assert flags == [0], (nth, flags)
     assert failed >= 4
     """)
+
+
+def test_weighted_build_allocations(stub):
+    """Two buffers of a weighted build are only for speed: without either the
+    scatter sums the weights itself, and no other request may fail."""
+    run(stub, """
+    n, t = 300, 100
+    x = np.zeros((t, n), np.float32)
+    summed, listed = "bucket_scatterILi2E", "bucket_scatterILi1E"
+    spared = refused = 0
+    for nth in range(1, 60):
+        ctx = pagani_amd.Context(0)
+        launches.clear()
+        stub.stub_fail_malloc(nth)
+        status = 0
+        try:
+            ctx.corr_build(x, n, t, 0.3, weighted=True)
+        except pagani_amd.PgError as e:
+            status = e.status
+        made = stub.stub_mallocs()
+        stub.stub_fail_malloc(0)
+        names = [x[0] for x in launches]
+        if status == 2:
+            refused += 1
+            continue
+        assert status == 0
+        if made < nth:
+            assert any(listed in x for x in names), names
+            break
+        assert any(summed in x for x in names) and not any(listed in x for x in names), (nth, names)
+        spared += 1
+    assert spared == 2 and refused >= 10, (spared, refused, nth)
+    """)
