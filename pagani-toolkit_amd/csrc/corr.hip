@@ -1852,7 +1852,14 @@ __global__ __launch_bounds__(256) void zchunk_copy(const double *__restrict__ z,
 // with slices of 4 chunks, 7.5 / 4.7 of 6, 6.9 / 6.4 of 2, 9.5 / 5.4 unsliced;
 // on unaligned rows of z64 13.5 / 8.1 unsliced, 9.6 / 8.2 sliced; a thread per
 // pair inside bucket_scatter took 18.9 / 33.3 ms.
+// A copy of up to VAL_ONE bytes goes in one launch, without partial sums: its
+// rows meet in the L2s anyway, and the launches are what is left.  A whole
+// weighted build, sliced / in one, by the copy's size: 5.0 MB (n = 3,000, t =
+// 200) 0.244 / 0.221 ms at a fixed r, 0.327 / 0.312 at 1%; 13.3 MB 0.323 / 0.301,
+// 0.369 / 0.349; 19.5 MB (4,000, 600) 0.655 / 0.591, 0.721 / 0.688; 26.6 MB 0.501 /
+// 0.489, 0.695 / 0.701; 49.9 MB 1.068 / 1.114, 1.769 / 1.999.
 constexpr int VAL_SLICE = 4;
+constexpr size_t VAL_ONE = 20 << 20;
 __global__ __launch_bounds__(256) void edge_values(EdgeSrc s, const double *__restrict__ zc, int n, int tc, int nsub,
                                                    int c0, int c1, double *__restrict__ part,
                                                    double *__restrict__ epart)
@@ -3731,7 +3738,9 @@ struct CorrRun {
     {
         const long long nw = src.nseg * seg_used, ne = std::max<long long>(src.extra_cap, 1);
         const int tc = (int)pg_cdiv(t, 16);
-        const size_t zb = slot_bytes((size_t)tc * n * 16 * 8), pb = tc > VAL_SLICE ? (size_t)(nw + ne) * 8 : 0;
+        const size_t zb = slot_bytes((size_t)tc * n * 16 * 8);
+        const int slice = zb <= VAL_ONE ? tc : VAL_SLICE;
+        const size_t pb = tc > slice ? (size_t)(nw + ne) * 8 : 0;
         float *w;
         char *sort;
         pg_status s = pg_bufT(ctx, "corr.segw", (size_t)(nw + ne), &w);
@@ -3746,9 +3755,9 @@ struct CorrRun {
         const int nsub = (int)std::max<long long>(1, pg_cdiv(3LL * std::max(ctx->num_cu, 1), std::max(src.nseg, 1)));
         const long long ex = std::max<long long>(1, std::min<long long>(pg_cdiv(src.extra_cap, 256), 2LL * std::max(ctx->num_cu, 1)));
         zchunk_copy<<<dim3((unsigned)pg_cdiv(n, 32), (unsigned)tc), 256, 0, st>>>(z64, n, t, zc);
-        for (int c0 = 0; c0 < tc; c0 += VAL_SLICE)
+        for (int c0 = 0; c0 < tc; c0 += slice)
             edge_values<<<(unsigned)(src.nseg * nsub + ex), 256, 0, st>>>(src, zc, n, tc, nsub, c0,
-                                                                          std::min(tc, c0 + VAL_SLICE), part, part + nw);
+                                                                          std::min(tc, c0 + slice), part, part + nw);
         PG_KERNEL_CHECK(ctx);
         return PG_OK;
     }

@@ -27,6 +27,23 @@ def test_weighted_values_bitwise(ctx, n, t):
         np.testing.assert_array_equal(val.view(np.uint32), oval.view(np.uint32))
 
 
+# chunked copies of the series just up to 20 MiB (values in one launch) and just
+# beyond (slices of four chunks with partial sums), the last chunk and slice ragged
+@pytest.mark.parametrize("n,t", [(2600, 1000), (2601, 1000), (2600, 1009), (9600, 270)])
+def test_weighted_values_in_slices(ctx, n, t):
+    from pagani_amd import synth
+    x = synth.bold(n + t, n, t, 7)
+    z64, _ = O.zscore(x)
+    for prec in (0, 1):
+        say(f"weighted values in slices n={n} t={t} prec={prec}")
+        info = ctx.corr_build(x, n, t, 0.4, weighted=True, prec=prec)
+        row, col, val = ctx.corr_csr(n, info.nnz, True)
+        orow, ocol, oval = O.corr_csr_r(z64, 0.4, True)
+        np.testing.assert_array_equal(row, orow)
+        np.testing.assert_array_equal(col, ocol)
+        np.testing.assert_array_equal(val.view(np.uint32), oval.view(np.uint32))
+
+
 # buckets of 16 rows beyond the 12,288 entries kept in registers, the last wave
 # of their entries with 1 to 63 lanes (bucket lengths vary with the rows)
 @pytest.mark.parametrize("n", [801, 1537, 2999, 4500])

@@ -141,4 +141,6 @@ def test_weighted_build_allocations(stub):
         assert any(summed in x for x in names) and not any(listed in x for x in names), (nth, names)
         spared += 1
     assert spared == 2 and refused >= 10, (spared, refused, nth)
+    # with the lists: a small network's values take one launch
+    assert sum("edge_values" in x for x in names) == 1, names
     """)
