@@ -3367,7 +3367,7 @@ struct SpReport {
     int rn;                          // row[n] of the CSR built
     int pad;
 };
-static_assert(sizeof(SpReport) <= PG_REPORT_BYTES, "report exceeds the pinned buffer");
+static_assert(sizeof(SpReport) <= PG_REPORT_BYTES - sizeof(PgCheck), "report reaches the checks' words");
 
 __global__ __launch_bounds__(256) void sp_report(const unsigned long long *__restrict__ seg_cnt, int nseg,
                                                  const unsigned long long *__restrict__ counters,
