@@ -395,6 +395,21 @@ __global__ __launch_bounds__(1024) void cm_scan(const int *__restrict__ in, int 
     pgdev::block_scan_1024(in, n, out, 1);
 }
 
+// What the host checks of a threshold, in the context's pinned memory: a launch
+// in place of a copy for each (a copy and its wait took 15 us of a region-level
+// call's 270).
+struct CmReport {
+    long long gt, tie;
+    int rn;
+};
+__global__ void cm_report(const long long *__restrict__ gt, const long long *__restrict__ tie,
+                          const int *__restrict__ rn, CmReport *__restrict__ out)
+{
+    if (gt) out->gt = *gt;
+    if (tie) out->tie = *tie;
+    if (rn) out->rn = *rn;
+}
+
 // The kept pairs (and values) of packed row i at base[i] on: values above the
 // bound, and ties at it while their row-major rank (tbase[i] + rank inside the
 // row) is below ntie; with ties the kept ties of earlier rows shift base[i],
@@ -599,11 +614,11 @@ extern "C" pg_status pg_cormat_threshold(pg_ctx *ctx, int32_t thr_kind, float th
     cm_row_counts<<<(unsigned)n, 256, 0, st>>>(a, n, bound, cgt, ctie);
     cm_scan<<<1, 1024, 0, st>>>(cgt, n, rp);
     if (smode) cm_scan<<<1, 1024, 0, st>>>(ctie, n, tbase);
+    volatile CmReport *rep = (CmReport *)ctx->h_report;
+    cm_report<<<1, 1, 0, st>>>(rp + n, smode ? tbase + n : nullptr, nullptr, (CmReport *)rep);
     PG_KERNEL_CHECK(ctx);
-    long long totgt = 0, tottie = 0;
-    PG_HIP(ctx, hipMemcpyAsync(&totgt, rp + n, 8, hipMemcpyDeviceToHost, st));
-    if (smode) PG_HIP(ctx, hipMemcpyAsync(&tottie, tbase + n, 8, hipMemcpyDeviceToHost, st));
     PG_HIP(ctx, hipStreamSynchronize(st));
+    const long long totgt = rep->gt, tottie = smode ? rep->tie : 0;
     if (smode) {
         ntie = kwant - totgt;
         if (ntie < 1 || ntie > tottie)
@@ -634,9 +649,10 @@ extern "C" pg_status pg_cormat_threshold(pg_ctx *ctx, int32_t thr_kind, float th
     cm_pairs<<<(unsigned)pg_cdiv(n, 4), 256, 0, st>>>(a, n, bound, smode, rp, tbase, ntie, pairs, w);
     PG_KERNEL_CHECK(ctx);
     PG_TRY(pg_csr_pairs(ctx, "cm.", pairs, w, kept, n, row, col, val));
-    int rn = 0;
-    PG_HIP(ctx, hipMemcpyAsync(&rn, row + n, 4, hipMemcpyDeviceToHost, st));
+    cm_report<<<1, 1, 0, st>>>(nullptr, nullptr, row + n, (CmReport *)rep);
+    PG_KERNEL_CHECK(ctx);
     PG_HIP(ctx, hipStreamSynchronize(st));
+    const int rn = rep->rn;
     if (rn != nnz) return pg_fail(ctx, PG_ETHRESH, "CSR holds %d entries, %lld wanted", rn, nnz);
     if (thr_kind == PG_THR_R) inf.s_thresh = (float)(100.0 * nnz / m1 / 2);
     inf.nnz = nnz;

@@ -144,3 +144,18 @@ def test_weighted_build_allocations(stub):
     # with the lists: a small network's values take one launch
     assert sum("edge_values" in x for x in names) == 1, names
     """)
+
+
+def test_threshold_of_an_average_copies_nothing_back(stub):
+    """What the host checks comes through pinned memory: no copy per number."""
+    run(stub, """
+    n = 116
+    x = np.zeros((50, n), np.float32)
+    ctx = pagani_amd.Context(0)
+    ctx.cormat_begin(n)
+    ctx.cormat_add(x, 50)
+    ctx.cormat_finish()
+    before = stub.stub_copies()
+    assert ctx.cormat_threshold(0.3).nnz == 0
+    assert stub.stub_copies() == before
+    """)
