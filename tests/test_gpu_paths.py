@@ -284,9 +284,11 @@ def test_segmented_modularity(ctx, n, m, hub, stop, weighted):
         assert got[4] == want[4]
 
 
-# one and two 4,096-source chunks; work-groups whose last round of 256 vertices
-# is whole (512, 4,096) or ragged
-@pytest.mark.parametrize("n,m,tail", [(70, 200, 10), (512, 3000, 20), (4096, 30000, 3), (4500, 40000, 300)])
+# one to four 4,096-source chunks (a work-group's waves of one chunk mark found
+# sources together up to three); work-groups whose last round of 256 vertices is
+# whole (512, 4,096) or ragged, whose last wave is past the end (4,501, 9,003)
+@pytest.mark.parametrize("n,m,tail", [(70, 200, 10), (512, 3000, 20), (4096, 30000, 3), (4500, 40000, 300),
+                                      (4501, 20000, 30), (9003, 30000, 40), (12301, 40000, 5)])
 def test_efficiency_components_and_tails(ctx, n, m, tail):
     """A random part, a chain hanging off it (sources that stay active for many
     levels), a separate triangle and isolated vertices."""
