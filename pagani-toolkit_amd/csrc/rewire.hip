@@ -381,7 +381,7 @@ __global__ __launch_bounds__(256) void rw_propose_bits(RwRound r, const int2 *__
                                                        const unsigned *__restrict__ bm, int nw,
                                                        unsigned long long *__restrict__ tab,
                                                        uint8_t *__restrict__ lost, int2 *__restrict__ F,
-                                                       int *__restrict__ part)
+                                                       long long *__restrict__ part)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     bool claimed = false;
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(256) void rw_propose_bits(RwRound r, const int2 *__
 template <bool MOVED>
 __global__ __launch_bounds__(256) void rw_restore(RwRound r, const int2 *__restrict__ E,
                                                   const uint8_t *__restrict__ lost, int2 *__restrict__ F,
-                                                  int *__restrict__ part)
+                                                  long long *__restrict__ part)
 {
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const bool back = t < r.p && lost[t] != 0;
@@ -427,7 +427,7 @@ __global__ __launch_bounds__(256) void rw_restore(RwRound r, const int2 *__restr
 }
 
 // swaps = the sum of the work-groups' counts (one work-group)
-__global__ __launch_bounds__(1024) void rw_count(const int *__restrict__ part, int np, unsigned long long *__restrict__ swaps)
+__global__ __launch_bounds__(1024) void rw_count(const long long *__restrict__ part, int np, unsigned long long *__restrict__ swaps)
 {
     __shared__ unsigned long long red[16];
     unsigned long long s = 0;
@@ -449,7 +449,7 @@ __global__ void rw_weights(RwRound r, const float *__restrict__ ew, float *__res
     if (p < r.m) fw[p] = ew[rw_perm((unsigned)p, r)];
 }
 
-__global__ void rw_zero(int *__restrict__ p, int n)
+__global__ void rw_zero(long long *__restrict__ p, int n)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = 0;
@@ -648,7 +648,7 @@ extern "C" pg_status pg_rewire(pg_ctx *ctx, const int32_t *row, const int32_t *c
         unsigned *lost = nullptr;  // a byte per attempt
         const long long half = (m + 1) / 2, nlost = (per_round + 3) / 4;
         const int np = (int)pg_cdiv(half, 256);
-        int *part = nullptr;
+        long long *part = nullptr;
         PG_TRY(pg_bufT(ctx, "rw.tab", (size_t)cap, &tab));
         if (bits) {
             PG_TRY(pg_bufT(ctx, "rw.lost", (size_t)nlost, &lost));
