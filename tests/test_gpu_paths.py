@@ -316,7 +316,7 @@ def test_efficiency_components_and_tails(ctx, n, m, tail):
 
 
 # bitmap of the edges (n^2 / 16 bytes up to 64 MB or 48 per edge), the hash
-# beyond; a hub row longer than the registers sort
+# beyond; a hub row
 @pytest.mark.parametrize("n,m,hub", [(31, 200, 0), (32, 300, 0), (33, 200, 20), (2000, 30000, 1500),
                                      (32000, 100000, 1500), (40000, 100000, 1500)])
 @pytest.mark.parametrize("weighted", [False, True])
@@ -337,6 +337,23 @@ def test_rewire_paths(ctx, n, m, hub, weighted):
         with pytest.raises(pagani_amd.PgError) as ex:
             ctx.rewire(row, bad, v, seed=9)
         assert ex.value.status == 4
+
+
+# 325,632: the last n whose rows the counting sort takes; beyond, rows are filled
+# and sorted one by one, those above 1,024 entries by a bitmap
+@pytest.mark.parametrize("n", [325632, 325633, 326000])
+@pytest.mark.parametrize("hub", [0, 1024, 1025, 5000])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_rewire_beyond_the_counting_sort(ctx, n, hub, weighted):
+    from helpers import check_rewired
+    row, col, val = _graph(n, 400000, n + hub, hub)
+    v = val if weighted else None
+    say(f"rewire rows n={n} hub={hub} nnz={col.size} weighted={weighted}")
+    if hub:
+        assert np.diff(row).max() >= hub
+    oc, ov, sw = ctx.rewire(row, col, v, seed=5)
+    check_rewired(row, col, v, oc, ov)
+    assert sw > 0.9 * col.size
 
 
 def _ladder(stages, width):

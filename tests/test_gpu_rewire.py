@@ -118,8 +118,8 @@ def test_statistics_match_oracle(ctx):
 
 
 def test_long_rows(ctx):
-    # a hub joined to every vertex (row of 2999 > 1024: the LDS-bitmap sort)
-    # over a dense random graph (rows of 500-700: the 16-per-lane sort)
+    # a hub joined to every vertex (a row of 2999) over a dense random graph
+    # (rows of 500-700)
     n = 3000
     row0, col0, _ = random_graph(n, 0.2, 8)
     edges = [(i, int(j)) for i in range(n) for j in col0[row0[i]:row0[i + 1]] if j > i]
