@@ -10,7 +10,8 @@
 //    |u - u0|^2, |u + u0|^2) in a fixed order, so all blocks take the same stop
 //    decision on the device and launches past the stop return at once.  The
 //    host looks once per batch of launches.  FP64 throughout, FP32 weights.
-//    The SpMV stages segments of the vector in LDS (pg_spmv.hpp).
+//    The SpMV stages segments of the vector in LDS, or, for a sparse network,
+//    gathers it (pg_spmv.hpp).
 //  * Participation coefficient (W/PC_CPU/PC_CPU/main.cpp:96-160): one wave per
 //    vertex, FP32 module sums accumulated in LDS in CSR order by one lane
 //    (entries staged 64 at a time), then the FP32 sum of squared shares over
@@ -63,8 +64,8 @@ __global__ __launch_bounds__(EC_TPB) void ec_init(int n, int R, double *__restri
 }
 
 // Iteration k.  Every block takes the norm and the stop decision from the
-// previous launch's partials, then its rows of A u by the LDS-staged SpMV of
-// pg_spmv.hpp on the raw u, scaled once per row.  n = 40,009 with 16 M entries:
+// previous launch's partials, then its rows of A u by the SpMV of
+// pg_spmv.hpp on the raw u, scaled once per row.  Staged, n = 40,009 with 16 M entries:
 // 20.0 us (27.1 us with one lane per row in blocks of 256 rows; 21.9 us with a
 // segment's first entries loaded behind its staging), three segments of about
 // 5 us each, bound by the entries' latency from beyond L2 (32 MB of them an

@@ -14,9 +14,9 @@
 //    FP64 dot products of unit-norm rows), so when r - delta and r + delta
 //    round to the same float that float is the oracle's; otherwise (mostly
 //    pairs with r near 0, where FP32 steps are tiny) the pair goes to a list
-//    that a second kernel recomputes in the oracle's sequential order, one
-//    thread per pair (a lane stalling its wave for a 240-step dependent sum
-//    would idle the matrix cores).
+//    that a second kernel recomputes in the oracle's sequential order, a wave
+//    per 16 pairs (a lane stalling its wave for a 240-step dependent sum would
+//    idle the matrix cores).
 //  * The epilogue adds every pair's FP32 r, or its Fisher z, to the packed
 //    accumulator straight from the MFMA result registers (16 consecutive
 //    columns of a row per 16 lanes); the first subject is written.

@@ -222,8 +222,8 @@ __global__ __launch_bounds__(256) void upper_lists(const int *__restrict__ row, 
 // N(u) a bitmap in LDS (its bit n stays clear), each wave scanning the lists
 // of every fourth neighbour.  A wave fetches the list bounds of 64 neighbours
 // at once and the first group of the next list under the current one.
-// Bound by LDS look-ups and the lists' L2 / MALL reads: N = 58,000 with 33.6 M
-// entries takes 4.0 ms (13.1 ms scanning the CSR itself, 4 bytes per look-up
+// Bound by VALU issue (92% of the SIMDs' cycles, the LDS busy 56%): N = 58,000
+// with 33.6 M entries takes 4.0 ms (13.1 ms scanning the CSR itself, 4 bytes per look-up
 // and a search for each list's start).
 template <class CT>
 __global__ __launch_bounds__(256) void triangles_lists(const int *__restrict__ row, const int *__restrict__ col,
@@ -337,8 +337,8 @@ __global__ __launch_bounds__(MEAN_TPB) void mean_kernel(const T *__restrict__ x,
     }
 }
 
-// Largest of m floats in two launches: MAX_WG work-groups take the part maxima
-// (one work-group over 9 M weights took 10.4 ms), the second reduces those.
+// Largest of m floats: one work-group, or, beyond 8,192, up to MAX_WG that take
+// the part maxima (one over 9 M weights took 10.4 ms) and a second launch.
 constexpr int MAX_WG = 1024;
 __global__ __launch_bounds__(256) void max_kernel(const float *__restrict__ x, long long m, float *__restrict__ out)
 {

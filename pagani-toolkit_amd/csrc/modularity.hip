@@ -96,7 +96,7 @@ enum { P_YY, P_YK, P_A, P_B, NPART };
 // per row, with the partials of |y|^2, y . k, v . y, v . v.  |v_li -+ v_(li-1)|
 // needs |y_li|, so its partials are taken here too and the vector stop looks
 // at them one launch later: the launch that finds it leaves y_li and y_(li-1)
-// in place.  n = 14,011 with 4.9 M weighted entries: 9.9 us an iteration, half of
+// in place.  n = 14,011 with 4.9 M weighted entries: 9.3 us an iteration, half of
 // it the launch and the chain of loads up to the first row (55 us as two
 // launches that gathered the vector from L2 with a wave per row, four per
 // CU).  Every skip below is uniform in a block.
