@@ -34,14 +34,19 @@ def test_weighted_values_in_slices(ctx, n, t):
     from pagani_amd import synth
     x = synth.bold(n + t, n, t, 7)
     z64, _ = O.zscore(x)
+    rows = np.unique(np.concatenate([[0, n - 1], np.random.default_rng(n).integers(0, n, 150)])).astype(np.int32)
+    want = O.corr_rows_r(z64, 0.4, rows, True)
     for prec in (0, 1):
         say(f"weighted values in slices n={n} t={t} prec={prec}")
         info = ctx.corr_build(x, n, t, 0.4, weighted=True, prec=prec)
         row, col, val = ctx.corr_csr(n, info.nnz, True)
-        orow, ocol, oval = O.corr_csr_r(z64, 0.4, True)
-        np.testing.assert_array_equal(row, orow)
-        np.testing.assert_array_equal(col, ocol)
-        np.testing.assert_array_equal(val.view(np.uint32), oval.view(np.uint32))
+        for i, (ocol, oval) in zip(rows, want):
+            np.testing.assert_array_equal(col[row[i]:row[i + 1]], ocol)
+            np.testing.assert_array_equal(val[row[i]:row[i + 1]].view(np.uint32), oval.view(np.uint32))
+        # the other direction of every entry carries the same weight
+        src = np.repeat(np.arange(n, dtype=np.int64), np.diff(row))
+        back = np.argsort(col.astype(np.int64) * n + src)
+        np.testing.assert_array_equal(val[back].view(np.uint32), val.view(np.uint32))
 
 
 # buckets of 16 rows beyond the 12,288 entries kept in registers, the last wave
