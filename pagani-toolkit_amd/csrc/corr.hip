@@ -3745,7 +3745,12 @@ struct CorrRun {
         char *sort;
         pg_status s = pg_bufT(ctx, "corr.segw", (size_t)(nw + ne), &w);
         if (s == PG_OK) s = pg_bufT(ctx, "corr.sort", std::max(zb + pb, sort_bytes(true, nnz)), &sort);
-        if (s == PG_ENOMEM) return PG_OK;
+        if (s == PG_ENOMEM) {
+            PgBuf &b = ctx->bufs["corr.segw"];
+            if (b.p) (void)hipFree(b.p);  // the sort may need its room
+            b = PgBuf();
+            return PG_OK;
+        }
         PG_TRY(s);
         src.seg_w = w;
         src.extra_w = w + nw;

@@ -36,6 +36,7 @@ extern "C" {
 void stub_hook(void (*f)(const char *, int, int, void **)) { hook = f; }
 void stub_fail_malloc(int nth) { mallocs = 0, fail_at = nth; }  // 1: the next one; 0: none
 int stub_mallocs() { return mallocs; }
+int stub_live() { return (int)ranges.size(); }
 int stub_copies() { return copies; }
 int stub_device() { return current; }
 void *stub_alloc(size_t bytes, int device, int managed)

@@ -119,7 +119,10 @@ def test_weighted_build_allocations(stub):
     x = np.zeros((t, n), np.float32)
     summed, listed = "bucket_scatterILi2E", "bucket_scatterILi1E"
     spared = refused = 0
+    live = []  # allocations after a build that summed
     for nth in range(1, 60):
+        if nth > 1:
+            ctx.close()
         ctx = pagani_amd.Context(0)
         launches.clear()
         stub.stub_fail_malloc(nth)
@@ -140,7 +143,10 @@ def test_weighted_build_allocations(stub):
             break
         assert any(summed in x for x in names) and not any(listed in x for x in names), (nth, names)
         spared += 1
+        live.append(stub.stub_live())
     assert spared == 2 and refused >= 10, (spared, refused, nth)
+    # the lists' weights are given back where the sort's buffer had no room
+    assert live[0] == live[1], live
     # with the lists: a small network's values take one launch
     assert sum("edge_values" in x for x in names) == 1, names
     """)
